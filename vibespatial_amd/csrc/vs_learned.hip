@@ -38,6 +38,7 @@
 // An escalated edge is evaluated by the exact fp64 step (stage-A filter, then
 // the exact expansion) on the original coordinates.
 #include <mutex>
+#include <type_traits>
 
 #include "vs_exact.h"
 #include "vs_internal.h"
@@ -73,6 +74,23 @@ constexpr int kWavePos = 256;              // wave mode: at most this many posit
 constexpr int kWaveEdges = 128;            // wave mode: at most this many edges per polygon (2 per lane)
 static_assert(kLJThreads / 64 == kClaim, "wave mode runs one claimed item per wave");
 constexpr int kCandPerThread = kChunk / kLJThreads;
+constexpr int kMaskParts = 32;             // parts whose crossing parities fit one mask per candidate
+constexpr int kEdgeCap = 512;              // edges staged in LDS per batch
+
+// Polygons every edge of which fits the LDS buffers: staged once per item and
+// refined straight from the scan ("direct path").  info: poly_info entry.
+__device__ __forceinline__ bool direct_polygon(const int4& info) {
+    return info.z <= kMaskParts && info.y - info.x <= kEdgeCap + 1;
+}
+
+// Scanned positions of one work item.  The others stream their edges through
+// LDS once per 256 candidates, so an item of theirs costs rounds x edges: with
+// 4,096 positions the last such item alone ran for milliseconds (a 5,000-vertex
+// row over a dense cluster), with 512 the launch ends with the rest.  Together
+// with the part masks below, whole joins: 1M points x 100k rows, 5% of them of
+// two parts, 3.86 -> 1.30 ms; 5M points under 20k rows, 2% of two parts, 16.5 ->
+// 4.7 ms; 10M x 100k single-part rows 2.13 -> 1.99 ms.
+__device__ __forceinline__ int item_positions(const int4& info) { return direct_polygon(info) ? kItemPos : kChunk; }
 
 // ---------------------------------------------------------------------------
 // MLP: forward, backward, training
@@ -697,8 +715,8 @@ __global__ __launch_bounds__(256) void cover_lookup_kernel(int64_t nq, const uns
     block_add_counters<3>(v, red, stat);
 }
 
-// Per query: total scan length and its number of work items (kItemPos
-// positions each); stat[3] += positions scanned.  Also the query's cost key
+// Per query: total scan length and its number of work items (item_positions
+// each); stat[3] += positions scanned.  Also the query's cost key
 // for the longest-first order, 8 bits, ascending = most expensive first:
 // (127 or, for a small item, 255) - min(127, 4 log2(1 + items x vertices)),
 // with idx[q] = q.
@@ -716,10 +734,11 @@ __global__ __launch_bounds__(256) void cover_total_kernel(int64_t nq, const int2
             const int2 r = ranges[q * kMaxRanges + k];
             total += r.y - r.x;
         }
-        const int32_t items = (int32_t)((total + kItemPos - 1) / kItemPos);
+        const int4 info = poly_info ? poly_info[q] : make_int4(0, 0, 1, 0);
+        const int per = item_positions(info);
+        const int32_t items = (int32_t)((total + per - 1) / per);
         n_items[q] = items;
         scan[0] += (unsigned long long)total;
-        const int4 info = poly_info ? poly_info[q] : make_int4(0, 0, 1, 0);
         const double v = poly_info ? (double)(info.y - info.x) : 1.0;
         const double cost = (double)items * (v > 1.0 ? v : 1.0);
         int lg = (int)(4.0 * log2(1.0 + cost));
@@ -822,7 +841,6 @@ __device__ __forceinline__ bool loc_pred(int loc) {
     return loc != 0;
 }
 
-constexpr int kEdgeCap = 512;  // edges staged in LDS per batch
 constexpr int kPosPerThread = 4;                       // direct path: positions per thread per round
 constexpr int kRoundPos = kLJThreads * kPosPerThread;  // direct path: positions per round
 constexpr int kOutCap = 2048;  // per-block output buffer (pairs)
@@ -906,12 +924,22 @@ __device__ Slabs build_slabs(const float4* __restrict__ Et, int ne, float ylo, f
     return S;
 }
 
-// Runs this thread's candidates against the edges of their own slabs.
+// Location code of a candidate from its per-part crossing parities and
+// boundary hits: the first part that is not outside decides.
+__device__ __forceinline__ int mask_loc(unsigned par, unsigned bnd) {
+    const unsigned m = par | bnd;
+    return m == 0 ? 0 : (bnd & m & (0u - m)) ? 1 : 2;
+}
+
+// Runs this thread's candidates against the edges of their own slabs.  par /
+// bnd: a bit per part (Ep[e]: the part of staged edge e, read when MULTI).
+template <bool MULTI>
 __device__ __forceinline__ void refine_slabs(const float4* __restrict__ Et, const int32_t* __restrict__ Ec,
-                                             const int* __restrict__ start, const uint16_t* __restrict__ list,
-                                             const Slabs& S, const RefineView& R, const float* pu, const float* pv,
-                                             const double* pxd, const double* pyd, float E, int* loc, int* par,
-                                             bool* done, bool* esc, unsigned& n_orient, unsigned long long& n_esc) {
+                                             const uint8_t* __restrict__ Ep, const int* __restrict__ start,
+                                             const uint16_t* __restrict__ list, const Slabs& S, const RefineView& R,
+                                             const float* pu, const float* pv, const double* pxd, const double* pyd,
+                                             float E, unsigned* par, unsigned* bnd, bool* done, bool* esc,
+                                             unsigned& n_orient, unsigned long long& n_esc) {
 #pragma unroll
     for (int j = 0; j < kCandPerThread; ++j) {
         if (done[j]) continue;
@@ -920,18 +948,49 @@ __device__ __forceinline__ void refine_slabs(const float4* __restrict__ Et, cons
         for (int k = start[b]; k < k1; ++k) {
             const int e = list[k];
             const float4 ed = Et[e];
-            if (edge_step_f32(pu[j], pv[j], ed.x, ed.y, ed.z, ed.w, E, par[j], n_orient)) {
+            const int part = MULTI ? Ep[e] : 0;
+            int flip = 0;
+            if (edge_step_f32(pu[j], pv[j], ed.x, ed.y, ed.z, ed.w, E, flip, n_orient)) {
                 ++n_esc;
                 esc[j] = true;
                 const int32_t c = Ec[e];
-                if (edge_step_f64(pxd[j], pyd[j], R.x[c - 1], R.y[c - 1], R.x[c], R.y[c], par[j])) {
-                    loc[j] = 1;
-                    done[j] = true;
-                    break;
+                if (edge_step_f64(pxd[j], pyd[j], R.x[c - 1], R.y[c - 1], R.x[c], R.y[c], flip)) {
+                    bnd[j] |= 1u << part;
+                    if (!MULTI) {
+                        done[j] = true;
+                        break;
+                    }
                 }
             }
+            par[j] ^= (unsigned)flip << part;
         }
     }
+}
+
+// One candidate of a polygon of several parts against the edges of its slab;
+// returns its location code.
+__device__ __forceinline__ int refine_parts(const float4* __restrict__ Et, const int32_t* __restrict__ Ec,
+                                           const uint8_t* __restrict__ Ep, const int* __restrict__ start,
+                                           const uint16_t* __restrict__ list, const Slabs& S, const RefineView& R,
+                                           float pu, float pv, double pxd, double pyd, float E, bool& esc,
+                                           unsigned& n_orient, unsigned long long& n_esc) {
+    unsigned par = 0, bnd = 0;
+    const int b = slab_of(pv, S);
+    const int k1 = start[b + 1];
+    for (int k = start[b]; k < k1; ++k) {
+        const int e = list[k];
+        const float4 ed = Et[e];
+        const int part = Ep[e];
+        int flip = 0;
+        if (edge_step_f32(pu, pv, ed.x, ed.y, ed.z, ed.w, E, flip, n_orient)) {
+            ++n_esc;
+            esc = true;
+            const int32_t c = Ec[e];
+            if (edge_step_f64(pxd, pyd, R.x[c - 1], R.y[c - 1], R.x[c], R.y[c], flip)) bnd |= 1u << part;
+        }
+        par ^= (unsigned)flip << part;
+    }
+    return mask_loc(par, bnd);
 }
 
 // One candidate against the edges of its slab; returns its location code.
@@ -974,13 +1033,19 @@ __device__ __forceinline__ int refine_one(const float4* __restrict__ Et, const i
     return par ? 2 : 0;
 }
 
-// Stages every edge (c-1, c), c in (lo, hi), of a single-part polygon with at
-// most kEdgeCap edges into Et/Ec (recentred fp32 and coordinate index).
+// Every thread's share of the staging counts of one pass: edges in the low 16
+// bits and part starts in the high 16, each inclusive within the wave.
+__device__ __forceinline__ int stage_counts(bool rel, int flags) {
+    return wave_inclusive_scan((rel ? 1 : 0) | ((flags & 2) ? 1 << 16 : 0));
+}
+
+// Stages every edge (c-1, c), c in (lo, hi), of a polygon with at most
+// kEdgeCap edges into Et/Ec/Ep (recentred fp32, coordinate index, part).
 // Block-uniform; returns the number staged.
 __device__ int stage_all_edges(int32_t lo, int32_t hi, double cx, double cy, const RefineView& R, float4* Et,
-                               int32_t* Ec, int* s_wsum) {
+                               int32_t* Ec, uint8_t* Ep, int* s_wsum) {
     const int tid = threadIdx.x, wid = tid >> 6, lane = tid & 63;
-    int ne = 0;
+    int ne = 0, parts = 0;
     for (int32_t base = lo; base < hi; base += kLJThreads) {
         const int32_t c = base + tid;
         const bool inr = c > lo && c < hi;
@@ -995,20 +1060,22 @@ __device__ int stage_all_edges(int32_t lo, int32_t hi, double cx, double cy, con
             by = R.y[c];
         }
         const bool rel = inr && !(f & 1);
-        const int inc = wave_inclusive_scan(rel ? 1 : 0);
+        const int inc = stage_counts(rel, f);
         if (lane == 63) s_wsum[wid] = inc;
         __syncthreads();
-        int woff = 0, tot = 0;
+        int woff = inc, tot = 0;
         for (int w2 = 0; w2 < kLJThreads / 64; ++w2) {
             woff += w2 < wid ? s_wsum[w2] : 0;
             tot += s_wsum[w2];
         }
         if (rel) {
-            const int slot = ne + woff + inc - 1;
+            const int slot = ne + (woff & 0xFFFF) - 1;
             Et[slot] = make_float4((float)(ax - cx), (float)(ay - cy), (float)(bx - cx), (float)(by - cy));
             Ec[slot] = c;
+            Ep[slot] = (uint8_t)(parts + (woff >> 16));
         }
-        ne += tot;
+        ne += tot & 0xFFFF;
+        parts += tot >> 16;
         __syncthreads();
     }
     return ne;
@@ -1028,8 +1095,8 @@ __device__ __forceinline__ void wave_lds_sync() {
 // instead of eight.  The slabs and lists are those build_slabs makes (list
 // order within a slab aside, which no decision depends on).  Block-uniform.
 __device__ Slabs stage_and_bin(int32_t lo, int32_t hi, double cx, double cy, float ylo, float yhi,
-                               const RefineView& R, float4* Et, int32_t* Ec, int* s_wsum, int* start, int* cur,
-                               uint16_t* list) {
+                               const RefineView& R, float4* Et, int32_t* Ec, uint8_t* Ep, int* s_wsum, int* start,
+                               int* cur, uint16_t* list) {
     const int tid = threadIdx.x, wid = tid >> 6, lane = tid & 63;
     const int32_t c = lo + tid;
     const bool inr = c > lo && c < hi;
@@ -1044,14 +1111,15 @@ __device__ Slabs stage_and_bin(int32_t lo, int32_t hi, double cx, double cy, flo
     }
     const bool rel = inr && !(f & 1);
     if (tid <= kMaxBins) start[tid] = 0;
-    const int inc = wave_inclusive_scan(rel ? 1 : 0);
+    const int inc = stage_counts(rel, f);
     if (lane == 63) s_wsum[wid] = inc;
     __syncthreads();
-    int woff = 0, ne = 0;
+    int woff = inc, ne = 0;
     for (int w2 = 0; w2 < kLJThreads / 64; ++w2) {
         woff += w2 < wid ? s_wsum[w2] : 0;
         ne += s_wsum[w2];
     }
+    ne &= 0xFFFF;
     Slabs S;
     S.B = 1;
     while (S.B < kMaxBins && S.B * 2 < ne) S.B <<= 1;
@@ -1061,12 +1129,13 @@ __device__ Slabs stage_and_bin(int32_t lo, int32_t hi, double cx, double cy, flo
         S.B = 1;
         S.inv = 0.0f;
     }
-    const int slot = woff + inc - 1;
+    const int slot = (woff & 0xFFFF) - 1;
     int b0 = 0, b1 = -1;
     if (rel) {
         const float4 ed = make_float4((float)(ax - cx), (float)(ay - cy), (float)(bx - cx), (float)(by - cy));
         Et[slot] = ed;
         Ec[slot] = c;
+        Ep[slot] = (uint8_t)(woff >> 16);
         if (S.B > 1) {
             b0 = slab_of(fminf(ed.y, ed.w), S);
             b1 = slab_of(fmaxf(ed.y, ed.w), S);
@@ -1105,55 +1174,63 @@ __device__ Slabs stage_and_bin(int32_t lo, int32_t hi, double cx, double cy, flo
 struct EdgeLds {
     float4* Et;
     int32_t* Ec;
+    uint8_t* Ep;  // part of the edge, counted within its polygon
     int* start;
     int* cur;
     uint16_t* list;
     int* wsum;
 };
 
-// Stages the edges (c-1, c), c in (lo, hi), of a single-part polygon that can
-// affect a point in [xmn, inf) x [ymn, ymx] (all of them when the bounds are
-// infinite) into Et/Ec in coordinate order, refining the candidates against a
-// full buffer before reusing it.  Block-uniform; returns the number left staged.
+// Stages the edges (c-1, c), c in (lo, hi), of a polygon of at most kMaskParts
+// parts that can affect a point in [xmn, inf) x [ymn, ymx] into Et/Ec/Ep in
+// coordinate order, refining the candidates against a full buffer before
+// reusing it.  Block-uniform; returns the number left staged.
+template <bool MULTI>
 __device__ int stage_edges(int32_t lo, int32_t hi, double xmn, double ymn, double ymx, double cx, double cy,
                            const RefineView& R, const EdgeLds& L, int ne, const float* pu, const float* pv,
-                           const double* pxd, const double* pyd, float E, int* loc, int* par, bool* done, bool* esc,
-                           unsigned& n_orient, unsigned long long& n_esc) {
+                           const double* pxd, const double* pyd, float E, unsigned* par, unsigned* bnd, bool* done,
+                           bool* esc, unsigned& n_orient, unsigned long long& n_esc) {
     const int tid = threadIdx.x, wid = tid >> 6, lane = tid & 63;
     float4* Et = L.Et;
     int32_t* Ec = L.Ec;
     int* s_wsum = L.wsum;
+    int parts = 0;
     for (int32_t base = lo; base < hi; base += kLJThreads) {
         const int32_t c = base + tid;
         bool rel = false;
         double ax = 0, ay = 0, bx = 0, by = 0;
-        if (c > lo && c < hi && !(R.flags[c] & 1)) {
+        int f = 1;
+        if (c > lo && c < hi) {
+            f = R.flags[c];
             ax = R.x[c - 1];
             ay = R.y[c - 1];
             bx = R.x[c];
             by = R.y[c];
-            rel = fmax(ay, by) >= ymn && fmin(ay, by) <= ymx && fmax(ax, bx) >= xmn;
+            rel = !(f & 1) && fmax(ay, by) >= ymn && fmin(ay, by) <= ymx && fmax(ax, bx) >= xmn;
         }
-        const int inc = wave_inclusive_scan(rel ? 1 : 0);
+        const int inc = stage_counts(rel, f);
         if (lane == 63) s_wsum[wid] = inc;
         __syncthreads();
-        int woff = 0, tot = 0;
+        int woff = inc, tot = 0;
         for (int w2 = 0; w2 < kLJThreads / 64; ++w2) {
             woff += w2 < wid ? s_wsum[w2] : 0;
             tot += s_wsum[w2];
         }
-        if (ne + tot > kEdgeCap) {
+        if (ne + (tot & 0xFFFF) > kEdgeCap) {
             const Slabs S = build_slabs(Et, ne, (float)(ymn - cy), (float)(ymx - cy), L.start, L.cur, L.list);
-            refine_slabs(Et, Ec, L.start, L.list, S, R, pu, pv, pxd, pyd, E, loc, par, done, esc, n_orient, n_esc);
+            refine_slabs<MULTI>(Et, Ec, L.Ep, L.start, L.list, S, R, pu, pv, pxd, pyd, E, par, bnd, done, esc,
+                                n_orient, n_esc);
             ne = 0;
             __syncthreads();
         }
         if (rel) {
-            const int slot = ne + woff + inc - 1;
+            const int slot = ne + (woff & 0xFFFF) - 1;
             Et[slot] = make_float4((float)(ax - cx), (float)(ay - cy), (float)(bx - cx), (float)(by - cy));
             Ec[slot] = c;
+            if (MULTI) L.Ep[slot] = (uint8_t)(parts + (woff >> 16));
         }
-        ne += tot;
+        ne += tot & 0xFFFF;
+        parts += tot >> 16;
         __syncthreads();
     }
     return ne;
@@ -1170,10 +1247,11 @@ static_assert(kChunk / kClaim >= kMaxBins + 1, "wave mode: a wave's slab starts 
 // (qbox = its bounds), output pairs (point, q).  MODE kLModeBox: query q is a
 // box, output pairs (q, point).  Items (up to kItemPos scanned positions of one
 // query) are taken in LPT order (queries sorted by decreasing estimated cost)
-// and processed in rounds of kChunk positions.  A small single-part polygon's
-// edges are staged in LDS once per item; larger ones are staged per round,
-// keeping only edges that can affect the round's candidates; multi-part
-// polygons stream every edge in order to settle each part's parity.
+// and processed in rounds.  A small polygon's edges are staged in LDS once per
+// item; larger ones are staged per 256 candidates, keeping only edges that can
+// affect those.  A polygon of several parts keeps one crossing parity and one
+// boundary bit per part and candidate; more parts than the mask holds stream
+// every edge in order, settling one part after the other.
 template <int MODE, int PRED>
 // Four waves per SIMD (the register cap costs a few spills; the latency of one
 // block's item start-up is hidden by the others on the CU).
@@ -1193,11 +1271,12 @@ __global__ __launch_bounds__(kLJThreads, 4) void learned_join_kernel(
     __shared__ int2 outb[kOutCap];
     __shared__ float4 Et[kEdgeCap];
     __shared__ int32_t Ec[kEdgeCap];
+    __shared__ uint8_t Ep[kEdgeCap];
     __shared__ int s_wsum[kLJThreads / 64];
     __shared__ double s_ext[kLJThreads / 64][3];
     __shared__ int s_bstart[kMaxBins + 1], s_bcur[kMaxBins];
     __shared__ uint16_t s_blist[kBinCap];
-    const EdgeLds L = {Et, Ec, s_bstart, s_bcur, s_blist, s_wsum};
+    const EdgeLds L = {Et, Ec, Ep, s_bstart, s_bcur, s_blist, s_wsum};
     const int tid = threadIdx.x, wid = tid >> 6, lane = tid & 63;
     const long long T = *total_items;
     unsigned long long st_cand = 0, st_cverts = 0, st_orient = 0, st_esc = 0, st_escpairs = 0;
@@ -1455,13 +1534,13 @@ __global__ __launch_bounds__(kLJThreads, 4) void learned_join_kernel(
         const int nout_item = uniform_i32(s_nout);
         __syncthreads();
         const int total = uniform_i32(s_pre[nr]);
-        const int first = chunk * kItemPos;
-        const int last = (first + kItemPos < total) ? first + kItemPos : total;
+        const bool direct = MODE == kLModeBox || direct_polygon(qinfo);
+        const int per = direct ? kItemPos : kChunk;  // item_positions(qinfo)
+        const int first = chunk * per;
+        const int last = (first + per < total) ? first + per : total;
         int4 info = make_int4(0, 0, 0, 0);
         double cx = 0, cy = 0;
         float E = 0.0f;
-        int ne_fixed = -1;  // edges staged once for the whole item (small single-part polygons)
-        Slabs fixed_slabs = {1, 0.0f, 0.0f};
         if (MODE != kLModeBox) {
             info = qinfo;
             cx = 0.5 * (box.x + box.z);
@@ -1472,9 +1551,8 @@ __global__ __launch_bounds__(kLJThreads, 4) void learned_join_kernel(
             cx = uniform_f64(cx);
             cy = uniform_f64(cy);
         }
-        const bool direct = MODE == kLModeBox || (info.z == 1 && info.y - info.x <= kEdgeCap + 1);
         if (direct) {
-            // Box queries and small single-part polygons: every thread scans
+            // Box queries and small polygons: every thread scans
             // kPosPerThread positions per round and refines its own candidates
             // at once against the item's slab lists (no candidate compaction).
             int32_t pos[kPosPerThread], orig[kPosPerThread];
@@ -1509,9 +1587,10 @@ __global__ __launch_bounds__(kLJThreads, 4) void learned_join_kernel(
             if (MODE != kLModeBox) {
                 const float ylo = (float)(box.y - cy), yhi = (float)(box.w - cy);
                 if (info.y - info.x <= kLJThreads) {
-                    S = stage_and_bin(info.x, info.y, cx, cy, ylo, yhi, R, Et, Ec, s_wsum, s_bstart, s_bcur, s_blist);
+                    S = stage_and_bin(info.x, info.y, cx, cy, ylo, yhi, R, Et, Ec, Ep, s_wsum, s_bstart, s_bcur,
+                                      s_blist);
                 } else {
-                    const int ne = stage_all_edges(info.x, info.y, cx, cy, R, Et, Ec, s_wsum);
+                    const int ne = stage_all_edges(info.x, info.y, cx, cy, R, Et, Ec, Ep, s_wsum);
                     S = build_slabs(Et, ne, ylo, yhi, s_bstart, s_bcur, s_blist);
                 }
             }
@@ -1537,8 +1616,12 @@ __global__ __launch_bounds__(kLJThreads, 4) void learned_join_kernel(
                     if (MODE != kLModeBox) {
                         bool esc = false;
                         if (inbox) {
-                            const int loc = refine_one(Et, Ec, s_bstart, s_blist, S, R, (float)(px[j] - cx),
-                                                       (float)(py[j] - cy), px[j], py[j], E, esc, n_orient, n_esc);
+                            const float pu = (float)(px[j] - cx), pv = (float)(py[j] - cy);
+                            const int loc = info.z == 1
+                                                ? refine_one(Et, Ec, s_bstart, s_blist, S, R, pu, pv, px[j], py[j], E,
+                                                             esc, n_orient, n_esc)
+                                                : refine_parts(Et, Ec, Ep, s_bstart, s_blist, S, R, pu, pv, px[j],
+                                                               py[j], E, esc, n_orient, n_esc);
                             keep = loc_pred<PRED>(loc);
                         }
                         // wave-uniform counters (scalar registers)
@@ -1592,20 +1675,10 @@ __global__ __launch_bounds__(kLJThreads, 4) void learned_join_kernel(
             if (ncand < kLJThreads && r0 + kLJThreads < last) continue;  // keep accumulating
             if (ncand == 0) continue;
             if (s_nout + ncand > kOutCap) flush();
-            if (MODE == kLModeBox) {
-                const int base = s_nout;
-                for (int k = tid; k < ncand; k += kLJThreads) outb[base + k] = make_int2(q, perm[cand[k]]);
-                __syncthreads();
-                if (tid == 0) {
-                    s_nout = base + ncand;
-                    s_ncand = 0;
-                }
-                __syncthreads();
-                continue;
-            }
             // 2. refine the round's candidates against the polygon
             const int32_t c0 = info.x, c1 = info.y;
-            int loc[kCandPerThread], par[kCandPerThread];
+            int loc[kCandPerThread];
+            unsigned par[kCandPerThread], bnd[kCandPerThread];
             bool done[kCandPerThread], esc[kCandPerThread];
             float pu[kCandPerThread], pv[kCandPerThread];
             double pxd[kCandPerThread], pyd[kCandPerThread];
@@ -1615,6 +1688,7 @@ __global__ __launch_bounds__(kLJThreads, 4) void learned_join_kernel(
                 const int k = tid + j * kLJThreads;
                 loc[j] = 0;
                 par[j] = 0;
+                bnd[j] = 0;
                 esc[j] = false;
                 done[j] = k >= ncand;
                 if (k < ncand) {
@@ -1632,16 +1706,7 @@ __global__ __launch_bounds__(kLJThreads, 4) void learned_join_kernel(
             }
             unsigned n_orient = 0;
             unsigned long long n_esc = 0;
-            if (info.z == 1 && c1 - c0 <= kEdgeCap + 1) {
-                if (ne_fixed < 0) {  // stage every edge and its slabs once for the item
-                    ne_fixed = stage_edges(c0, c1, -INFINITY, -INFINITY, INFINITY, cx, cy, R, L, 0, pu, pv, pxd, pyd,
-                                           E, loc, par, done, esc, n_orient, n_esc);
-                    fixed_slabs = build_slabs(Et, ne_fixed, (float)(box.y - cy), (float)(box.w - cy), s_bstart,
-                                              s_bcur, s_blist);
-                }
-                refine_slabs(Et, Ec, s_bstart, s_blist, fixed_slabs, R, pu, pv, pxd, pyd, E, loc, par, done, esc,
-                             n_orient, n_esc);
-            } else if (info.z == 1) {
+            if (info.z <= kMaskParts) {
                 exmin = wave_min(exmin);
                 eymin = wave_min(eymin);
                 eymax = wave_max(eymax);
@@ -1658,12 +1723,21 @@ __global__ __launch_bounds__(kLJThreads, 4) void learned_join_kernel(
                     ymx = fmax(ymx, s_ext[w2][2]);
                 }
                 __syncthreads();
-                const int ne = stage_edges(c0, c1, xmn, ymn, ymx, cx, cy, R, L, 0, pu, pv, pxd, pyd, E, loc, par,
-                                           done, esc, n_orient, n_esc);
-                const Slabs S = build_slabs(Et, ne, (float)(ymn - cy), (float)(ymx - cy), s_bstart, s_bcur, s_blist);
-                refine_slabs(Et, Ec, s_bstart, s_blist, S, R, pu, pv, pxd, pyd, E, loc, par, done, esc, n_orient,
-                             n_esc);
+                auto refine_all = [&](auto multi) {
+                    constexpr bool kMulti = decltype(multi)::value;
+                    const int ne = stage_edges<kMulti>(c0, c1, xmn, ymn, ymx, cx, cy, R, L, 0, pu, pv, pxd, pyd, E,
+                                                       par, bnd, done, esc, n_orient, n_esc);
+                    const Slabs S =
+                        build_slabs(Et, ne, (float)(ymn - cy), (float)(ymx - cy), s_bstart, s_bcur, s_blist);
+                    refine_slabs<kMulti>(Et, Ec, Ep, s_bstart, s_blist, S, R, pu, pv, pxd, pyd, E, par, bnd, done,
+                                         esc, n_orient, n_esc);
+                };
+                if (info.z == 1) refine_all(std::false_type{});
+                else refine_all(std::true_type{});
+#pragma unroll
+                for (int j = 0; j < kCandPerThread; ++j) loc[j] = mask_loc(par[j], bnd[j]);
             } else {
+                int run[kCandPerThread] = {};  // crossing parity of the part being streamed
                 float2* Vt = reinterpret_cast<float2*>(Et);
                 uint8_t* Ft = reinterpret_cast<uint8_t*>(Ec);
                 constexpr int kV = kEdgeCap;  // vertices per batch: 8 B + 1 B each fit the edge buffers
@@ -1681,11 +1755,11 @@ __global__ __launch_bounds__(kLJThreads, 4) void learned_join_kernel(
                         if (f & 2) {
 #pragma unroll
                             for (int j = 0; j < kCandPerThread; ++j) {
-                                if (!done[j] && par[j]) {
+                                if (!done[j] && run[j]) {
                                     loc[j] = 2;
                                     done[j] = true;
                                 }
-                                par[j] = 0;
+                                run[j] = 0;
                             }
                         }
                         if (f & 1) continue;
@@ -1693,10 +1767,10 @@ __global__ __launch_bounds__(kLJThreads, 4) void learned_join_kernel(
 #pragma unroll
                         for (int j = 0; j < kCandPerThread; ++j) {
                             if (done[j]) continue;
-                            if (edge_step_f32(pu[j], pv[j], a.x, a.y, b.x, b.y, E, par[j], n_orient)) {
+                            if (edge_step_f32(pu[j], pv[j], a.x, a.y, b.x, b.y, E, run[j], n_orient)) {
                                 ++n_esc;
                                 esc[j] = true;
-                                if (edge_step_f64(pxd[j], pyd[j], R.x[c - 1], R.y[c - 1], R.x[c], R.y[c], par[j])) {
+                                if (edge_step_f64(pxd[j], pyd[j], R.x[c - 1], R.y[c - 1], R.x[c], R.y[c], run[j])) {
                                     loc[j] = 1;
                                     done[j] = true;
                                 }
@@ -1705,7 +1779,9 @@ __global__ __launch_bounds__(kLJThreads, 4) void learned_join_kernel(
                     }
                 }
                 __syncthreads();
-                ne_fixed = -1;  // the edge buffers were reused as vertex buffers
+#pragma unroll
+                for (int j = 0; j < kCandPerThread; ++j)
+                    if (!done[j] && run[j]) loc[j] = 2;
             }
             st_orient += n_orient;
             st_esc += n_esc;
@@ -1714,7 +1790,6 @@ __global__ __launch_bounds__(kLJThreads, 4) void learned_join_kernel(
                 const int k = tid + j * kLJThreads;
                 st_escpairs += (unsigned)__popcll(__ballot(k < ncand && esc[j]));
                 if (k >= ncand) continue;
-                if (!done[j] && par[j]) loc[j] = 2;
                 if (loc_pred<PRED>(loc[j])) {
                     const int32_t orig = perm[cand[k]];
                     const int slot = atomicAdd(&s_nout, 1);

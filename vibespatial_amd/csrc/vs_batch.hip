@@ -1130,7 +1130,7 @@ int batched_intersects(const Polys& A, int64_t n_left, const Polys& B, int64_t n
         VS_LAUNCH_CHECK();
         VS_TRY(timing_end_public(s));
     }
-    VS_TRY(finish_pairs(W.fin_ws, W.ctl, n_left, capacity, true, out_l, out_r, d_result, s));
+    VS_TRY(finish_pairs(W.fin_ws, W.ctl, n_left, 0, capacity, true, out_l, out_r, d_result, s));
     hipLaunchKernelGGL(publish_batch_kernel, dim3(1), dim3(64), 0, s, W.cctl, W.ctl, d_result);
     VS_LAUNCH_CHECK();
     return VS_OK;

@@ -129,6 +129,11 @@ int sort_pairs_u32_dev_wide(uint32_t* keys, int32_t* vals, int64_t n, const unsi
                             int end_bit, void* ws, int64_t ws_bytes, hipStream_t s, int64_t* out_k, int64_t* out_v,
                             SortResult<uint32_t>* res);
 
+// Pairs (l, r) lexsorted into int64 out_l / out_r: radix passes over r's low
+// r_bits, then over l's low l_bits (n > 1, both bit counts > 0).
+int sort_lex_wide_u32(uint32_t* l, int32_t* r, int64_t n, const unsigned long long* d_n, int l_bits, int r_bits,
+                      void* ws, int64_t ws_bytes, hipStream_t s, int64_t* out_l, int64_t* out_r);
+
 // ---------------------------------------------------------------------------
 // Device helpers for 64-wide wavefronts.
 // ---------------------------------------------------------------------------

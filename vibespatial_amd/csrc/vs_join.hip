@@ -661,7 +661,7 @@ int vs_sjoin_points_polygons(const double* px, const double* py, int64_t n_point
     if (n_points > 0 && n_polys > 0)
         VS_TRY(vs::launch_traverse<vs::kModePip>(predicate, J.sx, J.sy, nullptr, J.perm, n_points, T, P, J,
                                                  capacity, s));
-    return vs::finish_pairs(J.fin_ws, J.ctl, n_points, capacity, true, out_left, out_right, d_result, s);
+    return vs::finish_pairs(J.fin_ws, J.ctl, n_points, 0, capacity, true, out_left, out_right, d_result, s);
 }
 
 int vs_sjoin_points_polygons_noalloc(const double* px, const double* py, int64_t n_points, const double* x,
@@ -719,7 +719,8 @@ int vs_query_boxes(const double* query_boxes, int64_t n_queries, const vs_tree_l
         VS_TRY(vs::launch_traverse<vs::kModeBox>(VS_PRED_INTERSECTS, nullptr, nullptr, qb, J.perm, n_queries, T, P,
                                                  J, capacity, s, one_box));
     }
-    return vs::finish_pairs(J.fin_ws, J.ctl, n_queries, capacity, sort != 0, out_left, out_right, d_result, s);
+    return vs::finish_pairs(J.fin_ws, J.ctl, n_queries, layout->n_items, capacity, sort != 0, out_left, out_right,
+                             d_result, s);
 }
 
 }  // extern "C"

@@ -27,11 +27,12 @@ void fill_i32(int32_t* p, int64_t n, int32_t v, hipStream_t s);
 // finish_stage carves from the finish workspace (left ids as u32, right ids as
 // i32, `capacity` slots, ctl->staged the count); finish_pairs turns them into
 // int64 output sorted by left id (and by right id within a left id when
-// sort_right) and publishes d_result[0..3].
+// sort_right) and publishes d_result[0..3].  n_right: right ids are below it
+// (0: not known); it lets a join of many hits per left row sort by both ids.
 int64_t finish_workspace_bytes(int64_t capacity);
 void finish_stage(void* fin_ws, int64_t capacity, uint32_t** stage_l, int32_t** stage_r);
-int finish_pairs(void* fin_ws, JoinCtl* ctl, int64_t n_left, int64_t capacity, bool sort_right, int64_t* out_l,
-                 int64_t* out_r, int64_t* d_result, hipStream_t s);
+int finish_pairs(void* fin_ws, JoinCtl* ctl, int64_t n_left, int64_t n_right, int64_t capacity, bool sort_right,
+                 int64_t* out_l, int64_t* out_r, int64_t* d_result, hipStream_t s);
 
 // Per-coordinate flags of the refine layout: bit0 first coordinate of a ring,
 // bit1 first coordinate of a part.

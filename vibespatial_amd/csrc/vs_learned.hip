@@ -2148,7 +2148,7 @@ int learned_query_t(int mode, int pred, const double4* qbox, int64_t nq, const L
         VS_LAUNCH_CHECK();
         VS_TRY(timing_end_public(s));
     }
-    VS_TRY(finish_pairs(Q.fin_ws, Q.ctl, n_left, capacity, sort, out_l, out_r, d_result, s));
+    VS_TRY(finish_pairs(Q.fin_ws, Q.ctl, n_left, mode == kLModePip ? nq : V.n, capacity, sort, out_l, out_r, d_result, s));
     hipLaunchKernelGGL(publish_learned_kernel, dim3(1), dim3(64), 0, s, Q.ctl, Q.cstat, B.meta, d_result);
     VS_LAUNCH_CHECK();
     return VS_OK;

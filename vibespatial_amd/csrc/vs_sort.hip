@@ -15,6 +15,8 @@
 //          mask of equal digits), combines waves through LDS counters, writes the
 //          tile into LDS in digit order and then streams it out so each digit
 //          run is written contiguously.
+#include <utility>
+
 #include "vs_internal.h"
 
 namespace vs {
@@ -434,6 +436,47 @@ int sort_pairs_nocopy(K* keys, int32_t* vals, int64_t n, const unsigned long lon
     res->vals = vi;
     res->alt_keys = ko;
     res->alt_vals = vo;
+    return VS_OK;
+}
+
+// Sorts the pairs (l, r) by r's bits [0, r_bits), then by l's bits [0, l_bits)
+// (stable, so lexsorted by (l, r)); the last pass writes int64 pairs to out_l /
+// out_r.  Same workspace as the u32 pair sort; r >= 0, r_bits and l_bits > 0.
+int sort_lex_wide_u32(uint32_t* l, int32_t* r, int64_t n, const unsigned long long* d_n, int l_bits, int r_bits,
+                      void* ws, int64_t ws_bytes, hipStream_t s, int64_t* out_l, int64_t* out_r) {
+    VS_REQUIRE(n > 1 && n < (int64_t)INT32_MAX, "sort_lex: n=%lld out of range", (long long)n);
+    VS_REQUIRE(l_bits > 0 && l_bits <= 32 && r_bits > 0 && r_bits <= 32, "sort_lex: bad bit counts");
+    VS_REQUIRE(ws_bytes >= sort_workspace_bytes_t<uint32_t>(n), "sort_lex: workspace too small");
+    const int nb = (int)ceil_div(n, kRsTile);
+    Carver c(ws);
+    uint32_t* lo = c.take<uint32_t>(n);
+    uint32_t* ro = reinterpret_cast<uint32_t*>(c.take<int32_t>(n));
+    int32_t* hist = c.take<int32_t>((int64_t)nb * kRsBins);
+    void* scan_ws = c.take<char>(scan_workspace_bytes((int64_t)nb * kRsBins));
+    uint32_t* li = l;
+    uint32_t* ri = reinterpret_cast<uint32_t*>(r);
+    for (int side = 0; side < 2; ++side) {
+        const int bits = side == 0 ? r_bits : l_bits;
+        for (int shift = 0; shift < bits; shift += 8) {
+            const int dmask = (1 << (bits - shift < 8 ? bits - shift : 8)) - 1;
+            const uint32_t* key = side == 0 ? ri : li;
+            const int32_t* val = reinterpret_cast<const int32_t*>(side == 0 ? li : ri);
+            hipLaunchKernelGGL(rs_hist_kernel<uint32_t>, dim3(nb), dim3(kRsThreads), 0, s, key, n, d_n, shift, dmask,
+                               hist, nb);
+            VS_LAUNCH_CHECK();
+            VS_TRY(exclusive_scan_i32(hist, hist, (int64_t)nb * kRsBins, nullptr, scan_ws, s));
+            if (side == 1 && shift + 8 >= bits) {
+                hipLaunchKernelGGL((rs_scatter_kernel<uint32_t, true>), dim3(nb), dim3(kRsThreads), 0, s, key, val,
+                                   out_l, out_r, n, d_n, shift, dmask, hist, nb);
+            } else {
+                hipLaunchKernelGGL((rs_scatter_kernel<uint32_t, false>), dim3(nb), dim3(kRsThreads), 0, s, key, val,
+                                   side == 0 ? ro : lo, side == 0 ? lo : ro, n, d_n, shift, dmask, hist, nb);
+            }
+            VS_LAUNCH_CHECK();
+            std::swap(li, lo);
+            std::swap(ri, ro);
+        }
+    }
     return VS_OK;
 }
 

@@ -346,6 +346,28 @@ int vs_learned_query_polygons(const void* index, int64_t n_points, int32_t key_b
                               int64_t* out_left, int64_t* out_right, int64_t* d_result, void* workspace,
                               int64_t workspace_bytes, void* stream);
 
+/* The two queries above in two steps, for callers that do not know how many
+ * pairs to expect.  vs_learned_query_plan finds the rank ranges of every query
+ * (boxes n_queries x 4; for polygon queries also their offsets, else null) into
+ * `plan` and writes d_positions[0] (device): the index positions the scan will
+ * visit, an upper bound of the pairs.  vs_learned_query_run scans the planned
+ * ranges with a capacity chosen from it: offsets null: a box query (x, y null,
+ * n_parts / n_rings / n_coords 0), else polygon queries with `predicate` as for
+ * vs_learned_query_polygons.  A plan holds for the same index, queries and
+ * offsets and may be run again (with a larger capacity). */
+int64_t vs_learned_plan_bytes(int64_t n_queries);
+int vs_learned_query_plan(const void* index, int64_t n_points, int32_t key_bytes, int32_t n_leaves,
+                          const double* boxes, const int32_t* geom_offsets, const int32_t* part_offsets,
+                          const int32_t* ring_offsets, int64_t n_queries, int32_t lookup_mode, int64_t* d_positions,
+                          void* plan, int64_t plan_bytes, void* stream);
+int64_t vs_learned_run_workspace_bytes(int64_t n_coords, int64_t capacity);
+int vs_learned_query_run(const void* index, int64_t n_points, int32_t key_bytes, int32_t n_leaves,
+                         const double* boxes, const double* x, const double* y, const int32_t* geom_offsets,
+                         const int32_t* part_offsets, const int32_t* ring_offsets, int64_t n_queries, int64_t n_parts,
+                         int64_t n_rings, int64_t n_coords, int32_t predicate, int64_t capacity, int32_t sort,
+                         int64_t* out_left, int64_t* out_right, int64_t* d_result, void* plan, int64_t plan_bytes,
+                         void* workspace, int64_t workspace_bytes, void* stream);
+
 int64_t vs_sjoin_points_polygons_learned_workspace_bytes(int64_t n_points, int64_t n_polys, int64_t n_coords,
                                                          int64_t capacity);
 

@@ -20,6 +20,9 @@
 //      global memory (merge by co-rank: each element's output slot is its
 //      index in its own half plus its rank in the other half).
 //
+// A stage with room for many pairs per left row (kLexSlots) is sorted by both
+// ids instead: radix passes over the right ids, then over the left ids.
+//
 // Pairs with the same left id come from one join and have distinct right ids,
 // but the merge is stable anyway (lower bound from the left half, upper bound
 // from the right half).
@@ -353,10 +356,12 @@ static int bits_for(int64_t n) {
 }
 
 // Slots per left row from which the pairs are sorted by both ids instead of by
-// left id and then run by run: there most runs pass kShortRun, and the block
-// sorts of long runs move 2.3e9 ids/s where a radix pass moves 2e11 B/s x its
-// 16 B (51M pairs in 50k runs: 22 ms of long runs against 0.8 ms for three more
-// passes).  Below it the short runs' registers are cheaper than the passes.
+// left id and then run by run: there most runs pass kShortRun and would go
+// through the block sorts of long runs (2.3e9 ids/s), where a further radix pass
+// over the right ids takes its 20 B per pair at 4 TB/s.  51M pairs in 50k runs:
+// 22 ms of long runs against 0.8 ms of passes (index build + box query 25.2 ->
+// 6.7 ms); 5M pairs in 20k runs, contains query 4.7 -> 2.1 ms.  Below it the
+// short runs, sorted in registers in one pass, are cheaper than three passes.
 constexpr int64_t kLexSlots = 32;
 
 int finish_pairs(void* fin_ws, JoinCtl* ctl, int64_t n_left, int64_t n_right, int64_t capacity, bool sort_right,

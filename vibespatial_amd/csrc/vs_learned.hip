@@ -1867,6 +1867,10 @@ __global__ void publish_learned_kernel(const JoinCtl* __restrict__ ctl, const un
     }
 }
 
+__global__ void publish_positions_kernel(const unsigned long long* __restrict__ cst, int64_t* __restrict__ out) {
+    if (threadIdx.x == 0) out[0] = (int64_t)cst[3];
+}
+
 // ---------------------------------------------------------------------------
 // Host orchestration
 // ---------------------------------------------------------------------------
@@ -2056,7 +2060,8 @@ struct QueryBufs {
 // typical covers; items beyond the map fall back to a binary search.
 inline int64_t item_cap_for(int64_t nq, int64_t n_left) { return 2 * nq + (8 * n_left) / kItemPos + 1024; }
 
-QueryBufs carve_query(Carver& c, int64_t nq, int64_t n_left, int64_t capacity) {
+// The part of a query that needs no pair capacity: covers, rank ranges, items.
+QueryBufs carve_plan(Carver& c, int64_t nq, int64_t n_left) {
     QueryBufs Q;
     Q.item_cap = item_cap_for(nq, n_left);
     Q.item_rec = c.take<int4>(Q.item_cap);
@@ -2076,10 +2081,20 @@ QueryBufs carve_query(Carver& c, int64_t nq, int64_t n_left, int64_t capacity) {
     Q.cstat = c.take<unsigned long long>(4);
     Q.scan_ws = c.take<char>(scan_workspace_bytes(nq));
     Q.ctl = c.take<JoinCtl>(1);
-    Q.fin_ws = c.take<char>(finish_workspace_bytes(capacity));
+    Q.fin_ws = nullptr;
     Q.stage_l = nullptr;
     Q.stage_r = nullptr;
-    if (c.base) finish_stage(Q.fin_ws, capacity, &Q.stage_l, &Q.stage_r);
+    return Q;
+}
+
+void carve_finish_ws(Carver& c, int64_t capacity, QueryBufs* Q) {
+    Q->fin_ws = c.take<char>(finish_workspace_bytes(capacity));
+    if (c.base) finish_stage(Q->fin_ws, capacity, &Q->stage_l, &Q->stage_r);
+}
+
+QueryBufs carve_query(Carver& c, int64_t nq, int64_t n_left, int64_t capacity) {
+    QueryBufs Q = carve_plan(c, nq, n_left);
+    carve_finish_ws(c, capacity, &Q);
     return Q;
 }
 
@@ -2096,12 +2111,12 @@ int cover_cells_launch(int mode, const double4* qbox, int64_t nq, const IndexBuf
     return VS_OK;
 }
 
+// First half of a query: rank ranges of every cover, work items in their
+// order, Q.cstat[3] = positions the scan will visit (a bound on its pairs).
 // cells_ready: cover_cells_launch already ran on `s` for these queries.
 template <class K>
-int learned_query_t(int mode, int pred, const double4* qbox, int64_t nq, const LearnedView<K>& V,
-                    const IndexBufs<K>& B, const RefineView& R, int64_t n_left, int64_t capacity, bool sort,
-                    const QueryBufs& Q, int64_t* out_l, int64_t* out_r, int64_t* d_result, hipStream_t s,
-                    bool cells_ready = false) {
+int learned_plan_t(int mode, const double4* qbox, int64_t nq, const LearnedView<K>& V, const IndexBufs<K>& B,
+                   const RefineView& R, const QueryBufs& Q, hipStream_t s, bool cells_ready = false) {
     ctl_reset(Q.ctl, s, Q.cstat, 4);
     VS_LAUNCH_CHECK();
     if (nq > 0) {
@@ -2123,6 +2138,17 @@ int learned_query_t(int mode, int pred, const double4* qbox, int64_t nq, const L
         hipLaunchKernelGGL(item_map_kernel, dim3(gq), dim3(256), 0, s, Q.item_off, Q.n_items_sorted, Q.order,
                            Q.cost_key, Q.nranges, nq, Q.item_rec, Q.item_cap);
         VS_LAUNCH_CHECK();
+    }
+    return VS_OK;
+}
+
+// Second half: the scan and refine of the planned items (Q.ctl cleared by the
+// caller or by learned_plan_t), then the finish pass.
+template <class K>
+int learned_run_t(int mode, int pred, const double4* qbox, int64_t nq, int64_t n_points, const IndexBufs<K>& B,
+                  const RefineView& R, int64_t n_left, int64_t capacity, bool sort, const QueryBufs& Q,
+                  int64_t* out_l, int64_t* out_r, int64_t* d_result, hipStream_t s) {
+    if (nq > 0) {
         int dev = 0, cus = 256;
         if (hipGetDevice(&dev) == hipSuccess) {
             int v = 0;
@@ -2148,10 +2174,20 @@ int learned_query_t(int mode, int pred, const double4* qbox, int64_t nq, const L
         VS_LAUNCH_CHECK();
         VS_TRY(timing_end_public(s));
     }
-    VS_TRY(finish_pairs(Q.fin_ws, Q.ctl, n_left, mode == kLModePip ? nq : V.n, capacity, sort, out_l, out_r, d_result, s));
+    VS_TRY(finish_pairs(Q.fin_ws, Q.ctl, n_left, mode == kLModePip ? nq : n_points, capacity, sort, out_l, out_r,
+                        d_result, s));
     hipLaunchKernelGGL(publish_learned_kernel, dim3(1), dim3(64), 0, s, Q.ctl, Q.cstat, B.meta, d_result);
     VS_LAUNCH_CHECK();
     return VS_OK;
+}
+
+template <class K>
+int learned_query_t(int mode, int pred, const double4* qbox, int64_t nq, const LearnedView<K>& V,
+                    const IndexBufs<K>& B, const RefineView& R, int64_t n_left, int64_t capacity, bool sort,
+                    const QueryBufs& Q, int64_t* out_l, int64_t* out_r, int64_t* d_result, hipStream_t s,
+                    bool cells_ready = false) {
+    VS_TRY(learned_plan_t<K>(mode, qbox, nq, V, B, R, Q, s, cells_ready));
+    return learned_run_t<K>(mode, pred, qbox, nq, V.n, B, R, n_left, capacity, sort, Q, out_l, out_r, d_result, s);
 }
 
 // The learned join on a carved workspace (fork: the index build's side
@@ -2366,6 +2402,98 @@ int vs_learned_query_polygons(const void* index, int64_t n_points, int32_t key_b
     return vs::learned_query_t<uint64_t>(vs::kLModePipQ, predicate, qb, n_polys,
                                          vs::view_of<uint64_t>(B, n_points, n_leaves, lookup_mode), B, R, n_polys,
                                          capacity, sort != 0, Q, out_left, out_right, d_result, s);
+}
+
+int64_t vs_learned_plan_bytes(int64_t n_queries) {
+    vs::Carver c(nullptr);
+    vs::carve_plan(c, n_queries, n_queries);
+    return c.bytes;
+}
+
+int vs_learned_query_plan(const void* index, int64_t n_points, int32_t key_bytes, int32_t n_leaves,
+                          const double* boxes, const int32_t* geom_offsets, const int32_t* part_offsets,
+                          const int32_t* ring_offsets, int64_t n_queries, int32_t lookup_mode, int64_t* d_positions,
+                          void* plan, int64_t plan_bytes, void* stream) {
+    vs::clear_error();
+    VS_REQUIRE(key_bytes == 4 || key_bytes == 8, "vs_learned_query_plan: key_bytes must be 4 or 8");
+    VS_REQUIRE(n_queries >= 0 && n_queries < (int64_t)INT32_MAX, "vs_learned_query_plan: n_queries out of range");
+    VS_REQUIRE(lookup_mode >= 0 && lookup_mode <= 2, "vs_learned_query_plan: lookup_mode in {0, 1, 2}");
+    VS_REQUIRE((geom_offsets != nullptr) == (part_offsets != nullptr) &&
+                   (geom_offsets != nullptr) == (ring_offsets != nullptr),
+               "vs_learned_query_plan: all polygon offsets or none");
+    VS_REQUIRE(d_positions != nullptr, "vs_learned_query_plan: null result");
+    VS_REQUIRE(plan_bytes >= vs_learned_plan_bytes(n_queries), "vs_learned_query_plan: plan too small");
+    vs::Carver ci(const_cast<void*>(index));
+    vs::Carver cp(plan);
+    const vs::QueryBufs Q = vs::carve_plan(cp, n_queries, n_queries);
+    const vs::RefineView R = {nullptr, nullptr, geom_offsets, part_offsets, ring_offsets, nullptr};
+    hipStream_t s = vs::stream_of(stream);
+    const double4* qb = reinterpret_cast<const double4*>(boxes);
+    const int mode = geom_offsets ? vs::kLModePipQ : vs::kLModeBox;
+    if (key_bytes == 4) {
+        const auto B = vs::carve_index<uint32_t>(ci, n_points, n_leaves);
+        VS_TRY(vs::learned_plan_t<uint32_t>(mode, qb, n_queries,
+                                            vs::view_of<uint32_t>(B, n_points, n_leaves, lookup_mode), B, R, Q, s));
+    } else {
+        const auto B = vs::carve_index<uint64_t>(ci, n_points, n_leaves);
+        VS_TRY(vs::learned_plan_t<uint64_t>(mode, qb, n_queries,
+                                            vs::view_of<uint64_t>(B, n_points, n_leaves, lookup_mode), B, R, Q, s));
+    }
+    hipLaunchKernelGGL(vs::publish_positions_kernel, dim3(1), dim3(64), 0, s, Q.cstat, d_positions);
+    VS_LAUNCH_CHECK();
+    return VS_OK;
+}
+
+int64_t vs_learned_run_workspace_bytes(int64_t n_coords, int64_t capacity) {
+    vs::Carver c(nullptr);
+    vs::QueryBufs Q = {};
+    c.take<uint8_t>(n_coords);
+    vs::carve_finish_ws(c, capacity, &Q);
+    return c.bytes;
+}
+
+int vs_learned_query_run(const void* index, int64_t n_points, int32_t key_bytes, int32_t n_leaves,
+                         const double* boxes, const double* x, const double* y, const int32_t* geom_offsets,
+                         const int32_t* part_offsets, const int32_t* ring_offsets, int64_t n_queries, int64_t n_parts,
+                         int64_t n_rings, int64_t n_coords, int32_t predicate, int64_t capacity, int32_t sort,
+                         int64_t* out_left, int64_t* out_right, int64_t* d_result, void* plan, int64_t plan_bytes,
+                         void* workspace, int64_t workspace_bytes, void* stream) {
+    vs::clear_error();
+    VS_REQUIRE(key_bytes == 4 || key_bytes == 8, "vs_learned_query_run: key_bytes must be 4 or 8");
+    VS_REQUIRE(n_queries >= 0 && n_queries < (int64_t)INT32_MAX, "vs_learned_query_run: n_queries out of range");
+    VS_REQUIRE(n_coords >= 0 && n_coords < (int64_t)INT32_MAX, "vs_learned_query_run: n_coords out of range");
+    VS_REQUIRE(capacity >= 0 && capacity < (int64_t)INT32_MAX, "vs_learned_query_run: capacity out of range");
+    VS_REQUIRE((geom_offsets != nullptr) == (part_offsets != nullptr) &&
+                   (geom_offsets != nullptr) == (ring_offsets != nullptr),
+               "vs_learned_query_run: all polygon offsets or none");
+    VS_REQUIRE(!geom_offsets || predicate == VS_PRED_CONTAINS || predicate == VS_PRED_CONTAINS_PROPERLY ||
+                   predicate == VS_PRED_COVERS || predicate == VS_PRED_INTERSECTS || predicate == VS_PRED_TOUCHES,
+               "vs_learned_query_run: unsupported predicate %d", predicate);
+    VS_REQUIRE(d_result != nullptr, "vs_learned_query_run: null result");
+    VS_REQUIRE(plan_bytes >= vs_learned_plan_bytes(n_queries), "vs_learned_query_run: plan too small");
+    VS_REQUIRE(workspace_bytes >= vs_learned_run_workspace_bytes(n_coords, capacity),
+               "vs_learned_query_run: workspace too small");
+    vs::Carver ci(const_cast<void*>(index));
+    vs::Carver cp(plan);
+    vs::Carver cw(workspace);
+    vs::QueryBufs Q = vs::carve_plan(cp, n_queries, n_queries);
+    uint8_t* flags = cw.take<uint8_t>(n_coords);
+    vs::carve_finish_ws(cw, capacity, &Q);
+    hipStream_t s = vs::stream_of(stream);
+    const int mode = geom_offsets ? vs::kLModePipQ : vs::kLModeBox;
+    if (geom_offsets) VS_TRY(vs::build_refine_flags(part_offsets, ring_offsets, n_parts, n_rings, n_coords, flags, s));
+    const vs::RefineView R = {x, y, geom_offsets, part_offsets, ring_offsets, flags};
+    const double4* qb = reinterpret_cast<const double4*>(boxes);
+    vs::ctl_reset(Q.ctl, s);  // a plan may be run more than once
+    VS_LAUNCH_CHECK();
+    if (key_bytes == 4) {
+        const auto B = vs::carve_index<uint32_t>(ci, n_points, n_leaves);
+        return vs::learned_run_t<uint32_t>(mode, predicate, qb, n_queries, n_points, B, R, n_queries, capacity,
+                                           sort != 0, Q, out_left, out_right, d_result, s);
+    }
+    const auto B = vs::carve_index<uint64_t>(ci, n_points, n_leaves);
+    return vs::learned_run_t<uint64_t>(mode, predicate, qb, n_queries, n_points, B, R, n_queries, capacity, sort != 0,
+                                       Q, out_left, out_right, d_result, s);
 }
 
 int64_t vs_sjoin_points_polygons_learned_workspace_bytes(int64_t n_points, int64_t n_polys, int64_t n_coords,

@@ -467,6 +467,10 @@ def _learned_stats(h, cap, retries) -> LearnedStats:
 
 LOOKUP_MODES = {"learned": 0, "leaves": 1, "binary": 2}
 
+# Largest output a planned query allocates from its scan length (24 B per slot
+# with the staged pairs, 16 B for the sort's alternates): 2^28 slots, 11 GB.
+POSITION_LIMIT = 2**28
+
 
 def sjoin_points_polygons_learned(Q: DevicePoints, P: DevicePolygons, bounds: torch.Tensor, predicate: str = "within",
                                   capacity: int | None = None, train_iters: int = 16, lookup: str = "learned"):
@@ -565,6 +569,43 @@ class LearnedPointIndex:
         s = st.cpu().tolist()
         return out[:m], {"probes": s[0], "mlp_fallbacks": s[1], "window_fallbacks": s[2]}
 
+    def _planned_query(self, boxes: torch.Tensor, P: DevicePolygons | None, predicate, lookup: str, sort: bool):
+        """query_boxes (P None) / query_polygons without a caller capacity: the
+        plan's scan length, an upper bound of the pairs, sizes the output, so
+        the scan runs once.  A bound over POSITION_LIMIT is not allocated: the
+        planned scan then runs twice, the first time to count."""
+        dev = require_gpu()
+        L = lib()
+        nq = int(boxes.shape[0])
+        offsets = [None] * 3 if P is None else [P.geom_offsets, P.part_offsets, P.ring_offsets]
+        xy = [None] * 2 if P is None else [P.x, P.y]
+        sizes = [0] * 3 if P is None else [P.n_parts, P.n_rings, P.n_coords]
+        index = [ptr(self.buf), self.n, self.key_bytes, self.n_leaves, ptr(boxes)]
+        plan = _ws(L.vs_learned_plan_bytes(nq), dev)
+        pos = torch.empty(1, dtype=torch.int64, device=dev)
+        check(L.vs_learned_query_plan(*index, *(ptr(t) for t in offsets), nq, LOOKUP_MODES[lookup], ptr(pos),
+                                      ptr(plan), plan.numel(), stream()), "vs_learned_query_plan")
+        bound = int(pos.item())
+        cap = max(1024, bound if bound <= POSITION_LIMIT else min(4 * nq, PAIR_LIMIT))
+        retries = 0
+        while True:
+            ws = _ws(L.vs_learned_run_workspace_bytes(sizes[2], cap), dev)
+            out_l = torch.empty(cap, dtype=torch.int64, device=dev)
+            out_r = torch.empty(cap, dtype=torch.int64, device=dev)
+            res = torch.zeros(16, dtype=torch.int64, device=dev)
+            check(L.vs_learned_query_run(*index, *(ptr(t) for t in xy + offsets), nq, *sizes,
+                                         PRED["intersects" if P is None else predicate], cap, int(bool(sort)),
+                                         ptr(out_l), ptr(out_r), ptr(res), ptr(plan), plan.numel(), ptr(ws),
+                                         ws.numel(), stream()), "vs_learned_query_run")
+            h = res.cpu().tolist()
+            if h[1] <= cap:
+                return out_l[: h[0]], out_r[: h[0]], _learned_stats(h, cap, retries)
+            if h[1] > PAIR_LIMIT:
+                raise _PairLimit(h[1])
+            del ws, out_l, out_r
+            cap = int(h[1])
+            retries += 1
+
     def query_boxes(self, boxes: torch.Tensor, lookup: str = "learned", capacity: int | None = None,
                     sort: bool = True):
         """(box, point) pairs with the point in the box (inclusive); lexsorted
@@ -573,8 +614,10 @@ class LearnedPointIndex:
         L = lib()
 
         def run(bx):
+            if capacity is None:
+                return self._planned_query(bx, None, None, lookup, sort)
             nb = int(bx.shape[0])
-            cap = int(capacity) if capacity is not None else max(1024, 4 * nb)
+            cap = int(capacity)
             cap = min(cap, PAIR_LIMIT)
             retries = 0
             while True:
@@ -606,8 +649,13 @@ class LearnedPointIndex:
         L = lib()
         if predicate not in ("contains", "contains_properly", "covers", "intersects", "touches"):
             raise NotImplementedError(f"polygon x point predicate {predicate!r}")
+        if capacity is None:
+            try:
+                return self._planned_query(bounds, P, predicate, lookup, sort)
+            except _PairLimit as e:
+                raise OverflowError(f"{e.args[0]} pairs exceed the int32 pair limit of one call") from None
         nq = len(P)
-        cap = int(capacity) if capacity is not None else max(1024, 4 * nq)
+        cap = int(capacity)
         cap = min(cap, PAIR_LIMIT)
         retries = 0
         while True:

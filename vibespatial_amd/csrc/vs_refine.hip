@@ -44,10 +44,11 @@ __device__ __forceinline__ int loc_keep(int pred, int loc) {
 //         intersects of a query polygon over tree points.
 // Pairs are visited in order[t] when given (polygon pairs grouped by right
 // row, so the lanes of a wave mostly share one right polygon).  Polygon pairs
-// whose coordinate counts multiply to more than the heavy-pair threshold go to `heavy`
-// (count in *n_heavy) for refine_heavy_kernel, one wave per pair; pairs the
-// cheap tests leave undecided go to `undecided` (count in *n_undecided) for
-// refine_relate_kernel, so this kernel carries none of the full relation's
+// whose coordinate counts multiply to more than the heavy-pair threshold, and
+// those the cheap tests leave undecided, go to `heavy` (count in *n_heavy) for
+// refine_heavy_kernel, one wave per pair, which decides all but rows whose
+// boundaries touch without crossing; those go to `undecided` for
+// refine_relate_kernel, so neither of the others carries the full relation's
 // registers.  At 2^8 small pairs (box x box: 25) stay one per lane; one lane
 // walking the edge pairs of two many-vertex polygons leaves the rest of its
 // wave idle, so those go one wave per pair (100k x 100k star polygons,
@@ -63,8 +64,6 @@ __global__ __launch_bounds__(256) void refine_pairs_kernel(int mode, int pred, c
                                                           const double* __restrict__ py, Polys A, Polys B,
                                                           int32_t* __restrict__ keep, int32_t* __restrict__ heavy,
                                                           unsigned long long* __restrict__ n_heavy,
-                                                          int32_t* __restrict__ undecided,
-                                                          unsigned long long* __restrict__ n_undecided,
                                                           int64_t heavy_pair) {
     for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < n; t += (int64_t)gridDim.x * 256) {
         const int64_t i = order ? (int64_t)order[t] : t;
@@ -80,27 +79,31 @@ __global__ __launch_bounds__(256) void refine_pairs_kernel(int mode, int pred, c
             k = 0;  // decided by refine_heavy_kernel
         } else {
             const int f = polygon_predicate_fast(pred, A, l, B, r);
-            if (f < 0) undecided[atomicAdd(n_undecided, 1ull)] = (int32_t)i;
+            if (f < 0) heavy[atomicAdd(n_heavy, 1ull)] = (int32_t)i;
             k = f > 0 ? 1 : 0;
         }
         keep[i] = k;
     }
 }
 
-// One wave per heavy polygon pair (grid-stride over the device count).
-__global__ __launch_bounds__(256) void refine_heavy_kernel(int pred, const int64_t* __restrict__ left,
+// One wave per heavy polygon pair (grid-stride over the device count).  The
+// pair's row numbers are made scalar, so its offsets come by scalar loads; the
+// register cap (four waves per SIMD) hides part of the offsets' load chain.
+__global__ __launch_bounds__(256, 4) void refine_heavy_kernel(int pred, const int64_t* __restrict__ left,
                                                           const int64_t* __restrict__ right,
                                                           const int32_t* __restrict__ heavy,
                                                           const unsigned long long* __restrict__ n_heavy, Polys A,
                                                           Polys B, int32_t* __restrict__ keep,
                                                           int32_t* __restrict__ undecided,
                                                           unsigned long long* __restrict__ n_undecided) {
+    __shared__ WaveEdgeLds lds[4];
     const int lane = threadIdx.x & 63;
     const int64_t m = (int64_t)*n_heavy;
     const int64_t waves = (int64_t)gridDim.x * 4;
-    for (int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); w < m; w += waves) {
+    const int wid = uniform_i32(threadIdx.x >> 6);
+    for (int64_t w = (int64_t)blockIdx.x * 4 + wid; w < m; w += waves) {
         const int64_t i = heavy[w];
-        const int f = wave_polygon_predicate_fast(pred, A, left[i], B, right[i], lane);
+        const int f = wave_polygon_predicate_fast(pred, A, left[i], B, right[i], lds[wid], lane);
         if (lane == 0) {
             keep[i] = f > 0 ? 1 : 0;
             if (f < 0) undecided[atomicAdd(n_undecided, 1ull)] = (int32_t)i;
@@ -108,7 +111,7 @@ __global__ __launch_bounds__(256) void refine_heavy_kernel(int pred, const int64
     }
 }
 
-// The full relation for the pairs the cheap tests left undecided, one wave
+// The full relation for the pairs the other kernels left undecided, one wave
 // per pair (grid-stride over the device count; lanes split the edges).
 __global__ __launch_bounds__(256) void refine_relate_kernel(int pred, const int64_t* __restrict__ left,
                                                            const int64_t* __restrict__ right,
@@ -315,7 +318,7 @@ int vs_refine_pairs(int32_t mode, int32_t predicate, const int64_t* left, const 
         }
         const int grid = (int)std::min<int64_t>(vs::ceil_div(n_pairs, 256), 16384);
         hipLaunchKernelGGL(vs::refine_pairs_kernel, dim3(grid), dim3(256), 0, s, mode, predicate, left, right,
-                           n_pairs, ord, px, py, A, B, keep, heavy, n_heavy, undecided, n_undecided, heavy_pair);
+                           n_pairs, ord, px, py, A, B, keep, heavy, n_heavy, heavy_pair);
         VS_LAUNCH_CHECK();
         if (mode == 1) {
             const int hgrid = (int)std::min<int64_t>(vs::ceil_div(n_pairs, 4), 2048);

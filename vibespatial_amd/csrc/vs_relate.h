@@ -28,6 +28,7 @@
 
 #include "vs_distance.h"
 #include "vs_exact.h"
+#include "vs_internal.h"
 #include "vs_polys.h"
 
 namespace vs {
@@ -253,9 +254,9 @@ struct Relation {
     bool touch;          // the boundaries meet
 };
 
-VS_HD Relation relate_polygons(const Polys& A, int64_t ra, const Polys& B, int64_t rb) {
-    const RelSide sa = relate_side(A, ra, B, rb, true);
-    const RelSide sb = relate_side(B, rb, A, ra, false);
+// The relation from the pieces of both boundaries (sa: A's pieces, with the
+// contact of the boundaries; sb: B's).
+VS_HD Relation merge_sides(const RelSide& sa, const RelSide& sb) {
     Relation R;
     const bool cross = sa.cross || sb.cross;
     R.interiors_meet = cross || sa.in_int || sb.in_int || sa.same || sb.same;
@@ -263,6 +264,11 @@ VS_HD Relation relate_polygons(const Polys& A, int64_t ra, const Polys& B, int64
     R.b_in_a = !cross && !sb.in_ext && !sa.in_int && sb.all_in;
     R.touch = sa.touch;
     return R;
+}
+
+VS_HD Relation relate_polygons(const Polys& A, int64_t ra, const Polys& B, int64_t rb) {
+    const RelSide sa = relate_side(A, ra, B, rb, true);
+    return merge_sides(sa, relate_side(B, rb, A, ra, false));
 }
 
 VS_HD double4 row_box(const Polys& P, int64_t row) {
@@ -339,73 +345,255 @@ VS_HD bool polygon_predicate(int pred, const Polys& A, int64_t ra, const Polys& 
 }
 
 // ---------------------------------------------------------------------------
-// One wave per pair, for pairs of large rows: lanes split the first row's
-// edges (each lane against every edge of the other row), votes decide.
+// One wave per pair, for pairs of large rows.
 // ---------------------------------------------------------------------------
 __device__ inline int32_t row_coords(const Polys& P, int64_t row) {
     return P.ring[P.part[P.geom[row + 1]]] - P.ring[P.part[P.geom[row]]];
 }
 
-// mode 0: some pair of edges touches (segments_touch); 1: some pair crosses
-// properly.
-__device__ inline bool wave_any_edge_pair(int mode, const Polys& A, int64_t ra, const Polys& B, int64_t rb,
-                                          int lane) {
-    // the row's rings are contiguous coordinates: lanes take its edges
-    // (c - 1, c) across every ring at once, c not the start of a ring; a row
-    // of at most 32 (16) positions gives each edge 2 (4) lanes, which split
-    // the other row's edges by stride
-    const int32_t r0 = A.part[A.geom[ra]], r1 = A.part[A.geom[ra + 1]];
-    if (r1 <= r0) return false;
-    const int32_t e0 = A.ring[r0] + 1, e1 = A.ring[r1];
-    const int split = e1 - e0 <= 16 ? 4 : (e1 - e0 <= 32 ? 2 : 1);
-    const int sub = lane % split;
-    for (int32_t base = e0; base < e1; base += 64 / split) {
-        const int32_t c = base + lane / split;
-        bool hit = false;
-        bool edge = c < e1;
-        for (int32_t r = r0 + 1; edge && r < r1; ++r)
-            if (A.ring[r] == c) edge = false;
-        if (edge) {
-            const double ax = A.x[c - 1], ay = A.y[c - 1], bx = A.x[c], by = A.y[c];
-            for (int32_t q = B.part[B.geom[rb]]; q < B.part[B.geom[rb + 1]] && !hit; ++q)
-                for (int32_t d = B.ring[q] + 1 + sub; d < B.ring[q + 1]; d += split) {
-                    const double cx = B.x[d - 1], cy = B.y[d - 1], dx = B.x[d], dy = B.y[d];
-                    if (fmax(ax, bx) < fmin(cx, dx) || fmax(cx, dx) < fmin(ax, bx) ||
-                        fmax(ay, by) < fmin(cy, dy) || fmax(cy, dy) < fmin(ay, by))
-                        continue;
-                    if (mode == 0) {
-                        if (segments_touch(ax, ay, bx, by, cx, cy, dx, dy)) {
-                            hit = true;
-                            break;
+// One wave's LDS for wave_edge_pairs.
+constexpr int kEdgeTile = 128;
+struct WaveEdgeLds {
+    int32_t a[kEdgeTile];     // A edges near B (their end coordinate)
+    int32_t b[kEdgeTile];     // a tile of B edges near A's current edges
+    float4 box[kEdgeTile];    // their boxes (min x, min y, max x, max y)
+    int32_t qa[kEdgeTile], qb[kEdgeTile];  // edge pairs whose boxes meet
+};
+
+// Orders one wave's LDS accesses where its lanes exchange data through LDS.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Coordinates [lo, hi) of a row and its rings [r0, r1).
+struct RowSpan {
+    int32_t lo, hi, r0, r1;
+};
+
+__device__ __forceinline__ RowSpan row_span(const Polys& P, int64_t row) {
+    RowSpan s;
+    s.r0 = P.part[P.geom[row]];
+    s.r1 = P.part[P.geom[row + 1]];
+    s.lo = P.ring[s.r0];
+    s.hi = P.ring[s.r1];
+    return s;
+}
+
+// (c - 1, c) is an edge of the row: c lies in it and starts none of its rings.
+__device__ __forceinline__ bool is_row_edge(const Polys& P, const RowSpan& s, int32_t c) {
+    if (c <= s.lo || c >= s.hi) return false;
+    if (s.r1 - s.r0 <= 8) {
+        bool start = false;
+        for (int32_t r = s.r0 + 1; r < s.r1; ++r) start |= P.ring[r] == c;
+        return !start;
+    }
+    int32_t lo = s.r0 + 1, hi = s.r1;
+    while (lo < hi) {
+        const int32_t m = (lo + hi) >> 1;
+        if (P.ring[m] < c) lo = m + 1;
+        else hi = m;
+    }
+    return lo >= s.r1 || P.ring[lo] != c;
+}
+
+// Boxes in fp32, every bound rounded to nearest.  Rounding is monotone, so
+// boxes that meet in fp64 meet in fp32: the tests on them only drop pairs that
+// cannot touch, and the exact tests see every other pair.
+__device__ __forceinline__ float4 edge_box_f32(const Polys& P, int32_t c) {
+    const float ax = (float)P.x[c - 1], ay = (float)P.y[c - 1], bx = (float)P.x[c], by = (float)P.y[c];
+    return make_float4(fminf(ax, bx), fminf(ay, by), fmaxf(ax, bx), fmaxf(ay, by));
+}
+
+__device__ __forceinline__ bool boxes_meet(const float4& a, const float4& b) {
+    return !(a.z < b.x || b.z < a.x || a.w < b.y || b.w < a.y);
+}
+
+__device__ __forceinline__ float4 wave_union(float4 b) {
+    for (int o = 32; o > 0; o >>= 1) {
+        b.x = fminf(b.x, __shfl_xor(b.x, o, 64));
+        b.y = fminf(b.y, __shfl_xor(b.y, o, 64));
+        b.z = fmaxf(b.z, __shfl_xor(b.z, o, 64));
+        b.w = fmaxf(b.w, __shfl_xor(b.w, o, 64));
+    }
+    return b;
+}
+
+__device__ __forceinline__ float4 box_cut(const float4& a, const float4& b) {
+    return make_float4(fmaxf(a.x, b.x), fmaxf(a.y, b.y), fminf(a.z, b.z), fminf(a.w, b.w));
+}
+
+__device__ __forceinline__ float4 empty_box_f32() { return make_float4(INFINITY, INFINITY, -INFINITY, -INFINITY); }
+
+// Box of the coordinates [s.lo, s.hi), in fp32, by one wave.
+__device__ inline float4 wave_row_box_f32(const Polys& P, const RowSpan& s, int lane) {
+    float4 b = empty_box_f32();
+    for (int32_t c = s.lo + lane; c < s.hi; c += 64) {
+        const float x = (float)P.x[c], y = (float)P.y[c];
+        b = make_float4(fminf(b.x, x), fminf(b.y, y), fmaxf(b.z, x), fmaxf(b.w, y));
+    }
+    return wave_union(b);
+}
+
+// How two segments meet: 0 not at all, 1 they touch (segments_touch), 2 they
+// cross in interior points of both.
+VS_HD int segment_contact(double ax, double ay, double bx, double by, double cx, double cy, double dx, double dy) {
+    if (fmax(ax, bx) < fmin(cx, dx) || fmax(cx, dx) < fmin(ax, bx) || fmax(ay, by) < fmin(cy, dy) ||
+        fmax(cy, dy) < fmin(ay, by))
+        return 0;
+    const int o1 = orient2d(ax, ay, bx, by, cx, cy);
+    const int o2 = orient2d(ax, ay, bx, by, dx, dy);
+    const int o3 = orient2d(cx, cy, dx, dy, ax, ay);
+    const int o4 = orient2d(cx, cy, dx, dy, bx, by);
+    if (o1 * o2 < 0 && o3 * o4 < 0) return 2;
+    if (o1 == 0 && cx >= fmin(ax, bx) && cx <= fmax(ax, bx) && cy >= fmin(ay, by) && cy <= fmax(ay, by)) return 1;
+    if (o2 == 0 && dx >= fmin(ax, bx) && dx <= fmax(ax, bx) && dy >= fmin(ay, by) && dy <= fmax(ay, by)) return 1;
+    if (o3 == 0 && ax >= fmin(cx, dx) && ax <= fmax(cx, dx) && ay >= fmin(cy, dy) && ay <= fmax(cy, dy)) return 1;
+    if (o4 == 0 && bx >= fmin(cx, dx) && bx <= fmax(cx, dx) && by >= fmin(cy, dy) && by <= fmax(cy, dy)) return 1;
+    return 0;
+}
+
+// The closest contact over the edge pairs of two rows, by one wave (every lane
+// returns it): 2 some pair crosses, 1 some pair touches and none crosses, 0
+// neither; returns at the first contact of at least `enough`.  ba / bb: the
+// rows' fp32 boxes.
+//
+// Only edges that meet both rows' boxes can touch, and of those few meet each
+// other, so: A's edges near B's box are listed and taken 64 at a time, one per
+// lane (fewer: each edge gets several lanes, which share B's edges); B's edges
+// near them are collected in LDS tiles as fp32 boxes; box pairs that meet are
+// queued, and a full queue gets the exact test with all lanes at work.  Bound
+// by instruction issue: testing every edge pair of the rows in fp64, with a
+// wave waiting for any lane's exact test, took 11.1 ms for 600k pairs of
+// 57 x 57 coordinates; this takes 2.0 ms (about 860 vector instructions a pair),
+// and rows without contact need no full relation (2.9 ms for the 3% that did).
+__device__ inline int wave_edge_pairs(const Polys& A, const RowSpan& sa, const float4& ba, const Polys& B,
+                                      const RowSpan& sb, const float4& bb, int enough, WaveEdgeLds& W, int lane) {
+    const float4 both = box_cut(ba, bb);
+    const uint64_t lt = lanemask_lt();
+    int found = 0, nq = 0;
+    // exact tests of the first `n` (at most 64) queued pairs
+    auto test_queue = [&](int n) {
+        wave_lds_fence();
+        int k = 0;
+        if (lane < n) {
+            const int32_t c = W.qa[lane], d = W.qb[lane];
+            k = segment_contact(A.x[c - 1], A.y[c - 1], A.x[c], A.y[c], B.x[d - 1], B.y[d - 1], B.x[d], B.y[d]);
+        }
+        if (__ballot(k == 2)) found = 2;
+        else if (found < 1 && __ballot(k == 1)) found = 1;
+    };
+    int na = 0;
+    for (int32_t a0 = sa.lo + 1; a0 < sa.hi; a0 += 64) {
+        {
+            const int32_t c = a0 + lane;
+            const bool near = is_row_edge(A, sa, c) && boxes_meet(edge_box_f32(A, c), both);
+            const uint64_t m = __ballot(near);
+            if (near) W.a[na + __popcll(m & lt)] = c;
+            na += __popcll(m);
+        }
+        const bool last = a0 + 64 >= sa.hi;
+        while (na >= 64 || (last && na > 0)) {
+            wave_lds_fence();
+            const int n = na < 64 ? na : 64;
+            int width = 1;  // lanes per pass over A's edges; 64 / width share each B tile
+            while (width < n) width <<= 1;
+            const int ai = lane & (width - 1), sub = lane / width, subs = 64 / width;
+            const bool has = ai < n;
+            const int32_t ca = W.a[has ? ai : 0];
+            const float4 abox = edge_box_f32(A, ca);
+            // several passes over A: each one's edges are consecutive along
+            // the rings, so B is filtered by their own box
+            const float4 lim = na == n && last && a0 == sa.lo + 1 ? both : box_cut(wave_union(abox), bb);
+            int nb = 0;
+            for (int32_t b0 = sb.lo + 1; b0 < sb.hi; b0 += 64) {
+                const int32_t d = b0 + lane;
+                float4 dbox = empty_box_f32();
+                bool near = is_row_edge(B, sb, d);
+                if (near) {
+                    dbox = edge_box_f32(B, d);
+                    near = boxes_meet(dbox, lim);
+                }
+                const uint64_t m = __ballot(near);
+                if (near) {
+                    const int slot = nb + __popcll(m & lt);
+                    W.b[slot] = d;
+                    W.box[slot] = dbox;
+                }
+                nb += __popcll(m);
+                if (nb <= 64 && b0 + 64 < sb.hi) continue;  // room for another 64
+                wave_lds_fence();
+                for (int k0 = 0; k0 < nb; k0 += subs) {
+                    const int k = k0 + sub;
+                    const bool hit = has && k < nb && boxes_meet(abox, W.box[k < nb ? k : 0]);
+                    const uint64_t h = __ballot(hit);
+                    if (!h) continue;
+                    if (hit) {
+                        const int slot = nq + __popcll(h & lt);
+                        W.qa[slot] = ca;
+                        W.qb[slot] = W.b[k];
+                    }
+                    nq += __popcll(h);
+                    if (nq >= 64) {
+                        test_queue(64);
+                        if (found >= enough) return found;
+                        nq -= 64;
+                        int32_t ma = 0, mb = 0;
+                        if (lane < nq) {
+                            ma = W.qa[64 + lane];
+                            mb = W.qb[64 + lane];
                         }
-                    } else if (orient2d(ax, ay, bx, by, cx, cy) * orient2d(ax, ay, bx, by, dx, dy) < 0 &&
-                               orient2d(cx, cy, dx, dy, ax, ay) * orient2d(cx, cy, dx, dy, bx, by) < 0) {
-                        hit = true;
-                        break;
+                        wave_lds_fence();
+                        if (lane < nq) {
+                            W.qa[lane] = ma;
+                            W.qb[lane] = mb;
+                        }
+                        wave_lds_fence();
                     }
                 }
+                wave_lds_fence();
+                nb = 0;
+            }
+            na -= n;
+            const int32_t rest = lane < na ? W.a[64 + lane] : 0;
+            wave_lds_fence();
+            if (lane < na) W.a[lane] = rest;
+            wave_lds_fence();
         }
-        if (__ballot(hit) != 0) return true;
+    }
+    if (nq > 0) test_queue(nq);
+    return found;
+}
+
+// The point lies inside row s of P or on its boundary, by one wave.
+__device__ inline bool wave_not_outside(double px, double py, const Polys& P, int64_t row, const RowSpan& s,
+                                        int lane) {
+    for (int32_t pp = P.geom[row]; pp < P.geom[row + 1]; ++pp) {
+        const RowSpan t = {P.ring[P.part[pp]], P.ring[P.part[pp + 1]], P.part[pp], P.part[pp + 1]};
+        int parity = 0;
+        bool on = false;
+        for (int32_t c0 = t.lo + 1; c0 < t.hi; c0 += 64) {
+            const int32_t c = c0 + lane;
+            if (is_row_edge(P, t, c)) on |= edge_step_f64(px, py, P.x[c - 1], P.y[c - 1], P.x[c], P.y[c], parity) != 0;
+        }
+        if (__ballot(on) != 0 || (__popcll(__ballot(parity)) & 1)) return true;
     }
     return false;
 }
 
-// Exact intersects (the rule of polygons_intersect) by one wave.
-__device__ inline bool wave_intersects(const Polys& A, int64_t ra, const Polys& B, int64_t rb, int lane) {
-    if (row_coords(A, ra) == 0 || row_coords(B, rb) == 0) return false;
-    if (wave_any_edge_pair(0, A, ra, B, rb, lane)) return true;
-    bool in = false;
-    for (int32_t r = A.part[A.geom[ra]] + lane; r < A.part[A.geom[ra + 1]]; r += 64) {
-        const int32_t c0 = A.ring[r];
-        if (A.ring[r + 1] > c0 && point_location_f64(A.x[c0], A.y[c0], B.x, B.y, B.geom, B.part, B.ring, rb) != 0)
-            in = true;
+// Some ring of row ra of A starts at a point of row rb of B (not outside).
+__device__ inline bool wave_rings_start_in(const Polys& A, const RowSpan& sa, const Polys& B, int64_t rb,
+                                           const RowSpan& sb, const float4& bb, int lane) {
+    for (int32_t r = sa.r0; r < sa.r1; ++r) {
+        const int32_t c = A.ring[r];
+        if (A.ring[r + 1] <= c) continue;
+        const double x = A.x[c], y = A.y[c];
+        const float fx = (float)x, fy = (float)y;
+        if (fx < bb.x || fx > bb.z || fy < bb.y || fy > bb.w) continue;  // outside B's box
+        if (wave_not_outside(x, y, B, rb, sb, lane)) return true;
     }
-    for (int32_t r = B.part[B.geom[rb]] + lane; r < B.part[B.geom[rb + 1]]; r += 64) {
-        const int32_t c0 = B.ring[r];
-        if (B.ring[r + 1] > c0 && point_location_f64(B.x[c0], B.y[c0], A.x, A.y, A.geom, A.part, A.ring, ra) != 0)
-            in = true;
-    }
-    return __ballot(in) != 0;
+    return false;
 }
 
 __device__ inline double4 wave_row_box(const Polys& P, int64_t row, int lane) {
@@ -491,34 +679,68 @@ __device__ inline RelSide wave_relate_side(const Polys& X, int64_t rx, const Pol
 
 __device__ inline Relation wave_relate_polygons(const Polys& A, int64_t ra, const Polys& B, int64_t rb, int lane) {
     const RelSide sa = wave_relate_side(A, ra, B, rb, true, lane);
-    const RelSide sb = wave_relate_side(B, rb, A, ra, false, lane);
-    Relation R;
-    const bool cross = sa.cross || sb.cross;
-    R.interiors_meet = cross || sa.in_int || sb.in_int || sa.same || sb.same;
-    R.a_in_b = !cross && !sa.in_ext && !sb.in_int && sa.all_in;
-    R.b_in_a = !cross && !sb.in_ext && !sa.in_int && sb.all_in;
-    R.touch = sa.touch;
-    return R;
+    return merge_sides(sa, wave_relate_side(B, rb, A, ra, false, lane));
 }
 
-// polygon_predicate_fast by one wave (every lane returns the answer).
+// One side of the relation of two rows whose boundaries do not meet: every
+// ring of A then lies in one piece inside or outside B, where its first vertex
+// does.  A ring without two distinct points has no piece.
+__device__ inline RelSide wave_apart_side(const Polys& A, int64_t ra, const Polys& B, int64_t rb, const RowSpan& sb,
+                                          const float4& bb, int lane) {
+    RelSide S = {false, false, false, false, false, true};
+    for (int32_t pp = A.geom[ra]; pp < A.geom[ra + 1]; ++pp) {
+        bool part_in = false;
+        for (int32_t r = A.part[pp]; r < A.part[pp + 1]; ++r) {
+            const int32_t c0 = A.ring[r], c1 = A.ring[r + 1];
+            if (c1 <= c0) continue;
+            const double x = A.x[c0], y = A.y[c0];
+            bool piece = false;
+            for (int32_t c = c0 + 1; c < c1 && !piece; c += 64)
+                piece = __ballot(c + lane < c1 && (A.x[c + lane] != x || A.y[c + lane] != y)) != 0;
+            if (!piece) continue;
+            const float fx = (float)x, fy = (float)y;
+            const bool in = !(fx < bb.x || fx > bb.z || fy < bb.y || fy > bb.w) &&
+                            wave_not_outside(x, y, B, rb, sb, lane);
+            S.in_int |= in;
+            S.in_ext |= !in;
+            part_in |= in;
+        }
+        S.all_in &= part_in;
+    }
+    return S;
+}
+
+// polygon_predicate_fast by one wave (every lane returns the answer); rows
+// whose boundaries do not meet are decided for good.
 __device__ inline int wave_polygon_predicate_fast(int pred, const Polys& A, int64_t ra, const Polys& B, int64_t rb,
-                                                  int lane) {
-    if (pred == VS_PRED_INTERSECTS) return wave_intersects(A, ra, B, rb, lane) ? 1 : 0;
+                                                  WaveEdgeLds& W, int lane) {
     if (pred == VS_PRED_CROSSES) return 0;
-    if (pred == VS_PRED_WITHIN || pred == VS_PRED_COVERED_BY || pred == VS_PRED_CONTAINS ||
-        pred == VS_PRED_COVERS || pred == VS_PRED_CONTAINS_PROPERLY) {
+    const RowSpan sa = row_span(A, ra), sb = row_span(B, rb);
+    const bool inclusion = pred == VS_PRED_WITHIN || pred == VS_PRED_COVERED_BY || pred == VS_PRED_CONTAINS ||
+                           pred == VS_PRED_COVERS || pred == VS_PRED_CONTAINS_PROPERLY;
+    if (inclusion) {
         const bool a_inner = pred == VS_PRED_WITHIN || pred == VS_PRED_COVERED_BY;
         const double4 in = a_inner ? wave_row_box(A, ra, lane) : wave_row_box(B, rb, lane);
         const double4 out = a_inner ? wave_row_box(B, rb, lane) : wave_row_box(A, ra, lane);
         if (!(out.x <= in.x && in.z <= out.z && out.y <= in.y && in.w <= out.w)) return 0;
-        if (wave_any_edge_pair(1, A, ra, B, rb, lane)) return 0;
-        return -1;
+    } else if (sa.hi <= sa.lo || sb.hi <= sb.lo) {
+        return 0;  // an empty row meets nothing
     }
-    // touches, overlaps
-    if (!wave_intersects(A, ra, B, rb, lane)) return 0;
-    if (wave_any_edge_pair(1, A, ra, B, rb, lane)) return pred == VS_PRED_OVERLAPS ? 1 : 0;
-    return -1;
+    const float4 ba = wave_row_box_f32(A, sa, lane), bb = wave_row_box_f32(B, sb, lane);
+    // the smaller row's edges go to the lanes
+    const int enough = pred == VS_PRED_INTERSECTS ? 1 : 2;
+    const int contact = sa.hi - sa.lo <= sb.hi - sb.lo ? wave_edge_pairs(A, sa, ba, B, sb, bb, enough, W, lane)
+                                                       : wave_edge_pairs(B, sb, bb, A, sa, ba, enough, W, lane);
+    if (contact == 2) return inclusion || pred == VS_PRED_TOUCHES ? 0 : 1;
+    if (!inclusion) {
+        // without contact the rows meet only if a ring of one starts in the other
+        const bool meet = contact == 1 || wave_rings_start_in(A, sa, B, rb, sb, bb, lane) ||
+                          wave_rings_start_in(B, sb, A, ra, sa, ba, lane);
+        if (!meet || pred == VS_PRED_INTERSECTS) return meet ? 1 : 0;
+    }
+    if (contact == 1) return -1;
+    const RelSide ea = wave_apart_side(A, ra, B, rb, sb, bb, lane), eb = wave_apart_side(B, rb, A, ra, sa, ba, lane);
+    return relation_decides(pred, merge_sides(ea, eb)) ? 1 : 0;
 }
 
 }  // namespace vs

@@ -9,8 +9,10 @@
 //   scan   tile = 256 threads x 16 items; reduce -> single-block scan of tile
 //          sums (int64) -> downsweep.  No decoupled look-back, so no inter-block
 //          spin waits.
-//   sort   8-bit digits, three launches per pass: LDS histogram per tile,
-//          device scan of the digit-major histogram, stable scatter.  The
+//   sort   8-bit digits; at most 4,096 pairs: one block, every pass in LDS;
+//          else per pass an LDS histogram per tile, a device scan of the
+//          digit-major histogram (few tiles: the scatter sums the histograms
+//          itself), a stable scatter.  The
 //          scatter ranks keys inside each wave with 8 ballots per item (peer
 //          mask of equal digits), combines waves through LDS counters, writes the
 //          tile into LDS in digit order and then streams it out so each digit
@@ -231,7 +233,7 @@ template <class K>
 __global__ __launch_bounds__(kRsThreads) void rs_hist_kernel(const K* __restrict__ keys, int64_t n,
                                                             const unsigned long long* __restrict__ d_n,
                                                             int shift, int dmask, int32_t* __restrict__ hist,
-                                                            int nblocks) {
+                                                            int nblocks, bool by_block) {
     n = device_count(n, d_n);
     __shared__ int cnt[kRsWaves][kRsBins];
     const int w = threadIdx.x >> 6;
@@ -267,16 +269,18 @@ __global__ __launch_bounds__(kRsThreads) void rs_hist_kernel(const K* __restrict
     int t = 0;
 #pragma unroll
     for (int k = 0; k < kRsWaves; ++k) t += cnt[k][d];
-    hist[(int64_t)d * nblocks + blockIdx.x] = t;
+    hist[by_block ? (int64_t)blockIdx.x * kRsBins + d : (int64_t)d * nblocks + blockIdx.x] = t;
 }
 
 // WIDE: the pass writes its keys and values as int64 (a sort's last pass
 // writing a join's output pairs directly).
+// by_block: `hist_scan` holds the histograms themselves, [block][digit], and
+// each block forms its own digit offsets from them (at most kRsFusedBlocks).
 template <class K, bool WIDE>
 __global__ __launch_bounds__(kRsThreads) void rs_scatter_kernel(
     const K* __restrict__ keys_in, const int32_t* __restrict__ vals_in, void* __restrict__ keys_out,
     void* __restrict__ vals_out, int64_t n, const unsigned long long* __restrict__ d_n, int shift,
-    int dmask, const int32_t* __restrict__ hist_scan, int nblocks) {
+    int dmask, const int32_t* __restrict__ hist_scan, int nblocks, bool by_block) {
     n = device_count(n, d_n);
     if ((int64_t)blockIdx.x * kRsTile >= n) return;  // whole tile past the valid count (block-uniform)
     __shared__ int wave_cnt[kRsWaves][kRsBins];
@@ -288,7 +292,19 @@ __global__ __launch_bounds__(kRsThreads) void rs_scatter_kernel(
 
     const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
     for (int i = tid; i < kRsWaves * kRsBins; i += kRsThreads) (&wave_cnt[0][0])[i] = 0;
-    digit_global[tid] = hist_scan[(int64_t)tid * nblocks + blockIdx.x];
+    if (by_block) {
+        int before = 0, total = 0;  // of this thread's digit: in the blocks before this one, in all
+#pragma unroll 8
+        for (int b = 0; b < nblocks; ++b) {
+            const int c = hist_scan[b * kRsBins + tid];
+            before += b < (int)blockIdx.x ? c : 0;
+            total += c;
+        }
+        long long all;
+        digit_global[tid] = block_exclusive_scan_i64(total, lds4, all) + before;
+    } else {
+        digit_global[tid] = hist_scan[(int64_t)tid * nblocks + blockIdx.x];
+    }
     __syncthreads();
 
     const int64_t base = (int64_t)blockIdx.x * kRsTile + (int64_t)w * (64 * kRsItems);
@@ -369,6 +385,149 @@ __global__ __launch_bounds__(kRsThreads) void rs_scatter_kernel(
     }
 }
 
+// The whole sort of at most kRsSmall pairs by one block: the pairs stay in LDS
+// between the passes.  A sort of a thousand pairs took four launches a pass,
+// 4-5 us each (24 of the 51 launches of a 1,003-point join); this is one of 6 us.
+constexpr int kRsSmallThreads = 1024;
+constexpr int kRsSmallItems = 4;
+constexpr int kRsSmall = kRsSmallThreads * kRsSmallItems;
+
+template <class K, bool WIDE>
+__global__ __launch_bounds__(kRsSmallThreads) void rs_small_kernel(const K* keys_in, const int32_t* vals_in,
+                                                                  void* keys_out, void* vals_out, int64_t n64,
+                                                                  const unsigned long long* __restrict__ d_n,
+                                                                  int begin_bit, int end_bit) {
+    constexpr int kWaves = kRsSmallThreads / 64;
+    __shared__ K skeys[kRsSmall];
+    __shared__ int32_t svals[kRsSmall];
+    __shared__ int cnt[kWaves][kRsBins];
+    __shared__ int digit_off[kRsBins];
+    __shared__ int part[kRsBins / 64];
+    const int n = (int)device_count(n64, d_n);
+    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+    const int items = (n + kRsSmallThreads - 1) / kRsSmallThreads;  // per thread; a wave's pairs are contiguous
+    const int base = w * 64 * items;
+    const uint64_t lt = lanemask_lt();
+    K k[kRsSmallItems];
+    int32_t v[kRsSmallItems];
+    int rank[kRsSmallItems];
+#pragma unroll
+    for (int i = 0; i < kRsSmallItems; ++i) {
+        const int idx = base + i * 64 + lane;
+        const bool valid = i < items && idx < n;
+        k[i] = valid ? keys_in[idx] : (K)0;
+        v[i] = valid ? (vals_in ? vals_in[idx] : idx) : 0;
+    }
+    for (int shift = begin_bit; shift < end_bit; shift += 8) {
+        const int dmask = (1 << (end_bit - shift < 8 ? end_bit - shift : 8)) - 1;
+        for (int i = tid; i < kWaves * kRsBins; i += kRsSmallThreads) (&cnt[0][0])[i] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kRsSmallItems; ++i) {
+            if (i >= items) break;
+            const bool valid = base + i * 64 + lane < n;
+            const int d = (int)((k[i] >> shift) & dmask);
+            uint64_t m = __ballot(valid);
+#pragma unroll
+            for (int b = 0; b < 8; ++b) {
+                const bool bit = (d >> b) & 1;
+                const uint64_t bb = __ballot(bit);
+                m &= bit ? bb : ~bb;
+            }
+            int cur = 0;
+            if (valid) cur = cnt[w][d];
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            rank[i] = cur + __popcll(m & lt);
+            if (valid && (m & lt) == 0) cnt[w][d] = cur + __popcll(m);
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+        __syncthreads();
+        int s = 0, inc = 0;
+        if (tid < kRsBins) {  // per digit: exclusive over waves, then over digits
+#pragma unroll
+            for (int ww = 0; ww < kWaves; ++ww) {
+                const int c = cnt[ww][tid];
+                cnt[ww][tid] = s;
+                s += c;
+            }
+            inc = wave_inclusive_scan(s);
+            if (lane == 63) part[w] = inc;
+        }
+        __syncthreads();
+        if (tid < kRsBins) {
+            int off = inc - s;
+            for (int ww = 0; ww < w; ++ww) off += part[ww];
+            digit_off[tid] = off;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kRsSmallItems; ++i) {
+            if (i >= items) break;
+            if (base + i * 64 + lane < n) {
+                const int d = (int)((k[i] >> shift) & dmask);
+                const int pos = digit_off[d] + cnt[w][d] + rank[i];
+                skeys[pos] = k[i];
+                svals[pos] = v[i];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kRsSmallItems; ++i) {
+            if (i >= items) break;
+            const int idx = base + i * 64 + lane;
+            if (idx < n) {
+                k[i] = skeys[idx];
+                v[i] = svals[idx];
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < kRsSmallItems; ++i) {
+        if (i >= items) break;
+        const int idx = base + i * 64 + lane;
+        if (idx < n) {
+            if (WIDE) {
+                static_cast<int64_t*>(keys_out)[idx] = (int64_t)k[i];
+                static_cast<int64_t*>(vals_out)[idx] = (int64_t)v[i];
+            } else {
+                static_cast<K*>(keys_out)[idx] = k[i];
+                static_cast<int32_t*>(vals_out)[idx] = v[i];
+            }
+        }
+    }
+}
+
+template <class K, bool WIDE>
+int rs_small(const K* ki, const int32_t* vi, void* ko, void* vo, int64_t n, const unsigned long long* d_n,
+             int begin_bit, int end_bit, hipStream_t s) {
+    hipLaunchKernelGGL((rs_small_kernel<K, WIDE>), dim3(1), dim3(kRsSmallThreads), 0, s, ki, vi, ko, vo, n, d_n,
+                       begin_bit, end_bit);
+    VS_LAUNCH_CHECK();
+    return VS_OK;
+}
+
+// Blocks up to which a pass is two launches: each scatter block reads every
+// block's histogram (1 KB each, from L2) instead of waiting for two scan
+// launches of 4-5 us.
+constexpr int kRsFusedBlocks = 128;
+
+// One radix pass: digit (key >> shift) & dmask, stable.
+template <class K, bool WIDE>
+int rs_pass(const K* ki, const int32_t* vi, void* ko, void* vo, int64_t n, const unsigned long long* d_n, int shift,
+            int dmask, int32_t* hist, void* scan_ws, int nb, hipStream_t s) {
+    const bool fused = nb <= kRsFusedBlocks;
+    hipLaunchKernelGGL(rs_hist_kernel<K>, dim3(nb), dim3(kRsThreads), 0, s, ki, n, d_n, shift, dmask, hist, nb,
+                       fused);
+    VS_LAUNCH_CHECK();
+    if (!fused) VS_TRY(exclusive_scan_i32(hist, hist, (int64_t)nb * kRsBins, nullptr, scan_ws, s));
+    hipLaunchKernelGGL((rs_scatter_kernel<K, WIDE>), dim3(nb), dim3(kRsThreads), 0, s, ki, vi, ko, vo, n, d_n, shift,
+                       dmask, hist, nb, fused);
+    VS_LAUNCH_CHECK();
+    return VS_OK;
+}
+
 template <class K>
 int64_t sort_workspace_bytes_t(int64_t n) {
     const int64_t nb = ceil_div(n > 0 ? n : 1, kRsTile);
@@ -407,27 +566,20 @@ int sort_pairs_nocopy(K* keys, int32_t* vals, int64_t n, const unsigned long lon
     K* ko = kalt;
     int32_t* vo = valt;
     const bool wide = wide_l != nullptr && n > 1 && begin_bit < end_bit;
-    if (n > 1) {
+    if (n > 1 && n <= kRsSmall && begin_bit < end_bit) {
+        if (wide) VS_TRY((rs_small<K, true>(ki, vi, wide_l, wide_r, n, d_n, begin_bit, end_bit, s)));
+        else VS_TRY((rs_small<K, false>(ki, vi, ki, vi, n, d_n, begin_bit, end_bit, s)));
+        if (wide) ki = nullptr;
+    } else if (n > 1) {
         for (int shift = begin_bit; shift < end_bit; shift += 8) {
             const int width = end_bit - shift < 8 ? end_bit - shift : 8;
             const int dmask = (1 << width) - 1;
-            hipLaunchKernelGGL(rs_hist_kernel<K>, dim3(nb), dim3(kRsThreads), 0, s, ki, n, d_n, shift, dmask, hist,
-                               nb);
-            VS_LAUNCH_CHECK();
-            VS_TRY(exclusive_scan_i32(hist, hist, (int64_t)nb * kRsBins, nullptr, scan_ws, s));
             if (wide && shift + 8 >= end_bit) {
-                hipLaunchKernelGGL((rs_scatter_kernel<K, true>), dim3(nb), dim3(kRsThreads), 0, s, ki, vi, wide_l,
-                                   wide_r, n, d_n, shift, dmask, hist, nb);
-                VS_LAUNCH_CHECK();
-                res->keys = nullptr;
-                res->vals = vi;  // read by this pass, free once it ran
-                res->alt_keys = ko;
-                res->alt_vals = vo;
-                return VS_OK;
+                VS_TRY((rs_pass<K, true>(ki, vi, wide_l, wide_r, n, d_n, shift, dmask, hist, scan_ws, nb, s)));
+                ki = nullptr;  // vals: read by this pass, free once it ran
+                break;
             }
-            hipLaunchKernelGGL((rs_scatter_kernel<K, false>), dim3(nb), dim3(kRsThreads), 0, s, ki, vi, ko, vo, n,
-                               d_n, shift, dmask, hist, nb);
-            VS_LAUNCH_CHECK();
+            VS_TRY((rs_pass<K, false>(ki, vi, ko, vo, n, d_n, shift, dmask, hist, scan_ws, nb, s)));
             K* tk = ki; ki = ko; ko = tk;
             int32_t* tv = vi; vi = vo; vo = tv;
         }
@@ -461,18 +613,11 @@ int sort_lex_wide_u32(uint32_t* l, int32_t* r, int64_t n, const unsigned long lo
             const int dmask = (1 << (bits - shift < 8 ? bits - shift : 8)) - 1;
             const uint32_t* key = side == 0 ? ri : li;
             const int32_t* val = reinterpret_cast<const int32_t*>(side == 0 ? li : ri);
-            hipLaunchKernelGGL(rs_hist_kernel<uint32_t>, dim3(nb), dim3(kRsThreads), 0, s, key, n, d_n, shift, dmask,
-                               hist, nb);
-            VS_LAUNCH_CHECK();
-            VS_TRY(exclusive_scan_i32(hist, hist, (int64_t)nb * kRsBins, nullptr, scan_ws, s));
-            if (side == 1 && shift + 8 >= bits) {
-                hipLaunchKernelGGL((rs_scatter_kernel<uint32_t, true>), dim3(nb), dim3(kRsThreads), 0, s, key, val,
-                                   out_l, out_r, n, d_n, shift, dmask, hist, nb);
-            } else {
-                hipLaunchKernelGGL((rs_scatter_kernel<uint32_t, false>), dim3(nb), dim3(kRsThreads), 0, s, key, val,
-                                   side == 0 ? ro : lo, side == 0 ? lo : ro, n, d_n, shift, dmask, hist, nb);
-            }
-            VS_LAUNCH_CHECK();
+            if (side == 1 && shift + 8 >= bits)
+                VS_TRY((rs_pass<uint32_t, true>(key, val, out_l, out_r, n, d_n, shift, dmask, hist, scan_ws, nb, s)));
+            else
+                VS_TRY((rs_pass<uint32_t, false>(key, val, side == 0 ? ro : lo, side == 0 ? lo : ro, n, d_n, shift,
+                                                 dmask, hist, scan_ws, nb, s)));
             std::swap(li, lo);
             std::swap(ri, ro);
         }
@@ -514,6 +659,8 @@ int sort_pairs_into(const K* in_keys, const int32_t* in_vals, K* out_keys, int32
         }
         return VS_OK;
     }
+    if (n <= kRsSmall)
+        return rs_small<K, false>(in_keys, in_vals, out_keys, out_vals, n, d_n, begin_bit, end_bit, s);
     const int nb = (int)ceil_div(n, kRsTile);
     Carver c(ws);
     K* kalt = c.take<K>(n);
@@ -527,12 +674,7 @@ int sort_pairs_into(const K* in_keys, const int32_t* in_vals, K* out_keys, int32
     for (int shift = begin_bit; shift < end_bit; shift += 8) {
         const int width = end_bit - shift < 8 ? end_bit - shift : 8;
         const int dmask = (1 << width) - 1;
-        hipLaunchKernelGGL(rs_hist_kernel<K>, dim3(nb), dim3(kRsThreads), 0, s, ki, n, d_n, shift, dmask, hist, nb);
-        VS_LAUNCH_CHECK();
-        VS_TRY(exclusive_scan_i32(hist, hist, (int64_t)nb * kRsBins, nullptr, scan_ws, s));
-        hipLaunchKernelGGL((rs_scatter_kernel<K, false>), dim3(nb), dim3(kRsThreads), 0, s, ki, vi, ko, vo, n, d_n,
-                           shift, dmask, hist, nb);
-        VS_LAUNCH_CHECK();
+        VS_TRY((rs_pass<K, false>(ki, vi, ko, vo, n, d_n, shift, dmask, hist, scan_ws, nb, s)));
         ki = ko;
         vi = vo;
         ko = ko == out_keys ? kalt : out_keys;

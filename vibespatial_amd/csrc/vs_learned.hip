@@ -113,54 +113,89 @@ __device__ __forceinline__ float mlp_eval(const float* P, float u) {
 
 // Gradient of the mean squared rank error, computed by one block in two
 // phases so that no thread holds all 97 partial derivatives:
-//   phase 1  thread-strided over samples: residual r_j = y_j - t_j into LDS,
-//            partial loss and output-bias gradient;
-//   phase 2  thread t owns hidden unit h = t mod 32 for the samples
-//            j = t div 32 (mod blocks/32): with z = w1_h u_j + b1_h > 0,
-//            dy = 2 r_j scale:  dL/dw2_h += dy z,  dL/dw1_h += dy w2_h u_j,
-//            dL/db1_h += dy w2_h.
+//   phase 1  kTrainSamples samples per thread: dy_j = 2 (y_j - t_j) scale
+//            into LDS, partial loss and output-bias gradient; the parameters
+//            sit in the lanes (unit h in lanes h and h + 32) and reach the
+//            others by readlane;
+//   phase 2  thread t owns hidden unit h = t mod 32 and the samples of group
+//            t div 32: with z = w1_h u_j + b1_h > 0,
+//            dL/dw2_h += dy z,  dL/dw1_h += dy w2_h u_j,  dL/db1_h += dy w2_h,
+//            four partial sums per derivative (samples 4 i + 0..3).
 // Parameters: P[h] = w1, P[32 + h] = b1, P[64 + h] = w2, P[96] = b2.
-constexpr int kTrainThreads = 1024;
+// Bound by the issue rate of one compute unit (the whole training is one
+// block, its steps a serial chain).  512 threads, two waves per SIMD: 3.6 us a
+// step, 256: 5.0, 1,024: 4.0; reading every parameter from LDS per sample took
+// 6.2 (256 steps at 10M points: 1,611 -> 930 us; 16 steps of a join: 106 -> 65).
+constexpr int kTrainThreads = 512;
 // Adam step (relative to each parameter's scale) of the join's index build:
 // larger steps leave the quantile-knot start best for the first tens of steps.
 constexpr float kJoinTrainLr = 3.0e-4f;
 constexpr int kTrainWaves = kTrainThreads / 64;
+constexpr int kTrainGroups = kTrainThreads / kHidden;
+constexpr int kGroupSamples = kSample / kTrainGroups;
+constexpr int kTrainSamples = kSample / kTrainThreads;  // samples per thread in phase 1
+static_assert(kSample % kTrainThreads == 0 && kGroupSamples % 4 == 0, "whole samples per thread, whole float4 groups");
 
 struct GradPart {
     float gw1 = 0.0f, gb1 = 0.0f, gw2 = 0.0f, gb2 = 0.0f, loss = 0.0f;
 };
 
-// Accumulates the contribution of samples (su, st)[0, S) (LDS) into gp; sr is
-// LDS scratch of S floats.  Called by every thread of the block.
-__device__ void mlp_grad_accumulate(const float* P, const float* su, const float* st, float* sr, int S, float scale,
-                                    GradPart& gp) {
+// Accumulates the contribution of samples (su, st)[0, S) (LDS, kSample floats
+// each, any finite values from S on) into gp; sr is LDS scratch of kSample
+// floats.  Called by every thread of the block.
+__device__ __forceinline__ void mlp_grad_accumulate(const float* P, const float4* su, const float4* st, float4* sr,
+                                                    int S, float scale, GradPart& gp) {
     const int tid = threadIdx.x;
-    for (int j = tid; j < S; j += blockDim.x) {
-        const float r = mlp_eval(P, su[j]) - st[j];
-        sr[j] = r;
-        gp.loss += r * r;
-        gp.gb2 += 2.0f * r * scale;
-    }
-    __syncthreads();
-    const int h = tid & (kHidden - 1), grp = tid / kHidden, ngrp = blockDim.x / kHidden;
-    const float w1 = P[h], b1 = P[kHidden + h], w2 = P[2 * kHidden + h];
-    for (int j = grp; j < S; j += ngrp) {
-        const float u = su[j];
-        const float z = w1 * u + b1;
-        if (z > 0.0f) {
-            const float dy = 2.0f * sr[j] * scale;
-            gp.gw2 += dy * z;
-            const float dz = dy * w2;
-            gp.gw1 += dz * u;
-            gp.gb1 += dz;
+    const int h = tid & (kHidden - 1), grp = tid / kHidden;
+    const float w1 = P[h], b1 = P[kHidden + h], w2 = P[2 * kHidden + h], b2 = P[3 * kHidden];
+    {
+        const float* u1 = reinterpret_cast<const float*>(su) + tid;
+        const float* t1 = reinterpret_cast<const float*>(st) + tid;
+        float* r1 = reinterpret_cast<float*>(sr) + tid;
+        float y[kTrainSamples], uu[kTrainSamples];
+#pragma unroll
+        for (int j = 0; j < kTrainSamples; ++j) {
+            y[j] = b2;
+            uu[j] = u1[j * kTrainThreads];
+        }
+#pragma unroll
+        for (int k = 0; k < kHidden; ++k) {
+            const float a = readlane_f32(w1, k), b = readlane_f32(b1, k), c = readlane_f32(w2, k);
+#pragma unroll
+            for (int j = 0; j < kTrainSamples; ++j) y[j] = fmaf(c, fmaxf(fmaf(a, uu[j], b), 0.0f), y[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < kTrainSamples; ++j) {
+            const float r = tid + j * kTrainThreads < S ? y[j] - t1[j * kTrainThreads] : 0.0f;
+            const float dy = 2.0f * r * scale;
+            gp.loss += r * r;
+            gp.gb2 += dy;
+            r1[j * kTrainThreads] = dy;
         }
     }
     __syncthreads();
+    float g1[4] = {}, g2[4] = {}, gb[4] = {};
+#pragma unroll 4
+    for (int i = 0; i < kGroupSamples / 4; ++i) {
+        const float4 u = su[grp * (kGroupSamples / 4) + i], d = sr[grp * (kGroupSamples / 4) + i];
+        const float uu[4] = {u.x, u.y, u.z, u.w}, dd[4] = {d.x, d.y, d.z, d.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float z = fmaf(w1, uu[j], b1);
+            const float dy = z > 0.0f ? dd[j] : 0.0f;
+            g2[j] = fmaf(dy, z, g2[j]);
+            g1[j] = fmaf(dy, uu[j], g1[j]);
+            gb[j] += dy;
+        }
+    }
+    gp.gw2 += (g2[0] + g2[1]) + (g2[2] + g2[3]);
+    gp.gw1 += w2 * ((g1[0] + g1[1]) + (g1[2] + g1[3]));
+    gp.gb1 += w2 * ((gb[0] + gb[1]) + (gb[2] + gb[3]));
 }
 
-// Block reduction of the per-thread parts into out[0..kNParams] (gradient,
-// then the summed squared residual at out[kNParams]).
-__device__ void mlp_grad_reduce(const GradPart& gp, float (*red)[kNParams + 1], float* out) {
+// Wave sums of the per-thread parts into red[wave][0..kNParams] (gradient,
+// then the summed squared residual at [kNParams]); no barrier.
+__device__ __forceinline__ void mlp_grad_wave_sums(const GradPart& gp, float (*red)[kNParams + 1]) {
     const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
     float gw1 = gp.gw1, gb1 = gp.gb1, gw2 = gp.gw2, gb2 = gp.gb2, loss = gp.loss;
     // lanes l and l ^ 32 hold the same hidden unit (two sample groups per wave)
@@ -180,13 +215,13 @@ __device__ void mlp_grad_reduce(const GradPart& gp, float (*red)[kNParams + 1], 
         red[w][3 * kHidden] = gb2;
         red[w][kNParams] = loss;
     }
-    __syncthreads();
-    for (int k = tid; k <= kNParams; k += blockDim.x) {
-        float v = 0.0f;
-        for (int ww = 0; ww < (int)(blockDim.x >> 6); ++ww) v += red[ww][k];
-        out[k] = v;
-    }
-    __syncthreads();
+}
+
+__device__ __forceinline__ float mlp_grad_total(const float (*red)[kNParams + 1], int k) {
+    float v = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kTrainWaves; ++w) v += red[w][k];
+    return v;
 }
 
 // One block: sample, quantile-knot initialisation, `iters` full-batch Adam
@@ -196,18 +231,18 @@ __global__ __launch_bounds__(kTrainThreads) void mlp_train_kernel(const K* __res
                                                                  float lr, float* __restrict__ params_out,
                                                                  float* __restrict__ losses,
                                                                  int32_t* __restrict__ meta) {
-    __shared__ float su[kSample], st[kSample], sr[kSample];
-    __shared__ float P[kNParams], M1[kNParams], M2[kNParams], SC[kNParams], BEST[kNParams];
+    __shared__ float4 su4[kSample / 4], st4[kSample / 4], sr4[kSample / 4];
+    __shared__ float P[kNParams], SC[kNParams];
     __shared__ float red[kTrainWaves][kNParams + 1];
-    __shared__ float tot[kNParams + 1];
-    __shared__ float best_loss, init_loss;
+    float* su = reinterpret_cast<float*>(su4);
+    float* st = reinterpret_cast<float*>(st4);
     // one block beside the coordinate gather: raise its waves' issue priority
     __builtin_amdgcn_s_setprio(3);
     const int tid = threadIdx.x;
     if (meta && tid < 4) meta[tid] = 0;  // the leaf error pass that follows takes maxima there
     const int S = n >= kSample ? kSample : (int)n;
-    for (int j = tid; j < S; j += blockDim.x) {
-        const int64_t i = S > 1 ? (int64_t)((n - 1) * (double)j / (double)(S - 1)) : 0;
+    for (int j = tid; j < kSample; j += kTrainThreads) {
+        const int64_t i = S > 1 && j < S ? (int64_t)((n - 1) * (double)j / (double)(S - 1)) : 0;
         su[j] = key_unit<K>(keys[i]);
         st[j] = (float)((double)i / (double)n);
     }
@@ -234,44 +269,40 @@ __global__ __launch_bounds__(kTrainThreads) void mlp_train_kernel(const K* __res
         if (h == 0) {
             P[3 * kHidden] = st[0];
             SC[3 * kHidden] = 1.0f / kHidden;
-            best_loss = INFINITY;
         }
-    }
-    for (int k = tid; k < kNParams; k += blockDim.x) {
-        M1[k] = 0.0f;
-        M2[k] = 0.0f;
     }
     __syncthreads();
     const float scale = 1.0f / (float)(S > 0 ? S : 1);
     const float b1 = 0.9f, b2 = 0.999f;
     float b1t = 1.0f, b2t = 1.0f;
+    // thread k < kNParams keeps parameter k's Adam state and best value; the
+    // losses are the same in every thread
+    float m1 = 0.0f, m2 = 0.0f, best = 0.0f, init_loss = 0.0f, best_loss = INFINITY;
     for (int it = 0; it <= iters; ++it) {
         GradPart gp;
-        mlp_grad_accumulate(P, su, st, sr, S, scale, gp);
-        mlp_grad_reduce(gp, red, tot);
-        const float L = tot[kNParams] * scale;
-        const bool better = L < best_loss;  // uniform: every thread reads the same LDS values
-        if (tid < kNParams && better) BEST[tid] = P[tid];
+        mlp_grad_accumulate(P, su4, st4, sr4, S, scale, gp);
+        mlp_grad_wave_sums(gp, red);
         __syncthreads();
-        if (tid == 0) {
-            if (it == 0) init_loss = L;
-            if (better) best_loss = L;
-        }
-        if (it == iters) break;
+        const float L = mlp_grad_total(red, kNParams) * scale;
+        const bool better = L < best_loss;
+        if (it == 0) init_loss = L;
+        if (better) best_loss = L;
         b1t *= b1;
         b2t *= b2;
         if (tid < kNParams) {
-            const int k = tid;
-            const float gk = tot[k];
-            M1[k] = b1 * M1[k] + (1.0f - b1) * gk;
-            M2[k] = b2 * M2[k] + (1.0f - b2) * gk * gk;
-            const float mh = M1[k] / (1.0f - b1t), vh = M2[k] / (1.0f - b2t);
-            P[k] -= lr * SC[k] * mh / (sqrtf(vh) + 1.0e-12f);
+            const float p = P[tid];
+            if (better) best = p;
+            if (it < iters) {
+                const float gk = mlp_grad_total(red, tid);
+                m1 = b1 * m1 + (1.0f - b1) * gk;
+                m2 = b2 * m2 + (1.0f - b2) * gk * gk;
+                const float mh = m1 / (1.0f - b1t), vh = m2 / (1.0f - b2t);
+                P[tid] = p - lr * SC[tid] * mh / (sqrtf(vh) + 1.0e-12f);
+            }
         }
         __syncthreads();
     }
-    __syncthreads();
-    for (int k = tid; k < kNParams; k += blockDim.x) params_out[k] = BEST[k];
+    if (tid < kNParams) params_out[tid] = best;
     if (tid == 0) {
         losses[0] = init_loss;
         losses[1] = best_loss;
@@ -285,27 +316,26 @@ __global__ __launch_bounds__(kTrainThreads) void mlp_loss_grad_kernel(const floa
                                                                      const float* __restrict__ t, int64_t n,
                                                                      float* __restrict__ grad_out,
                                                                      float* __restrict__ loss_out) {
-    __shared__ float su[kSample], st[kSample], sr[kSample];
+    __shared__ float4 su4[kSample / 4], st4[kSample / 4], sr4[kSample / 4];
     __shared__ float P[kNParams];
     __shared__ float red[kTrainWaves][kNParams + 1];
-    __shared__ float tot[kNParams + 1];
-    for (int k = threadIdx.x; k < kNParams; k += blockDim.x) P[k] = params[k];
+    for (int k = threadIdx.x; k < kNParams; k += kTrainThreads) P[k] = params[k];
     const float scale = 1.0f / (float)(n > 0 ? n : 1);
     GradPart gp;
     for (int64_t c0 = 0; c0 < n; c0 += kSample) {
         const int S = (n - c0) < kSample ? (int)(n - c0) : kSample;
         __syncthreads();
-        for (int j = threadIdx.x; j < S; j += blockDim.x) {
-            su[j] = u[c0 + j];
-            st[j] = t[c0 + j];
+        for (int j = threadIdx.x; j < kSample; j += kTrainThreads) {
+            reinterpret_cast<float*>(su4)[j] = j < S ? u[c0 + j] : 0.0f;
+            reinterpret_cast<float*>(st4)[j] = j < S ? t[c0 + j] : 0.0f;
         }
         __syncthreads();
-        mlp_grad_accumulate(P, su, st, sr, S, scale, gp);
+        mlp_grad_accumulate(P, su4, st4, sr4, S, scale, gp);
     }
+    mlp_grad_wave_sums(gp, red);
     __syncthreads();
-    mlp_grad_reduce(gp, red, tot);
-    for (int k = threadIdx.x; k < kNParams; k += blockDim.x) grad_out[k] = tot[k];
-    if (threadIdx.x == 0) loss_out[0] = tot[kNParams] * scale;
+    for (int k = threadIdx.x; k < kNParams; k += kTrainThreads) grad_out[k] = mlp_grad_total(red, k);
+    if (threadIdx.x == 0) loss_out[0] = mlp_grad_total(red, kNParams) * scale;
 }
 
 // ---------------------------------------------------------------------------

@@ -95,6 +95,12 @@ int vs_polygon_bounds(const double* x, const double* y, const int32_t* geom_offs
  * (kernels/core/geometry_analysis_source.py:31-72). */
 int vs_point_boxes(const double* px, const double* py, int64_t n, double* boxes, void* stream);
 
+/* out5 (device) = union (x0, y0, x1, y1) and number of the boxes whose four
+ * bounds are finite ((inf, inf, -inf, -inf, 0) when there is none). */
+int64_t vs_boxes_extent_workspace_bytes(void);
+int vs_boxes_extent(const double* boxes, int64_t n, double* out5, void* workspace, int64_t workspace_bytes,
+                    void* stream);
+
 /* ---------------------------------------------------------------------
  * Packed Hilbert tree over boxes
  * --------------------------------------------------------------------- */

@@ -63,6 +63,8 @@ SIGNATURES = {
     "vs_last_error": (ctypes.c_int, [ctypes.c_char_p, _i64]),
     "vs_polygon_bounds": (ctypes.c_int, [_p, _p, _p, _p, _p, _i64, _p, _p]),
     "vs_point_boxes": (ctypes.c_int, [_p, _p, _i64, _p, _p]),
+    "vs_boxes_extent_workspace_bytes": (_i64, []),
+    "vs_boxes_extent": (ctypes.c_int, [_p, _i64, _p, _p, _i64, _p]),
     "vs_tree_plan": (ctypes.c_int, [_i64, _i32, _LP]),
     "vs_index_workspace_bytes": (_i64, [_i64]),
     "vs_index_build": (ctypes.c_int, [_p, _i64, _LP, _p, _p, _p, _p, _i64, _p]),

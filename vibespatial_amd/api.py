@@ -138,6 +138,7 @@ class _FamilyIndex:
         self.ga = ga
         self._trees = {}
         self._bounds = {}
+        self._extents = {}
         self._learned = None
 
     def bounds(self, family: str) -> torch.Tensor:
@@ -151,6 +152,13 @@ class _FamilyIndex:
                 b = _family_bounds_device(self.ga)
             self._bounds[family] = b
         return b
+
+    def extent(self, family: str):
+        """(x0, y0, x1, y1, count) of the family's rows with finite bounds."""
+        e = self._extents.get(family)
+        if e is None:
+            e = self._extents[family] = J.boxes_extent(self.bounds(family))
+        return e
 
     def tree(self, family: str) -> J.DeviceTree:
         t = self._trees.get(family)
@@ -238,7 +246,7 @@ def _strategy(q_fam: str, t_fam: str, predicate, qarr) -> str:
 
 def _pairs_family(q_fam: str, qarr, t_fam: str, tarr, tindex: _FamilyIndex, predicate, dist=None, log=None):
     """Pairs (query family idx, tree family idx), lexsorted, device int64.
-    dist: per query-family row distances (fp64) for dwithin.  log: a list the
+    dist: dwithin's distance, one float or one per query-family row (fp64).  log: a list the
     chosen strategy is appended to."""
     dev = require_gpu()
     if predicate in _EMPTY_PAIRS.get((q_fam, t_fam), ()):
@@ -262,7 +270,10 @@ def _pairs_family(q_fam: str, qarr, t_fam: str, tarr, tindex: _FamilyIndex, pred
     if predicate == "dwithin":
         # boxes grown by each row's distance (outward-rounded), then the exact
         # distance refine (spatial/query.py:663-826 route)
-        d = torch.as_tensor(np.ascontiguousarray(dist, dtype=np.float64), device=dev)
+        if isinstance(dist, float):
+            d = torch.full((len(qarr),), dist, dtype=torch.float64, device=dev)
+        else:
+            d = torch.as_tensor(np.ascontiguousarray(dist, dtype=np.float64), device=dev)
         qb = J.point_boxes(device_points(qarr)) if q_fam == "point" else J.polygon_bounds(device_polygons(qarr))
         l, r, _ = J.query_boxes(J.expand_boxes(qb, d), tree, kind="dwithin")
         return J.refine_dwithin(l, r, d, _dev_geom(q_fam, qarr), _dev_geom(t_fam, tarr))
@@ -277,17 +288,28 @@ def _pairs_family(q_fam: str, qarr, t_fam: str, tarr, tindex: _FamilyIndex, pred
     raise NotImplementedError(f"{q_fam} x {t_fam} predicate {predicate!r}")
 
 
+def _identity_rows(rows: np.ndarray) -> bool:
+    return len(rows) == 0 or (rows[0] == 0 and rows[-1] == len(rows) - 1)
+
+
+def _rows_distance(distance, rows: np.ndarray):
+    """The distances of a family's column rows (None and one float as they are)."""
+    if distance is None or isinstance(distance, float) or _identity_rows(rows) and len(rows) == len(distance):
+        return distance
+    return distance[rows]
+
+
 def _map_rows(idx: torch.Tensor, rows: np.ndarray) -> torch.Tensor:
     """Family index -> column row (rows ascending, so order is kept)."""
-    if len(rows) == 0 or (rows[0] == 0 and rows[-1] == len(rows) - 1):
-        return idx  # identity
+    if _identity_rows(rows):
+        return idx
     return torch.as_tensor(rows, device=idx.device)[idx]
 
 
 def query_pairs(query: GeometryArray, tree_ga: GeometryArray, tindex: _FamilyIndex, predicate, distance=None,
                 log=None):
     """Lexsorted (query_row, tree_row) pairs as device int64 tensors.
-    distance: per query row fp64 array (dwithin only); log: a list that
+    distance (dwithin only): one float or a per query row fp64 array; log: a list that
     receives (query family, tree family, strategy) per family pair."""
     dev = require_gpu()
     fams_q = [(f, a, rows) for f, a, rows in (("point", query.points, query.point_rows),
@@ -296,13 +318,13 @@ def query_pairs(query: GeometryArray, tree_ga: GeometryArray, tindex: _FamilyInd
                                                ("polygon", tree_ga.polygons, tree_ga.polygon_rows)) if a is not None]
     if len(fams_q) == 1 and len(fams_t) == 1:
         (qf, qa, qrows), (tf, ta, trows) = fams_q[0], fams_t[0]
-        dist = None if distance is None else distance[qrows]
+        dist = _rows_distance(distance, qrows)
         l, r = _pairs_family(qf, qa, tf, ta, tindex, predicate, dist, log)
         return _map_rows(l, qrows), _map_rows(r, trows)
     parts_l, parts_r = [], []
     for qf, qa, qrows in fams_q:
         for tf, ta, trows in fams_t:
-            dist = None if distance is None else distance[qrows]
+            dist = _rows_distance(distance, qrows)
             l, r = _pairs_family(qf, qa, tf, ta, tindex, predicate, dist, log)
             parts_l.append(qrows[l.cpu().numpy()])
             parts_r.append(trows[r.cpu().numpy()])
@@ -372,17 +394,23 @@ class SpatialIndex:
         else:
             dist = None
             if predicate == "dwithin":
+                dist = np.asarray(distance, dtype=np.float64)
                 try:
-                    dist = np.ascontiguousarray(np.broadcast_to(np.asarray(distance, dtype=np.float64), (len(q),)))
+                    rows = np.broadcast_to(dist, (len(q),))
                 except ValueError as exc:
                     raise ValueError("distance array must be broadcastable to the geometry input") from exc
+                # one distance stays one number: its rows are filled on the device
+                if rows.strides == (0,):
+                    dist = float(rows[0])
+                elif dist.shape != rows.shape or not dist.flags.writeable:
+                    dist = rows.copy()
             self.last_strategy = []
             l, r = query_pairs(q, self._ga, self._index, predicate, dist, self.last_strategy)
         if return_device:
             return r if scalar else torch.stack([l, r])
+        if output_format == "indices":  # one copy of the stacked rows
+            return r.cpu().numpy() if scalar else torch.stack([l, r]).cpu().numpy()
         lh, rh = l.cpu().numpy(), r.cpu().numpy()
-        if output_format == "indices":
-            return rh if scalar else np.vstack([lh, rh])
         n_tree = len(self._ga)
         if scalar:
             dense = np.zeros(n_tree, dtype=bool)
@@ -399,20 +427,15 @@ class SpatialIndex:
     def _nearest_family(self, qf, qa, tf, ta, max_distance, return_all, exclusive):
         """(query family idx, tree family idx, distance) device tensors."""
         qb = J.point_boxes(device_points(qa)) if qf == "point" else J.polygon_bounds(device_polygons(qa))
-        tb_h, qb_h = ta.bounds(), qa.bounds()
-        fin = np.isfinite(tb_h).all(axis=1)
-        if not fin.any():
+        tx0, ty0, tx1, ty1, n_t = self._index.extent(tf)
+        if n_t == 0:
             return None
-        both = np.concatenate([tb_h[fin], qb_h[np.isfinite(qb_h).all(axis=1)]])
-        x0, y0 = both[:, 0].min(), both[:, 1].min()
-        x1, y1 = both[:, 2].max(), both[:, 3].max()
+        qx0, qy0, qx1, qy1, _ = J.boxes_extent(qb)
         # a radius at which every grown query box covers every tree box
-        cover = float(np.hypot(x1 - x0, y1 - y0)) * 1.01 + 1e-300
+        cover = float(np.hypot(max(tx1, qx1) - min(tx0, qx0), max(ty1, qy1) - min(ty0, qy0))) * 1.01 + 1e-300
         if not np.isfinite(cover):
             cover = float(np.finfo(np.float64).max)
-        t0, t1 = tb_h[fin].min(axis=0), tb_h[fin].max(axis=0)
-        w, h = t1[2] - t0[0], t1[3] - t0[1]
-        n_t = int(fin.sum())
+        w, h = tx1 - tx0, ty1 - ty0
         # the mean spacing of the tree rows as the first radius
         start = float(np.sqrt(w * h / n_t)) if w > 0 and h > 0 else max(w, h) / n_t
         if not (start > 0) or not np.isfinite(start):
@@ -446,8 +469,12 @@ class SpatialIndex:
                 res = self._nearest_family(qf, qa, tf, ta, max_distance, return_all or len(fams_t) > 1, exclusive)
                 if res is None:
                     continue
-                l, r, d = (t.cpu().numpy() for t in res)
-                parts.append((qrows[l], trows[r], d))
+                l, r, d = res
+                l, r = _map_rows(l, qrows), _map_rows(r, trows)
+                if len(fams_q) == 1 and len(fams_t) == 1:  # in order already
+                    idx = torch.stack([l, r]).cpu().numpy()
+                    return (idx, d.cpu().numpy()) if return_distance else idx
+                parts.append((l.cpu().numpy(), r.cpu().numpy(), d.cpu().numpy()))
         if parts:
             lh = np.concatenate([p[0] for p in parts]).astype(np.int64)
             rh = np.concatenate([p[1] for p in parts]).astype(np.int64)

@@ -230,6 +230,64 @@ __global__ __launch_bounds__(256) void extent_final_kernel(const double4* __rest
 
 constexpr int kExtentBlocks = 2048;  // 8 blocks per CU
 
+// Union and number of the boxes whose four bounds are finite, in blocks of
+// grid-stride rows; the last step folds the blocks' parts.
+__global__ __launch_bounds__(256) void boxes_extent_kernel(const double4* __restrict__ b, int64_t n,
+                                                          double4* __restrict__ part, double* __restrict__ count) {
+    __shared__ double4 red[4];
+    __shared__ double cnt[4];
+    double x0 = INFINITY, y0 = INFINITY, x1 = -INFINITY, y1 = -INFINITY, k = 0.0;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        const double4 v = b[i];
+        if (isfinite(v.x) && isfinite(v.y) && isfinite(v.z) && isfinite(v.w)) {
+            x0 = fmin(x0, v.x); y0 = fmin(y0, v.y);
+            x1 = fmax(x1, v.z); y1 = fmax(y1, v.w);
+            k += 1.0;
+        }
+    }
+    x0 = wave_min(x0); y0 = wave_min(y0); x1 = wave_max(x1); y1 = wave_max(y1);
+    for (int o = 32; o > 0; o >>= 1) k += __shfl_xor(k, o, 64);
+    if ((threadIdx.x & 63) == 0) {
+        red[threadIdx.x >> 6] = make_double4(x0, y0, x1, y1);
+        cnt[threadIdx.x >> 6] = k;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double4 r = red[0];
+        for (int w = 1; w < 4; ++w) {
+            r.x = fmin(r.x, red[w].x); r.y = fmin(r.y, red[w].y);
+            r.z = fmax(r.z, red[w].z); r.w = fmax(r.w, red[w].w);
+        }
+        part[blockIdx.x] = r;
+        count[blockIdx.x] = cnt[0] + cnt[1] + cnt[2] + cnt[3];
+    }
+}
+
+__global__ __launch_bounds__(256) void boxes_extent_final_kernel(const double4* __restrict__ part,
+                                                                const double* __restrict__ count, int nb,
+                                                                double* __restrict__ out5) {
+    double x0 = INFINITY, y0 = INFINITY, x1 = -INFINITY, y1 = -INFINITY, k = 0.0;
+    if (threadIdx.x < 64) {
+        for (int i = threadIdx.x; i < nb; i += 64) {
+            const double4 v = part[i];
+            x0 = fmin(x0, v.x); y0 = fmin(y0, v.y);
+            x1 = fmax(x1, v.z); y1 = fmax(y1, v.w);
+            k += count[i];
+        }
+        x0 = wave_min(x0); y0 = wave_min(y0); x1 = wave_max(x1); y1 = wave_max(y1);
+        for (int o = 32; o > 0; o >>= 1) k += __shfl_xor(k, o, 64);
+        if (threadIdx.x == 0) {
+            out5[0] = x0;
+            out5[1] = y0;
+            out5[2] = x1;
+            out5[3] = y1;
+            out5[4] = k;
+        }
+    }
+}
+
+constexpr int kBoxesExtentBlocks = 512;
+
 int64_t extent_workspace_bytes() { return sizeof(double4) * (kExtentBlocks + 1) + 256; }
 
 int centre_extent(const double4* b, int64_t n, double4* ext, void* ws, hipStream_t s) {
@@ -662,6 +720,32 @@ int vs_polygon_bounds(const double* x, const double* y, const int32_t* geom_offs
     VS_REQUIRE(n_rows >= 0, "vs_polygon_bounds: negative n_rows");
     return vs::polygon_bounds(x, y, geom_offsets, part_offsets, ring_offsets, n_rows, bounds,
                               vs::stream_of(stream));
+}
+
+int64_t vs_boxes_extent_workspace_bytes(void) {
+    vs::Carver c(nullptr);
+    c.take<double4>(vs::kBoxesExtentBlocks);
+    c.take<double>(vs::kBoxesExtentBlocks);
+    return c.bytes;
+}
+
+int vs_boxes_extent(const double* boxes, int64_t n, double* out5, void* workspace, int64_t workspace_bytes,
+                    void* stream) {
+    vs::clear_error();
+    VS_REQUIRE(n >= 0, "vs_boxes_extent: negative n");
+    VS_REQUIRE(out5 != nullptr, "vs_boxes_extent: null result");
+    VS_REQUIRE(workspace_bytes >= vs_boxes_extent_workspace_bytes(), "vs_boxes_extent: workspace too small");
+    vs::Carver c(workspace);
+    double4* part = c.take<double4>(vs::kBoxesExtentBlocks);
+    double* count = c.take<double>(vs::kBoxesExtentBlocks);
+    hipStream_t s = vs::stream_of(stream);
+    const int nb = (int)std::min<int64_t>(vs::kBoxesExtentBlocks, std::max<int64_t>(1, vs::ceil_div(n, 256)));
+    hipLaunchKernelGGL(vs::boxes_extent_kernel, dim3(nb), dim3(256), 0, s, reinterpret_cast<const double4*>(boxes), n,
+                       part, count);
+    VS_LAUNCH_CHECK();
+    hipLaunchKernelGGL(vs::boxes_extent_final_kernel, dim3(1), dim3(64), 0, s, part, count, nb, out5);
+    VS_LAUNCH_CHECK();
+    return VS_OK;
 }
 
 int vs_point_boxes(const double* px, const double* py, int64_t n, double* boxes, void* stream) {

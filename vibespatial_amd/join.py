@@ -88,6 +88,18 @@ def point_boxes(Q: DevicePoints) -> torch.Tensor:
     return out
 
 
+def boxes_extent(boxes: torch.Tensor) -> tuple[float, float, float, float, int]:
+    """(x0, y0, x1, y1, count) of the (n, 4) device boxes with finite bounds
+    (vs_boxes_extent); synchronises."""
+    dev = require_gpu()
+    out = torch.empty(5, dtype=torch.float64, device=dev)
+    ws = _ws(lib().vs_boxes_extent_workspace_bytes(), dev)
+    check(lib().vs_boxes_extent(ptr(boxes), int(boxes.shape[0]), ptr(out), ptr(ws), ws.numel(), stream()),
+          "vs_boxes_extent")
+    *box, count = out.cpu().tolist()
+    return (*box, int(count))
+
+
 def build_tree(bounds: torch.Tensor, fanout: int = FANOUT) -> DeviceTree:
     """vs_index_build over (n, 4) fp64 device boxes."""
     dev = require_gpu()

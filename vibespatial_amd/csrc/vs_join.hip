@@ -170,16 +170,15 @@ __device__ bool refine_pip_wave(double px, double py, bool active, int32_t c0, i
 
 // Persistent traversal kernel.  MODE kModePip: queries are points (qa, qb =
 // sorted x, y), 64 per wave, with fused refine.  MODE kModeBox: queries are
-// boxes given as (qbox, perm) and every bbox pair is emitted; with one_box,
-// one box per wave (claimed kBoxClaim at a time): the lanes test a node's
-// children and a leaf group's hits are appended with one ballot (boxes with
-// many hits); else 64 boxes per wave walk the union of their boxes (many
-// boxes with few hits).
+// boxes given as (qbox, perm) and every bbox pair is emitted, one box per wave
+// (claimed kBoxClaim at a time): the lanes test a node's children and a leaf
+// group's hits are appended with one ballot (boxes with many hits; boxes with
+// few go through box_walk_kernel).
 template <int MODE, int PRED>
 __global__ __launch_bounds__(kJoinThreads) void traverse_kernel(
     const double* __restrict__ qx, const double* __restrict__ qy, const double4* __restrict__ qbox,
     const int32_t* __restrict__ perm, int64_t n, TreeView T, PolyView P, uint32_t* __restrict__ stage_l,
-    int32_t* __restrict__ stage_r, int64_t capacity, JoinCtl* __restrict__ ctl, int one_box) {
+    int32_t* __restrict__ stage_r, int64_t capacity, JoinCtl* __restrict__ ctl) {
     __shared__ double4 top[kTopMax];
     __shared__ long long stack_s[kJoinWaves][MODE == kModeBox ? kStackMaxBox : kStackMax];
     __shared__ int2 outbuf_s[kJoinWaves][kOutBuf];
@@ -209,9 +208,8 @@ __global__ __launch_bounds__(kJoinThreads) void traverse_kernel(
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         nbuf = 0;
     };
-    // work units: kBoxClaim boxes (one-box mode) or 64 queries
-    const bool one = MODE == kModeBox && one_box;
-    const int64_t W = one ? (n + kBoxClaim - 1) / kBoxClaim : (n + 63) >> 6;
+    // work units: kBoxClaim boxes or 64 points
+    const int64_t W = MODE == kModeBox ? (n + kBoxClaim - 1) / kBoxClaim : (n + 63) >> 6;
     const int home = blockIdx.x & 7;
     const int last = T.n_levels - 1;
     const int F = T.fanout;
@@ -227,7 +225,7 @@ __global__ __launch_bounds__(kJoinThreads) void traverse_kernel(
             ++xq;
             continue;
         }
-        if (one) {
+        if (MODE == kModeBox) {
             for (int bq = 0; bq < kBoxClaim; ++bq) {
                 const int64_t qi = (r0 + t) * kBoxClaim + bq;  // wave-uniform
                 if (qi >= n) break;
@@ -275,22 +273,11 @@ __global__ __launch_bounds__(kJoinThreads) void traverse_kernel(
         }
         const int64_t idx = (r0 + t) * 64 + lane;
         const bool inr = idx < n;
-        double x0, y0, x1, y1;
-        int32_t orig = 0;
-        if (MODE == kModePip) {
-            x0 = inr ? qx[idx] : NAN;
-            y0 = inr ? qy[idx] : NAN;
-            x1 = x0;
-            y1 = y0;
-            orig = inr ? perm[idx] : 0;
-        } else {
-            orig = inr ? (perm ? perm[idx] : (int32_t)idx) : 0;
-            const double4 b = inr ? qbox[orig] : make_double4(NAN, NAN, NAN, NAN);
-            x0 = b.x; y0 = b.y; x1 = b.z; y1 = b.w;
-        }
-        const bool valid = inr && x0 == x0 && y0 == y0 && x1 == x1 && y1 == y1;
+        const double x0 = inr ? qx[idx] : NAN, y0 = inr ? qy[idx] : NAN;
+        const int32_t orig = inr ? perm[idx] : 0;
+        const bool valid = inr && x0 == x0 && y0 == y0;
         const double ux0 = wave_min(valid ? x0 : INFINITY), uy0 = wave_min(valid ? y0 : INFINITY);
-        const double ux1 = wave_max(valid ? x1 : -INFINITY), uy1 = wave_max(valid ? y1 : -INFINITY);
+        const double ux1 = wave_max(valid ? x0 : -INFINITY), uy1 = wave_max(valid ? y0 : -INFINITY);
         if (__ballot(valid) != 0 && T.level_count[0] > 0) {
             int sp = 1;
             if (lane == 0) stack[0] = 0;  // group 0 of level 0 = the root
@@ -317,22 +304,17 @@ __global__ __launch_bounds__(kJoinThreads) void traverse_kernel(
                         m &= m - 1;
                         const double bx0 = readlane_f64(b.x, s), by0 = readlane_f64(b.y, s);
                         const double bx1 = readlane_f64(b.z, s), by1 = readlane_f64(b.w, s);
-                        const bool hit = valid && box_overlap(x0, y0, x1, y1, bx0, by0, bx1, by1);
+                        const bool hit = valid && box_overlap(x0, y0, x0, y0, bx0, by0, bx1, by1);
                         const uint64_t hm = __ballot(hit);
                         if (!hm) continue;
                         const int32_t row = T.item_ids[first + s];
-                        bool res;
-                        if (MODE == kModePip) {
-                            const int2 rng = P.item_range[first + s];
-                            const unsigned long long h = (unsigned long long)__popcll(hm);
-                            st_cand += h;
-                            st_cverts += h * (unsigned long long)(rng.y - rng.x);
-                            // every active point lies in (wave box) x (item box)
-                            res = refine_pip_wave<PRED>(x0, y0, hit, rng.x, rng.y, fmax(ux0, bx0), fmax(uy0, by0),
-                                                        fmin(uy1, by1), P);
-                        } else {
-                            res = hit;
-                        }
+                        const int2 rng = P.item_range[first + s];
+                        const unsigned long long h = (unsigned long long)__popcll(hm);
+                        st_cand += h;
+                        st_cverts += h * (unsigned long long)(rng.y - rng.x);
+                        // every active point lies in (wave box) x (item box)
+                        const bool res = refine_pip_wave<PRED>(x0, y0, hit, rng.x, rng.y, fmax(ux0, bx0),
+                                                               fmax(uy0, by0), fmin(uy1, by1), P);
                         const uint64_t rm = __ballot(res);
                         if (rm) {
                             const int k = __popcll(rm);
@@ -358,6 +340,223 @@ __global__ __launch_bounds__(kJoinThreads) void traverse_kernel(
         atomicAdd(&ctl->stat[0], st_cand);
         atomicAdd(&ctl->stat[1], st_cverts);
     }
+}
+
+// ---------------------------------------------------------------------------
+// Many query boxes with few hits each: a wave walks the tree with the union of
+// 64 boxes that are neighbours in Hilbert order.
+//
+// Every step takes as many node groups off the stack as the wave has lanes for
+// (four of fanout 16), so a small union needs one step per level; item ids are
+// loaded with the item boxes.  Where the boxes lie far apart their union covers
+// far more items than they hit: a union that meets more than kWalkSplit items'
+// worth of the nodes staged in LDS is walked as four units of 16 boxes, and
+// those as four of 4; each item is then tested by 16 or 4 lanes, 4 or 16 items
+// at a time.
+//
+// Bound by latency and by the atomics on the stage counter, not by work (3% of
+// the issue slots): each costs about 20 ns in turn, whichever wave sends it.
+// So the units are dealt out in turn with no queue, and a wave buffers 1,024
+// pairs.  3M points x 100k boxes (6.4M pairs): 2,180 us with one node group
+// per step, item ids loaded one by one, unions left whole, eight queues and 256
+// pairs a wave; 1,410 with the steps and splits above; 470 without the queues;
+// 250 with the larger buffer.  72k scattered boxes of a nearest search: 1,410 ->
+// 144 us; 100k x 100k polygon boxes: 231 -> 58 us.
+// ---------------------------------------------------------------------------
+constexpr int kWalkStack = 1152;  // 640 staged nodes + at most 60 more entries per level below + one step's 64
+constexpr int kWalkSplit = 1024;
+constexpr int kWalkBlocks = 2;   // blocks per compute unit (LDS)
+
+constexpr int kWalkOut = 1024;   // pairs buffered per wave
+
+struct WalkLds {
+    uint32_t group[kWalkStack];
+    uint8_t level[kWalkStack];
+    int2 out[kWalkOut];
+};
+
+struct BoxWalk {
+    const TreeView& T;
+    const double4* top;               // LDS: T.box[0, T.n_top)
+    const long long* level_start;     // LDS copies of the layout
+    const long long* level_count;
+    WalkLds& W;
+    uint32_t* stage_l;
+    int32_t* stage_r;
+    int64_t capacity;
+    JoinCtl* ctl;
+    int lane, slot, child, groups;    // lane = slot * fanout + child; groups per step
+    int staged_level;                 // last staged level (-1: none)
+    int64_t staged_first, staged_count, staged_items;
+    int nbuf;
+
+    __device__ __forceinline__ void fence() const {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+
+    // Appends the wave's buffered pairs to the stage with one atomic.
+    __device__ void flush() {
+        if (nbuf == 0) return;
+        unsigned long long base = 0;
+        if (lane == 0) base = atomicAdd(&ctl->staged, (unsigned long long)nbuf);
+        base = __shfl(base, 0, 64);
+        fence();
+        for (int i = lane; i < nbuf; i += 64) {
+            const unsigned long long at = base + (unsigned long long)i;
+            if (at < (unsigned long long)capacity) {
+                const int2 e = W.out[i];
+                stage_l[at] = (uint32_t)e.x;
+                stage_r[at] = e.y;
+            }
+        }
+        fence();
+        nbuf = 0;
+    }
+
+    // U boxes, box k in the lanes k, k + U, ...
+    template <int U>
+    __device__ void walk(double x0, double y0, double x1, double y1, bool valid, int32_t orig) {
+        constexpr int R = 64 / U;  // items tested at a time
+        if (__ballot(valid) == 0) return;
+        const uint64_t lt = lanemask_lt();
+        const double ux0 = wave_min(valid ? x0 : INFINITY), uy0 = wave_min(valid ? y0 : INFINITY);
+        const double ux1 = wave_max(valid ? x1 : -INFINITY), uy1 = wave_max(valid ? y1 : -INFINITY);
+        const int last = T.n_levels - 1;
+        int sp = 0;
+        if (staged_level < 0) {
+            if (lane == 0) {
+                W.group[0] = 0;
+                W.level[0] = 0;
+            }
+            sp = 1;
+        }
+        for (int64_t j0 = 0; j0 < staged_count; j0 += 64) {
+            const int64_t j = j0 + lane;
+            bool ov = j < staged_count;
+            if (ov) {
+                const double4 b = top[staged_first + j];
+                ov = box_overlap(ux0, uy0, ux1, uy1, b.x, b.y, b.z, b.w);
+            }
+            const uint64_t m = __ballot(ov);
+            if (ov) {
+                const int at = sp + __popcll(m & lt);
+                W.group[at] = (uint32_t)j;
+                W.level[at] = (uint8_t)(staged_level + 1);
+            }
+            sp += __popcll(m);
+        }
+        if constexpr (U > 4) {
+            if ((int64_t)sp * staged_items > kWalkSplit) {
+                for (int k = 0; k < 4; ++k) {
+                    const int from = k * (U / 4) + (lane & (U / 4 - 1));
+                    walk<U / 4>(__shfl(x0, from, 64), __shfl(y0, from, 64), __shfl(x1, from, 64),
+                                __shfl(y1, from, 64), __shfl((int)valid, from, 64) != 0, __shfl(orig, from, 64));
+                }
+                return;
+            }
+        }
+        const int sub = lane / U;
+        while (sp > 0) {
+            fence();
+            const int np = sp < groups ? sp : groups;
+            const bool act = slot < np;
+            const int at = act ? sp - 1 - slot : 0;
+            const int l = W.level[at];
+            const int64_t pos = (int64_t)W.group[at] * T.fanout + child;
+            sp -= np;
+            fence();
+            const bool in = act && pos < level_count[l];
+            double4 b = make_double4(NAN, NAN, NAN, NAN);
+            if (in) {
+                const int64_t g = level_start[l] + pos;
+                b = g < T.n_top ? top[g] : T.box[g];
+            }
+            const bool leaf = in && l == last;
+            int32_t id = 0;
+            if (leaf) id = T.item_ids[pos];
+            const bool ov = in && box_overlap(ux0, uy0, ux1, uy1, b.x, b.y, b.z, b.w);
+            const uint64_t mi = __ballot(ov && !leaf);
+            if (ov && !leaf) {
+                const int to = sp + __popcll(mi & lt);
+                W.group[to] = (uint32_t)pos;
+                W.level[to] = (uint8_t)(l + 1);
+            }
+            sp += __popcll(mi);
+            uint64_t ml = __ballot(ov && leaf);
+            while (ml) {
+                bool hit = valid;
+                int32_t row;
+                if constexpr (U == 64) {
+                    const int src = __ffsll((unsigned long long)ml) - 1;
+                    ml &= ml - 1;
+                    hit = hit && box_overlap(x0, y0, x1, y1, readlane_f64(b.x, src), readlane_f64(b.y, src),
+                                             readlane_f64(b.z, src), readlane_f64(b.w, src));
+                    row = readlane_i32(id, src);
+                } else {
+                    int src = -1;
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        const int bit = ml ? __ffsll((unsigned long long)ml) - 1 : -1;
+                        ml &= ml - 1;  // 0 stays 0
+                        if (sub == r) src = bit;
+                    }
+                    const int from = src < 0 ? 0 : src;
+                    const double bx0 = __shfl(b.x, from, 64), by0 = __shfl(b.y, from, 64);
+                    const double bx1 = __shfl(b.z, from, 64), by1 = __shfl(b.w, from, 64);
+                    row = __shfl(id, from, 64);
+                    hit = hit && src >= 0 && box_overlap(x0, y0, x1, y1, bx0, by0, bx1, by1);
+                }
+                const uint64_t h = __ballot(hit);
+                if (!h) continue;
+                const int k = __popcll(h);
+                if (nbuf + k > kWalkOut) flush();
+                if (hit) W.out[nbuf + __popcll(h & lt)] = make_int2(orig, row);
+                nbuf += k;
+            }
+        }
+    }
+};
+
+// unit: boxes per work unit, 64 or 16 (when 64 would leave waves without work).
+__global__ __launch_bounds__(kJoinThreads) void box_walk_kernel(const double4* __restrict__ qbox,
+                                                               const int32_t* __restrict__ perm, int64_t n, int unit,
+                                                               TreeView T, uint32_t* __restrict__ stage_l,
+                                                               int32_t* __restrict__ stage_r, int64_t capacity,
+                                                               JoinCtl* __restrict__ ctl) {
+    __shared__ double4 top[kTopMax];
+    __shared__ long long level_start[VS_MAX_LEVELS], level_count[VS_MAX_LEVELS];
+    __shared__ WalkLds lds[kJoinWaves];
+    for (int i = threadIdx.x; i < T.n_top; i += kJoinThreads) top[i] = T.box[i];
+    if (threadIdx.x < VS_MAX_LEVELS) {
+        level_start[threadIdx.x] = T.level_start[threadIdx.x];
+        level_count[threadIdx.x] = T.level_count[threadIdx.x];
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & 63;
+    int staged_level = -1;
+    for (int l = 0; l + 1 < T.n_levels; ++l)
+        if (T.level_start[l] + T.level_count[l] <= T.n_top) staged_level = l;
+    const bool st = staged_level >= 0;
+    const int64_t n_staged = st ? T.level_count[staged_level] : 0;
+    const int64_t n_items = T.level_count[T.n_levels - 1];
+    BoxWalk walk = {T, top, level_start, level_count, lds[threadIdx.x >> 6], stage_l, stage_r, capacity, ctl,
+                    lane, lane / T.fanout, lane % T.fanout, 64 / T.fanout,
+                    staged_level, st ? T.level_start[staged_level] : 0, n_staged,
+                    st ? (n_items + n_staged - 1) / n_staged : 0, 0};
+    const int64_t units = (n + unit - 1) / unit;
+    const int64_t waves = (int64_t)gridDim.x * kJoinWaves;
+    for (int64_t u = (int64_t)blockIdx.x * kJoinWaves + uniform_i32(threadIdx.x >> 6); u < units; u += waves) {
+        const int64_t idx = u * unit + (lane & (unit - 1));
+        const bool inr = idx < n;
+        const int32_t orig = inr ? perm[idx] : 0;
+        const double4 b = inr ? qbox[orig] : make_double4(NAN, NAN, NAN, NAN);
+        const bool valid = b.x == b.x && b.y == b.y && b.z == b.z && b.w == b.w;
+        if (unit == 64) walk.walk<64>(b.x, b.y, b.z, b.w, valid, orig);
+        else walk.walk<16>(b.x, b.y, b.z, b.w, valid, orig);
+    }
+    walk.flush();
 }
 
 // Refine-layout preparation (per join: O(V + R + P + M), tiny next to the join).
@@ -505,12 +704,12 @@ int timing_end_public(hipStream_t s) { return timing_end(s); }
 template <int MODE>
 int launch_traverse(int pred, const double* qx, const double* qy, const double4* qbox,
                     const int32_t* perm, int64_t n, const TreeView& T, const PolyView& P,
-                    const JoinWs& J, int64_t capacity, hipStream_t s, bool one_box = false) {
-    const int grid = grid_for(one_box ? ceil_div(n, kBoxClaim) : ceil_div(n, 64));
+                    const JoinWs& J, int64_t capacity, hipStream_t s) {
+    const int grid = grid_for(MODE == kModeBox ? ceil_div(n, kBoxClaim) : ceil_div(n, 64));
     VS_TRY(timing_begin(s));
 #define VS_LAUNCH_T(PR)                                                                          \
     hipLaunchKernelGGL((traverse_kernel<MODE, PR>), dim3(grid), dim3(kJoinThreads), 0, s, qx, qy, \
-                       qbox, perm, n, T, P, J.stage_l, J.stage_r, capacity, J.ctl, (int)one_box)
+                       qbox, perm, n, T, P, J.stage_l, J.stage_r, capacity, J.ctl)
     switch (pred) {
         case VS_PRED_WITHIN: VS_LAUNCH_T(VS_PRED_WITHIN); break;
         case VS_PRED_INTERSECTS: VS_LAUNCH_T(VS_PRED_INTERSECTS); break;
@@ -519,6 +718,19 @@ int launch_traverse(int pred, const double* qx, const double* qy, const double4*
         default: VS_REQUIRE(false, "unsupported predicate %d for this join", pred);
     }
 #undef VS_LAUNCH_T
+    VS_LAUNCH_CHECK();
+    VS_TRY(timing_end(s));
+    return VS_OK;
+}
+
+int launch_box_walk(const double4* qbox, const int32_t* perm, int64_t n, const TreeView& T, const JoinWs& J,
+                    int64_t capacity, hipStream_t s) {
+    // units of 64 boxes once every wave of a full grid gets several of them
+    const int64_t full = stride_grid(INT64_MAX / 2, kJoinThreads, kWalkBlocks);
+    const int unit = n >= 2 * 64 * kJoinWaves * full ? 64 : 16;
+    const int grid = (int)std::min<int64_t>(full, ceil_div(n, (int64_t)unit * kJoinWaves));
+    VS_TRY(timing_begin(s));
+    hipLaunchKernelGGL(box_walk_kernel, dim3(grid), dim3(kJoinThreads), 0, s, qbox, perm, n, unit, T, J.stage_l, J.stage_r, capacity, J.ctl);
     VS_LAUNCH_CHECK();
     VS_TRY(timing_end(s));
     return VS_OK;
@@ -715,9 +927,11 @@ int vs_query_boxes(const double* query_boxes, int64_t n_queries, const vs_tree_l
         VS_TRY(vs::box_order(qb, n_queries, J.perm, J.order_ws, s));  // waves of nearby boxes
         // the traversal's shape follows the hits the caller expects per box
         // (capacity / n_queries); both shapes give the same pairs
-        const bool one_box = capacity >= (int64_t)vs::kOneBoxHits * n_queries;
-        VS_TRY(vs::launch_traverse<vs::kModeBox>(VS_PRED_INTERSECTS, nullptr, nullptr, qb, J.perm, n_queries, T, P,
-                                                 J, capacity, s, one_box));
+        if (capacity >= (int64_t)vs::kOneBoxHits * n_queries)
+            VS_TRY(vs::launch_traverse<vs::kModeBox>(VS_PRED_INTERSECTS, nullptr, nullptr, qb, J.perm, n_queries, T, P,
+                                                     J, capacity, s));
+        else
+            VS_TRY(vs::launch_box_walk(qb, J.perm, n_queries, T, J, capacity, s));
     }
     return vs::finish_pairs(J.fin_ws, J.ctl, n_queries, layout->n_items, capacity, sort != 0, out_left, out_right,
                              d_result, s);

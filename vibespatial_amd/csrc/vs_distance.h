@@ -246,14 +246,60 @@ __device__ inline bool point_polygon_within(double px, double py, const Polys& P
     const double lim = far_limit(d);
     for (int32_t pp = p0; pp < p1; ++pp) {
         int parity = 0;
-        for (int32_t r = P.part[pp]; r < P.part[pp + 1]; ++r)
-            for (int32_t c = P.ring[r] + 1; c < P.ring[r + 1]; ++c) {
-                const double ax = P.x[c - 1], ay = P.y[c - 1], bx = P.x[c], by = P.y[c];
-                if (!segment_far(px, py, ax, ay, bx, by, lim) && point_segment_within(px, py, ax, ay, bx, by, d))
-                    return true;
-                if (edge_step_f64(px, py, ax, ay, bx, by, parity)) return true;  // on the boundary
-            }
+        for (int32_t r = P.part[pp]; r < P.part[pp + 1]; ++r) {
+            const bool hit = any_near_edge(
+                P, P.ring[r], P.ring[r + 1], px, py, lim, parity, [&](double ax, double ay, double bx, double by) {
+                    return (!segment_far(px, py, ax, ay, bx, by, lim) &&
+                            point_segment_within(px, py, ax, ay, bx, by, d)) ||
+                           edge_step_f64(px, py, ax, ay, bx, by, parity) != 0;  // within d, or on the boundary
+                });
+            if (hit) return true;
+        }
         if (parity) return true;  // inside this part
+    }
+    return false;
+}
+
+// point_polygon_within by one wave (every lane returns the answer), for rows of
+// many edges: lanes split each part's edges, a part's parity is the parity of
+// its lanes' sum.
+__device__ inline bool wave_point_polygon_within(double px, double py, const Polys& P, int64_t row, double d,
+                                                 int lane) {
+    if (!(d >= 0.0) || px != px || py != py) return false;
+    const int32_t p0 = P.geom[row], p1 = P.geom[row + 1];
+    if (P.ring[P.part[p1]] <= P.ring[P.part[p0]]) return false;  // empty
+    if (d == INFINITY) return true;
+    const double lim = far_limit(d);
+    for (int32_t pp = p0; pp < p1; ++pp) {
+        const RowSpan s = {P.ring[P.part[pp]], P.ring[P.part[pp + 1]], P.part[pp], P.part[pp + 1]};
+        int parity = 0;
+        for (int32_t c0 = s.lo + 1; c0 < s.hi; c0 += 4 * 64) {
+            double ax[4], ay[4], bx[4], by[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int32_t c = c0 + k * 64 + lane < s.hi ? c0 + k * 64 + lane : s.hi - 1;  // c >= lo + 1
+                ax[k] = P.x[c - 1];
+                ay[k] = P.y[c - 1];
+                bx[k] = P.x[c];
+                by[k] = P.y[c];
+            }
+            bool hit = false;
+            uint32_t left = 0;  // this lane's edges that are not apart
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (is_row_edge(P, s, c0 + k * 64 + lane) &&
+                    !edge_apart(see_vertex(ax[k], ay[k], px, py, lim), see_vertex(bx[k], by[k], px, py, lim), parity))
+                    left |= 1u << k;
+            for (; left; left &= left - 1u) {
+                const int32_t c = c0 + (__ffs(left) - 1) * 64 + lane;
+                const double qx = P.x[c - 1], qy = P.y[c - 1], rx = P.x[c], ry = P.y[c];
+                hit |= (!segment_far(px, py, qx, qy, rx, ry, lim) &&
+                        point_segment_within(px, py, qx, qy, rx, ry, d)) ||
+                       edge_step_f64(px, py, qx, qy, rx, ry, parity) != 0;  // within d, or on the boundary
+            }
+            if (__ballot(hit) != 0) return true;
+        }
+        if (__popcll(__ballot(parity)) & 1) return true;  // inside this part
     }
     return false;
 }

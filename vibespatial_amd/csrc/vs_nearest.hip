@@ -88,27 +88,78 @@ __device__ double boundary_dist_f64(double px, double py, const Polys& P, int64_
 __device__ double point_polygon_dist_f64(double px, double py, const Polys& P, int64_t row, bool outside,
                                          double cap) {
     if (px != px || py != py || poly_empty(P, row)) return INFINITY;
-    double best = cap;
+    double best = cap, lim = best * (1.0 + 0x1p-30);
     bool found = false;
     for (int32_t pp = P.geom[row]; pp < P.geom[row + 1]; ++pp) {
         int parity = 0;
-        for (int32_t r = P.part[pp]; r < P.part[pp + 1]; ++r)
-            for (int32_t c = P.ring[r] + 1; c < P.ring[r + 1]; ++c) {
-                const double ax = P.x[c - 1], ay = P.y[c - 1], bx = P.x[c], by = P.y[c];
-                if (!outside && edge_step_f64(px, py, ax, ay, bx, by, parity)) return 0.0;  // on the boundary
-                const double lim = best * (1.0 + 0x1p-30);
-                if (px - fmax(ax, bx) > lim || fmin(ax, bx) - px > lim || py - fmax(ay, by) > lim ||
-                    fmin(ay, by) - py > lim)
+        for (int32_t r = P.part[pp]; r < P.part[pp + 1]; ++r) {
+            const bool on = any_near_edge(
+                P, P.ring[r], P.ring[r + 1], px, py, lim, parity, [&](double ax, double ay, double bx, double by) {
+                    if (!outside && edge_step_f64(px, py, ax, ay, bx, by, parity)) return true;
+                    if (px - fmax(ax, bx) > lim || fmin(ax, bx) - px > lim || py - fmax(ay, by) > lim ||
+                        fmin(ay, by) - py > lim)
+                        return false;
+                    const double d = segment_dist_f64(px, py, ax, ay, bx, by);
+                    if (d <= best) {
+                        best = d;
+                        lim = best * (1.0 + 0x1p-30);
+                        found = true;
+                    }
+                    return false;
+                });
+            if (on) return 0.0;  // on the boundary
+        }
+        if (!outside && parity) return 0.0;  // inside this part
+    }
+    return found ? best : INFINITY;
+}
+
+// point_polygon_dist_f64 by one wave (every lane returns the distance): the
+// least over the same segment distances, each lane skipping segments farther
+// than its own least one.
+__device__ double wave_point_polygon_dist_f64(double px, double py, const Polys& P, int64_t row, bool outside,
+                                              double cap, int lane) {
+    if (px != px || py != py || poly_empty(P, row)) return INFINITY;
+    double best = cap, lim = best * (1.0 + 0x1p-30);
+    bool found = false;
+    for (int32_t pp = P.geom[row]; pp < P.geom[row + 1]; ++pp) {
+        const RowSpan s = {P.ring[P.part[pp]], P.ring[P.part[pp + 1]], P.part[pp], P.part[pp + 1]};
+        int parity = 0;
+        bool on = false;
+        for (int32_t c0 = s.lo + 1; c0 < s.hi; c0 += 4 * 64) {
+            double ax[4], ay[4], bx[4], by[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int32_t c = c0 + k * 64 + lane < s.hi ? c0 + k * 64 + lane : s.hi - 1;  // c >= lo + 1
+                ax[k] = P.x[c - 1];
+                ay[k] = P.y[c - 1];
+                bx[k] = P.x[c];
+                by[k] = P.y[c];
+            }
+            uint32_t left = 0;  // this lane's edges that are not apart
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (is_row_edge(P, s, c0 + k * 64 + lane) &&
+                    !edge_apart(see_vertex(ax[k], ay[k], px, py, lim), see_vertex(bx[k], by[k], px, py, lim), parity))
+                    left |= 1u << k;
+            for (; left; left &= left - 1u) {
+                const int32_t c = c0 + (__ffs(left) - 1) * 64 + lane;
+                const double qx = P.x[c - 1], qy = P.y[c - 1], rx = P.x[c], ry = P.y[c];
+                if (!outside) on |= edge_step_f64(px, py, qx, qy, rx, ry, parity) != 0;
+                if (px - fmax(qx, rx) > lim || fmin(qx, rx) - px > lim || py - fmax(qy, ry) > lim ||
+                    fmin(qy, ry) - py > lim)
                     continue;
-                const double d = segment_dist_f64(px, py, ax, ay, bx, by);
+                const double d = segment_dist_f64(px, py, qx, qy, rx, ry);
                 if (d <= best) {
                     best = d;
+                    lim = best * (1.0 + 0x1p-30);
                     found = true;
                 }
             }
-        if (parity) return 0.0;  // inside this part
+        }
+        if (!outside && (__ballot(on) != 0 || (__popcll(__ballot(parity)) & 1))) return 0.0;  // on the boundary or inside
     }
-    return found ? best : INFINITY;
+    return wave_min(found ? best : INFINITY);
 }
 
 __device__ double polygons_dist_f64(const Polys& A, int64_t ra, const Polys& B, int64_t rb) {
@@ -130,17 +181,23 @@ __device__ double polygons_dist_f64(const Polys& A, int64_t ra, const Polys& B, 
 // (order[t]) when given.
 constexpr int kDistExclusive = 1, kDistOutside = 2;
 
-__global__ __launch_bounds__(256) void pair_distances_kernel(int left_kind, int right_kind,
+template <int left_kind, int right_kind>  // one body for each: the pairs of polygons need the most registers
+__global__ __launch_bounds__(256) void pair_distances_kernel(
                                                             const int64_t* __restrict__ left,
                                                             const int64_t* __restrict__ right, int64_t n,
                                                             const int32_t* __restrict__ order, int flags,
                                                             const double* __restrict__ cap, Polys L, Polys R,
-                                                            double* __restrict__ out) {
+                                                            double* __restrict__ out, int32_t* __restrict__ heavy,
+                                                            unsigned long long* __restrict__ n_heavy) {
     for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < n; t += (int64_t)gridDim.x * 256) {
         const int64_t i = order ? (int64_t)order[t] : t;
         const int64_t l = left[i], r = right[i];
         const double c = cap && cap[l] == cap[l] ? cap[l] : INFINITY;  // NaN: no cap
         double d;
+        if (left_kind + right_kind == 1 && row_coords(left_kind ? L : R, left_kind ? l : r) > kWaveRowCoords) {
+            heavy[atomicAdd(n_heavy, 1ull)] = (int32_t)i;  // one atomic per wave
+            continue;
+        }
         if (left_kind == 0 && right_kind == 0) {
             const double px = L.x[l], py = L.y[l], qx = R.x[r], qy = R.y[r];
             if (px != px || py != py || qx != qx || qy != qy) d = INFINITY;
@@ -155,6 +212,30 @@ __global__ __launch_bounds__(256) void pair_distances_kernel(int left_kind, int 
         }
         out[i] = d > c ? INFINITY : d;
     }
+}
+
+// One wave per listed pair of a point and a row of many coordinates.
+__global__ __launch_bounds__(256) void pair_distances_wave_kernel(int left_kind, const int64_t* __restrict__ left,
+                                                                 const int64_t* __restrict__ right,
+                                                                 const int32_t* __restrict__ heavy,
+                                                                 const unsigned long long* __restrict__ n_heavy,
+                                                                 int flags, const double* __restrict__ cap, Polys L,
+                                                                 Polys R, double* __restrict__ out) {
+    const int lane = threadIdx.x & 63;
+    const int64_t m = (int64_t)*n_heavy;
+    for (int64_t w = (int64_t)blockIdx.x * 4 + uniform_i32(threadIdx.x >> 6); w < m; w += (int64_t)gridDim.x * 4) {
+        const int64_t i = heavy[w];
+        const int64_t l = left[i], r = right[i];
+        const double c = cap && cap[l] == cap[l] ? cap[l] : INFINITY;  // NaN: no cap
+        const double d = left_kind == 0 ? wave_point_polygon_dist_f64(L.x[l], L.y[l], R, r,
+                                                                      (flags & kDistOutside) != 0, c, lane)
+                                        : wave_point_polygon_dist_f64(R.x[r], R.y[r], L, l, false, c, lane);
+        if (lane == 0) out[i] = d > c ? INFINITY : d;
+    }
+}
+
+__global__ void zero_heavy_kernel(unsigned long long* c) {
+    if (threadIdx.x == 0) *c = 0;
 }
 
 __global__ __launch_bounds__(256) void right_order_keys_kernel(const int64_t* __restrict__ right, int64_t n,
@@ -173,6 +254,7 @@ int64_t pair_distances_workspace_bytes(int64_t n) {
     c.take<uint32_t>(n);
     c.take<int32_t>(n);
     c.take<char>(sort_workspace_bytes_u32(n));
+    c.take<unsigned long long>(1);
     return c.bytes;
 }
 
@@ -371,6 +453,7 @@ struct NearestTree {
 constexpr int kBoundStack = 256;
 constexpr int kBoundPops = 4096;  // visit limit per query (bounds the time of a pathological query)
 constexpr int kBoundExact = 2;    // exact item distances per query
+constexpr int kBoundWide = 16;    // up to this many lanes' wide rows are measured by the whole wave, one by one
 
 __device__ __forceinline__ double box_gap2(const double4 q, const double4 b) {
     const double gx = fmax(0.0, fmax(b.x - q.z, q.x - b.z));
@@ -378,57 +461,83 @@ __device__ __forceinline__ double box_gap2(const double4 q, const double4 b) {
     return gx * gx + gy * gy;
 }
 
-__device__ double nearest_upper_bound(const double4 q, const NearestTree& T) {
+//
+// The wave's lanes walk until each holds an item to measure (or is done), and
+// measure together: one by one they would each hold up the other 63 for a
+// whole polygon.  Rows of more than kWaveRowCoords coordinates are measured by
+// the whole wave, one after the other.
+__device__ double nearest_upper_bound(const double4 q, const NearestTree& T, bool live, int lane) {
     int64_t stack[kBoundStack];
     int sp = 0;
     const int last = T.n_levels - 1;
-    for (int64_t c = 0; c < T.level_count[0] && sp < kBoundStack; ++c) stack[sp++] = c;  // level 0
+    for (int64_t c = 0; live && c < T.level_count[0] && sp < kBoundStack; ++c) stack[sp++] = c;  // level 0
     double ub2 = INFINITY;
     int exact = (T.polys && q.x == q.z && q.y == q.w) ? kBoundExact : 0;
-    for (int pops = 0; sp > 0 && pops < kBoundPops; ++pops) {
-        const int64_t e = stack[--sp];
-        const int l = (int)(e >> 48);
-        const int64_t c = e & ((1ll << 48) - 1);
-        const double4 b = T.box[T.level_start[l] + c];
-        if (!(b.x == b.x) || box_gap2(q, b) > ub2) continue;
-        if (l == last) {
-            // farthest point of the query box from the item box, and from a
-            // point of the item itself (never farther, often much nearer)
-            const double dx = fmax(q.z - b.x, b.z - q.x), dy = fmax(q.w - b.y, b.w - q.y);
-            ub2 = fmin(ub2, dx * dx + dy * dy);
-            const double2 p = T.rep[c];
-            if (p.x == p.x) {
-                const double ex = fmax(fabs(p.x - q.x), fabs(p.x - q.z)), ey = fmax(fabs(p.y - q.y), fabs(p.y - q.w));
-                ub2 = fmin(ub2, ex * ex + ey * ey);
+    int pops = 0;
+    for (;;) {
+        int32_t item = -1;  // row to measure
+        for (; sp > 0 && pops < kBoundPops && item < 0; ++pops) {
+            const int64_t e = stack[--sp];
+            const int l = (int)(e >> 48);
+            const int64_t c = e & ((1ll << 48) - 1);
+            const double4 b = T.box[T.level_start[l] + c];
+            if (!(b.x == b.x) || box_gap2(q, b) > ub2) continue;
+            if (l == last) {
+                // farthest point of the query box from the item box, and from a
+                // point of the item itself (never farther, often much nearer)
+                const double dx = fmax(q.z - b.x, b.z - q.x), dy = fmax(q.w - b.y, b.w - q.y);
+                ub2 = fmin(ub2, dx * dx + dy * dy);
+                const double2 p = T.rep[c];
+                if (p.x == p.x) {
+                    const double ex = fmax(fabs(p.x - q.x), fabs(p.x - q.z)), ey = fmax(fabs(p.y - q.y), fabs(p.y - q.w));
+                    ub2 = fmin(ub2, ex * ex + ey * ey);
+                }
+                if (exact > 0) {
+                    --exact;
+                    item = T.item_ids[c];
+                }
+                continue;
             }
-            if (exact > 0) {
-                --exact;
-                // at most the box bound just taken up to rounding; +inf
-                // (rounding, empty row) leaves the bound as it is
-                const double d = point_polygon_dist_f64(q.x, q.y, T.P, T.item_ids[c], false, sqrt(ub2));
-                if (d < INFINITY) ub2 = fmin(ub2, d * d);
+            const int64_t lo = c * T.fanout;
+            const int64_t hi = lo + T.fanout < T.level_count[l + 1] ? lo + T.fanout : T.level_count[l + 1];
+            // push the children within the bound, the nearest one last (popped first)
+            int64_t best = -1;
+            double bestd = INFINITY;
+            for (int64_t k0 = lo; k0 < hi; k0 += 4) {
+                double4 cb[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) cb[u] = T.box[T.level_start[l + 1] + (k0 + u < hi ? k0 + u : hi - 1)];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int64_t k = k0 + u;
+                    if (k >= hi || !(cb[u].x == cb[u].x)) continue;
+                    const double g = box_gap2(q, cb[u]);
+                    if (g > ub2) continue;
+                    if (g < bestd) {
+                        if (best >= 0 && sp < kBoundStack) stack[sp++] = ((int64_t)(l + 1) << 48) | best;
+                        best = k;
+                        bestd = g;
+                    } else if (sp < kBoundStack) {
+                        stack[sp++] = ((int64_t)(l + 1) << 48) | k;
+                    }
+                }
             }
-            continue;
+            if (best >= 0 && sp < kBoundStack) stack[sp++] = ((int64_t)(l + 1) << 48) | best;
         }
-        const int64_t lo = c * T.fanout;
-        const int64_t hi = lo + T.fanout < T.level_count[l + 1] ? lo + T.fanout : T.level_count[l + 1];
-        // push the children within the bound, the nearest one last (popped first)
-        int64_t best = -1;
-        double bestd = INFINITY;
-        for (int64_t k = lo; k < hi; ++k) {
-            const double4 cb = T.box[T.level_start[l + 1] + k];
-            if (!(cb.x == cb.x)) continue;
-            const double g = box_gap2(q, cb);
-            if (g > ub2) continue;
-            if (g < bestd) {
-                if (best >= 0 && sp < kBoundStack) stack[sp++] = ((int64_t)(l + 1) << 48) | best;
-                best = k;
-                bestd = g;
-            } else if (sp < kBoundStack) {
-                stack[sp++] = ((int64_t)(l + 1) << 48) | k;
-            }
+        if (__ballot(item >= 0) == 0) break;
+        // a distance is at most the box bound just taken up to rounding; +inf
+        // (rounding, empty row) leaves the bound as it is
+        bool wide = item >= 0 && row_coords(T.P, item) > kWaveRowCoords;
+        if (__popcll(__ballot(wide)) > kBoundWide) wide = false;
+        double d = INFINITY;
+        if (item >= 0 && !wide) d = point_polygon_dist_f64(q.x, q.y, T.P, item, false, sqrt(ub2));
+        for (uint64_t m = __ballot(wide); m; m &= m - 1) {
+            const int j = __ffsll((unsigned long long)m) - 1;
+            const double dj = wave_point_polygon_dist_f64(__shfl(q.x, j), __shfl(q.y, j), T.P, __shfl(item, j), false,
+                                                          sqrt(__shfl(ub2, j)), lane);
+            if (lane == j) d = dj;
         }
-        if (best >= 0 && sp < kBoundStack) stack[sp++] = ((int64_t)(l + 1) << 48) | best;
+        if (d < INFINITY) ub2 = fmin(ub2, d * d);
     }
     return sqrt(ub2) * (1.0 + 0x1p-40);
 }
@@ -443,10 +552,9 @@ __global__ __launch_bounds__(256) void nearest_bound_kernel(const double4* __res
                                                            NearestTree T, double cap, double* __restrict__ radius,
                                                            double* __restrict__ search) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= m) return;
-    const int64_t q = rows[perm[i]];
-    const double ub = nearest_upper_bound(qboxes[q], T);
-    if (ub < INFINITY) {
+    const int64_t q = rows[perm[i < m ? i : m - 1]];
+    const double ub = nearest_upper_bound(qboxes[q], T, i < m, threadIdx.x & 63);  // whole waves
+    if (i < m && ub < INFINITY) {
         const double r = fmin(ub, cap);
         radius[q] = r;
         search[q] = r * kSearchSlack;
@@ -558,6 +666,7 @@ int vs_pair_distances(int32_t left_kind, int32_t right_kind, const int64_t* left
     uint32_t* key_out = c.take<uint32_t>(n_pairs);
     int32_t* order = c.take<int32_t>(n_pairs);
     void* sort_ws = c.take<char>(vs::sort_workspace_bytes_u32(n_pairs));
+    unsigned long long* n_heavy = c.take<unsigned long long>(1);
     const vs::Polys L = {lx, ly, l_geom, l_part, l_ring};
     const vs::Polys R = {rx, ry, r_geom, r_part, r_ring};
     const int32_t* ord = nullptr;
@@ -572,9 +681,24 @@ int vs_pair_distances(int32_t left_kind, int32_t right_kind, const int64_t* left
         ord = order;
     }
     const int grid = (int)std::min<int64_t>(vs::ceil_div(n_pairs, 256), 16384);
-    hipLaunchKernelGGL(vs::pair_distances_kernel, dim3(grid), dim3(256), 0, s, left_kind, right_kind, left, right,
-                       n_pairs, ord, flags & (vs::kDistExclusive | vs::kDistOutside), cap, L, R, out_distance);
+    int32_t* heavy = idx_in;  // free after the sort
+    const bool mixed = left_kind + right_kind == 1;
+    flags &= vs::kDistExclusive | vs::kDistOutside;
+    if (mixed) {
+        hipLaunchKernelGGL(vs::zero_heavy_kernel, dim3(1), dim3(64), 0, s, n_heavy);
+        VS_LAUNCH_CHECK();
+    }
+    auto kernel = left_kind == 0 ? (right_kind == 0 ? vs::pair_distances_kernel<0, 0> : vs::pair_distances_kernel<0, 1>)
+                                 : (right_kind == 0 ? vs::pair_distances_kernel<1, 0> : vs::pair_distances_kernel<1, 1>);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, s, left, right, n_pairs, ord, flags, cap, L, R, out_distance,
+                       heavy, n_heavy);
     VS_LAUNCH_CHECK();
+    if (mixed) {
+        hipLaunchKernelGGL(vs::pair_distances_wave_kernel,
+                           dim3((unsigned)std::min<int64_t>(vs::ceil_div(n_pairs, 4), 2048)), dim3(256), 0, s,
+                           left_kind, left, right, heavy, n_heavy, flags, cap, L, R, out_distance);
+        VS_LAUNCH_CHECK();
+    }
     return VS_OK;
 }
 

@@ -15,6 +15,118 @@ struct Polys {
     const int32_t* ring;
 };
 
+__device__ inline int32_t row_coords(const Polys& P, int64_t row) {
+    return P.ring[P.part[P.geom[row + 1]]] - P.ring[P.part[P.geom[row]]];
+}
+
+// A vertex as a point p sees it: beyond p by more than lim to the left, right,
+// below or above, and above p's rightward ray.  Rounding is monotone, so the
+// differences decide exactly what the same tests on an edge's least and
+// greatest coordinates would.
+struct SeenVertex {
+    double x, y;
+    bool l, r, d, u, above;
+};
+
+__device__ __forceinline__ SeenVertex see_vertex(double x, double y, double px, double py, double lim) {
+    const double dx = x - px, dy = y - py;
+    return {x, y, dx < -lim, dx > lim, dy < -lim, dy > lim, dy > 0.0};
+}
+
+// Edge a->b is farther than lim on an axis, on one side of p: it can neither
+// come within lim nor hold p, and p's ray crosses it only to the right.
+__device__ __forceinline__ bool edge_apart(const SeenVertex& a, const SeenVertex& b, int& parity) {
+    const bool right = a.r && b.r;
+    parity ^= (int)(right && a.above != b.above);
+    return right || (a.l && b.l) || (a.d && b.d) || (a.u && b.u);
+}
+
+// near(ax, ay, bx, by) over the edges of the ring of coordinates [lo, hi) that
+// are not apart from p, until it returns true (then true is returned).  The
+// lanes of a wave (points of one polygon, mostly) first pass over 32 edges with
+// the 7 instructions that set apart ones aside, the next four vertices being
+// loaded meanwhile, and then take the edges left to each together: testing
+// edge by edge, nearly every edge is near for some lane and all 64 wait for
+// its 60 instructions.
+template <class F>
+__device__ __forceinline__ bool any_near_edge(const Polys& P, int32_t lo, int32_t hi, double px, double py,
+                                              const double& lim, int& parity, F&& near) {
+    constexpr int kAhead = 4;
+    if (hi - lo < 2) return false;
+    SeenVertex a = see_vertex(P.x[lo], P.y[lo], px, py, lim);
+    double nx[kAhead], ny[kAhead];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+        const int32_t c = lo + 1 + k < hi ? lo + 1 + k : hi - 1;
+        nx[k] = P.x[c];
+        ny[k] = P.y[c];
+    }
+    for (int32_t base = lo + 1; base < hi; base += 32) {
+        uint32_t left = 0;  // edges base + bit that are not apart
+        for (int32_t c0 = base; c0 < hi && c0 < base + 32; c0 += kAhead) {
+            uint32_t some = 0;
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) {
+                const SeenVertex b = see_vertex(nx[k], ny[k], px, py, lim);
+                // past the ring's end its last vertex is read again: an edge
+                // of no length, which crosses no ray
+                some |= edge_apart(a, b, parity) ? 0u : 1u << k;
+                a = b;
+                const int32_t c = c0 + kAhead + k < hi ? c0 + kAhead + k : hi - 1;
+                nx[k] = P.x[c];
+                ny[k] = P.y[c];
+            }
+            left |= some << (c0 - base);
+        }
+        if (hi - base < 32) left &= (1u << (hi - base)) - 1u;
+        while (left) {
+            const int32_t c = base + __ffs(left) - 1;
+            left &= left - 1u;
+            if (near(P.x[c - 1], P.y[c - 1], P.x[c], P.y[c])) return true;
+        }
+    }
+    return false;
+}
+
+// Point x polygon pairs of rows with more coordinates than this get a wave of
+// their own, so that no lane walks thousands of edges while the chip idles.
+// Rows with fewer are cheaper by lanes, which share the row's loads (6.6M
+// dwithin pairs of rows of 3 to 2,048 coordinates, lanes + waves: from 128
+// coordinates on 773 + 581 us, from 256 918 + 112, from 512 1020 + 20, with no
+// rule and edge by edge 1828; 1.4M distances: 400 + 117, 432 + 27, 571 + 18, 900).
+constexpr int32_t kWaveRowCoords = 256;
+
+// Coordinates [lo, hi) of a row and its rings [r0, r1).
+struct RowSpan {
+    int32_t lo, hi, r0, r1;
+};
+
+__device__ __forceinline__ RowSpan row_span(const Polys& P, int64_t row) {
+    RowSpan s;
+    s.r0 = P.part[P.geom[row]];
+    s.r1 = P.part[P.geom[row + 1]];
+    s.lo = P.ring[s.r0];
+    s.hi = P.ring[s.r1];
+    return s;
+}
+
+// (c - 1, c) is an edge of the row: c lies in it and starts none of its rings.
+__device__ __forceinline__ bool is_row_edge(const Polys& P, const RowSpan& s, int32_t c) {
+    if (c <= s.lo || c >= s.hi) return false;
+    if (s.r1 - s.r0 <= 8) {
+        bool start = false;
+        for (int32_t r = s.r0 + 1; r < s.r1; ++r) start |= P.ring[r] == c;
+        return !start;
+    }
+    int32_t lo = s.r0 + 1, hi = s.r1;
+    while (lo < hi) {
+        const int32_t m = (lo + hi) >> 1;
+        if (P.ring[m] < c) lo = m + 1;
+        else hi = m;
+    }
+    return lo >= s.r1 || P.ring[lo] != c;
+}
+
 // Exact `intersects` of row ra of A and row rb of B
 // (src/vibespatial/predicates/polygon_kernels.py:163-228): some boundary
 // segment of A touches or crosses one of B, else a point of one lies in the

@@ -153,22 +153,46 @@ __global__ void total_to_result_kernel(const long long* __restrict__ total, int6
 // rows.  d = distance[left row].
 // Pairs are visited in right-row order (order[t]), so the lanes of a wave
 // mostly share one right geometry: same coordinates, same loop lengths.
-__global__ __launch_bounds__(256) void dwithin_pairs_kernel(int left_kind, int right_kind,
+template <int left_kind, int right_kind>  // one body for each: the pairs of polygons need the most registers
+__global__ __launch_bounds__(256) void dwithin_pairs_kernel(
                                                            const int64_t* __restrict__ left,
                                                            const int64_t* __restrict__ right, int64_t n,
                                                            const int32_t* __restrict__ order,
                                                            const double* __restrict__ distance, Polys L, Polys R,
-                                                           int32_t* __restrict__ keep) {
+                                                           int32_t* __restrict__ keep, int32_t* __restrict__ heavy,
+                                                           unsigned long long* __restrict__ n_heavy) {
     for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < n; t += (int64_t)gridDim.x * 256) {
         const int64_t i = order[t];
         const int64_t l = left[i], r = right[i];
         const double d = distance[l];
         bool k;
+        if (left_kind + right_kind == 1 && row_coords(left_kind ? L : R, left_kind ? l : r) > kWaveRowCoords) {
+            heavy[atomicAdd(n_heavy, 1ull)] = (int32_t)i;  // one atomic per wave
+            continue;
+        }
         if (left_kind == 0 && right_kind == 0) k = point_point_within(L.x[l], L.y[l], R.x[r], R.y[r], d);
         else if (left_kind == 0) k = point_polygon_within(L.x[l], L.y[l], R, r, d);
         else if (right_kind == 0) k = point_polygon_within(R.x[r], R.y[r], L, l, d);
         else k = polygons_within(L, l, R, r, d);
         keep[i] = k ? 1 : 0;
+    }
+}
+
+// One wave per listed pair of a point and a row of many coordinates.
+__global__ __launch_bounds__(256) void dwithin_wave_kernel(int left_kind, const int64_t* __restrict__ left,
+                                                          const int64_t* __restrict__ right,
+                                                          const int32_t* __restrict__ heavy,
+                                                          const unsigned long long* __restrict__ n_heavy,
+                                                          const double* __restrict__ distance, Polys L, Polys R,
+                                                          int32_t* __restrict__ keep) {
+    const int lane = threadIdx.x & 63;
+    const int64_t m = (int64_t)*n_heavy;
+    for (int64_t w = (int64_t)blockIdx.x * 4 + uniform_i32(threadIdx.x >> 6); w < m; w += (int64_t)gridDim.x * 4) {
+        const int64_t i = heavy[w];
+        const int64_t l = left[i], r = right[i];
+        const bool k = left_kind == 0 ? wave_point_polygon_within(L.x[l], L.y[l], R, r, distance[l], lane)
+                                      : wave_point_polygon_within(R.x[r], R.y[r], L, l, distance[l], lane);
+        if (lane == 0) keep[i] = k ? 1 : 0;
     }
 }
 
@@ -191,6 +215,7 @@ int64_t dwithin_workspace_bytes(int64_t n) {
     c.take<uint32_t>(n);
     c.take<int32_t>(n);
     c.take<char>(sort_workspace_bytes_u32(n));
+    c.take<unsigned long long>(2);
     return c.bytes;
 }
 
@@ -380,6 +405,7 @@ int vs_refine_dwithin(int32_t left_kind, int32_t right_kind, const int64_t* left
     uint32_t* key_out = c.take<uint32_t>(n_pairs);
     int32_t* order = c.take<int32_t>(n_pairs);
     void* sort_ws = c.take<char>(vs::sort_workspace_bytes_u32(n_pairs));
+    unsigned long long* n_heavy = c.take<unsigned long long>(2);
     vs::Carver cr(refine_ws);
     int32_t* keep = cr.take<int32_t>(n_pairs);
     int32_t* pos = cr.take<int32_t>(n_pairs);
@@ -396,9 +422,23 @@ int vs_refine_dwithin(int32_t left_kind, int32_t right_kind, const int64_t* left
         VS_TRY(vs::sort_pairs_into_u32(key_in, idx_in, key_out, order, n_pairs, 0, bits, sort_ws,
                                        vs::sort_workspace_bytes_u32(n_pairs), s));
         const int grid = (int)std::min<int64_t>(vs::ceil_div(n_pairs, 256), 16384);
-        hipLaunchKernelGGL(vs::dwithin_pairs_kernel, dim3(grid), dim3(256), 0, s, left_kind, right_kind, left, right,
-                           n_pairs, order, distance, L, R, keep);
+        int32_t* heavy = idx_in;  // free after the sort
+        if (left_kind + right_kind == 1) {
+            hipLaunchKernelGGL(vs::zero_count_kernel, dim3(1), dim3(64), 0, s, n_heavy);
+            VS_LAUNCH_CHECK();
+        }
+        auto kernel = left_kind == 0
+                          ? (right_kind == 0 ? vs::dwithin_pairs_kernel<0, 0> : vs::dwithin_pairs_kernel<0, 1>)
+                          : (right_kind == 0 ? vs::dwithin_pairs_kernel<1, 0> : vs::dwithin_pairs_kernel<1, 1>);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, s, left, right, n_pairs, order, distance, L, R, keep,
+                           heavy, n_heavy);
         VS_LAUNCH_CHECK();
+        if (left_kind + right_kind == 1) {
+            hipLaunchKernelGGL(vs::dwithin_wave_kernel,
+                               dim3((unsigned)std::min<int64_t>(vs::ceil_div(n_pairs, 4), 2048)), dim3(256), 0, s,
+                               left_kind, left, right, heavy, n_heavy, distance, L, R, keep);
+            VS_LAUNCH_CHECK();
+        }
     }
     VS_TRY(vs::exclusive_scan_i32(keep, pos, n_pairs, total, scan_ws, s));
     if (n_pairs > 0) {

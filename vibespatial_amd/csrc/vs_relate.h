@@ -347,10 +347,6 @@ VS_HD bool polygon_predicate(int pred, const Polys& A, int64_t ra, const Polys& 
 // ---------------------------------------------------------------------------
 // One wave per pair, for pairs of large rows.
 // ---------------------------------------------------------------------------
-__device__ inline int32_t row_coords(const Polys& P, int64_t row) {
-    return P.ring[P.part[P.geom[row + 1]]] - P.ring[P.part[P.geom[row]]];
-}
-
 // One wave's LDS for wave_edge_pairs.
 constexpr int kEdgeTile = 128;
 struct WaveEdgeLds {
@@ -365,37 +361,6 @@ __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Coordinates [lo, hi) of a row and its rings [r0, r1).
-struct RowSpan {
-    int32_t lo, hi, r0, r1;
-};
-
-__device__ __forceinline__ RowSpan row_span(const Polys& P, int64_t row) {
-    RowSpan s;
-    s.r0 = P.part[P.geom[row]];
-    s.r1 = P.part[P.geom[row + 1]];
-    s.lo = P.ring[s.r0];
-    s.hi = P.ring[s.r1];
-    return s;
-}
-
-// (c - 1, c) is an edge of the row: c lies in it and starts none of its rings.
-__device__ __forceinline__ bool is_row_edge(const Polys& P, const RowSpan& s, int32_t c) {
-    if (c <= s.lo || c >= s.hi) return false;
-    if (s.r1 - s.r0 <= 8) {
-        bool start = false;
-        for (int32_t r = s.r0 + 1; r < s.r1; ++r) start |= P.ring[r] == c;
-        return !start;
-    }
-    int32_t lo = s.r0 + 1, hi = s.r1;
-    while (lo < hi) {
-        const int32_t m = (lo + hi) >> 1;
-        if (P.ring[m] < c) lo = m + 1;
-        else hi = m;
-    }
-    return lo >= s.r1 || P.ring[lo] != c;
 }
 
 // Boxes in fp32, every bound rounded to nearest.  Rounding is monotone, so

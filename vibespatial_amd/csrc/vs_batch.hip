@@ -295,13 +295,6 @@ __global__ __launch_bounds__(256) void task_recs_kernel(const int64_t* __restric
 }
 
 // Persistent: waves take (job, 64 sorted left rows) tasks round-robin.
-// Orders one wave's LDS accesses where its lanes exchange data through LDS.
-__device__ __forceinline__ void wave_lds_order() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 __global__ __launch_bounds__(256) void forest_query_kernel(const double4* __restrict__ lbox,
                                                           const int32_t* __restrict__ lperm,
                                                           const TaskRec* __restrict__ tasks,

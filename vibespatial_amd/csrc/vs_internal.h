@@ -179,6 +179,13 @@ __device__ __forceinline__ double uniform_f64(double v) {
     return u.d;
 }
 
+// Orders one wave's LDS accesses where its lanes exchange data through LDS.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 template <class T>
 __device__ __forceinline__ T wave_min(T v) {
     for (int o = 32; o > 0; o >>= 1) {

@@ -114,11 +114,14 @@ __device__ double point_polygon_dist_f64(double px, double py, const Polys& P, i
     return found ? best : INFINITY;
 }
 
-// point_polygon_dist_f64 by one wave (every lane returns the distance): the
-// least over the same segment distances, each lane skipping segments farther
-// than its own least one.
-__device__ double wave_point_polygon_dist_f64(double px, double py, const Polys& P, int64_t row, bool outside,
-                                              double cap, int lane) {
+// point_polygon_dist_f64 by W lanes in step (16: a quarter of the wave; all of
+// them return the distance): the least over the same segment distances, each
+// lane skipping segments farther than its own least one.
+template <int W>
+__device__ double lanes_point_polygon_dist_f64(double px, double py, const Polys& P, int64_t row, bool outside,
+                                               double cap, int lane) {
+    const uint64_t mine = W == 64 ? ~0ull : ((1ull << (W & 63)) - 1) << (lane & ~(W - 1));  // lane: of the wave
+    lane &= W - 1;
     if (px != px || py != py || poly_empty(P, row)) return INFINITY;
     double best = cap, lim = best * (1.0 + 0x1p-30);
     bool found = false;
@@ -126,11 +129,11 @@ __device__ double wave_point_polygon_dist_f64(double px, double py, const Polys&
         const RowSpan s = {P.ring[P.part[pp]], P.ring[P.part[pp + 1]], P.part[pp], P.part[pp + 1]};
         int parity = 0;
         bool on = false;
-        for (int32_t c0 = s.lo + 1; c0 < s.hi; c0 += 4 * 64) {
+        for (int32_t c0 = s.lo + 1; c0 < s.hi; c0 += 4 * W) {
             double ax[4], ay[4], bx[4], by[4];
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                const int32_t c = c0 + k * 64 + lane < s.hi ? c0 + k * 64 + lane : s.hi - 1;  // c >= lo + 1
+                const int32_t c = c0 + k * W + lane < s.hi ? c0 + k * W + lane : s.hi - 1;  // c >= lo + 1
                 ax[k] = P.x[c - 1];
                 ay[k] = P.y[c - 1];
                 bx[k] = P.x[c];
@@ -139,11 +142,11 @@ __device__ double wave_point_polygon_dist_f64(double px, double py, const Polys&
             uint32_t left = 0;  // this lane's edges that are not apart
 #pragma unroll
             for (int k = 0; k < 4; ++k)
-                if (is_row_edge(P, s, c0 + k * 64 + lane) &&
+                if (is_row_edge(P, s, c0 + k * W + lane) &&
                     !edge_apart(see_vertex(ax[k], ay[k], px, py, lim), see_vertex(bx[k], by[k], px, py, lim), parity))
                     left |= 1u << k;
             for (; left; left &= left - 1u) {
-                const int32_t c = c0 + (__ffs(left) - 1) * 64 + lane;
+                const int32_t c = c0 + (__ffs(left) - 1) * W + lane;
                 const double qx = P.x[c - 1], qy = P.y[c - 1], rx = P.x[c], ry = P.y[c];
                 if (!outside) on |= edge_step_f64(px, py, qx, qy, rx, ry, parity) != 0;
                 if (px - fmax(qx, rx) > lim || fmin(qx, rx) - px > lim || py - fmax(qy, ry) > lim ||
@@ -157,9 +160,11 @@ __device__ double wave_point_polygon_dist_f64(double px, double py, const Polys&
                 }
             }
         }
-        if (!outside && (__ballot(on) != 0 || (__popcll(__ballot(parity)) & 1))) return 0.0;  // on the boundary or inside
+        if (!outside && ((__ballot(on) & mine) != 0 || (__popcll(__ballot(parity) & mine) & 1))) return 0.0;  // on the boundary or inside
     }
-    return wave_min(found ? best : INFINITY);
+    best = found ? best : INFINITY;
+    for (int o = W / 2; o > 0; o >>= 1) best = fmin(best, __shfl_xor(best, o, 64));
+    return best;
 }
 
 __device__ double polygons_dist_f64(const Polys& A, int64_t ra, const Polys& B, int64_t rb) {
@@ -227,9 +232,9 @@ __global__ __launch_bounds__(256) void pair_distances_wave_kernel(int left_kind,
         const int64_t i = heavy[w];
         const int64_t l = left[i], r = right[i];
         const double c = cap && cap[l] == cap[l] ? cap[l] : INFINITY;  // NaN: no cap
-        const double d = left_kind == 0 ? wave_point_polygon_dist_f64(L.x[l], L.y[l], R, r,
+        const double d = left_kind == 0 ? lanes_point_polygon_dist_f64<64>(L.x[l], L.y[l], R, r,
                                                                       (flags & kDistOutside) != 0, c, lane)
-                                        : wave_point_polygon_dist_f64(R.x[r], R.y[r], L, l, false, c, lane);
+                                        : lanes_point_polygon_dist_f64<64>(R.x[r], R.y[r], L, l, false, c, lane);
         if (lane == 0) out[i] = d > c ? INFINITY : d;
     }
 }
@@ -450,10 +455,16 @@ struct NearestTree {
 // kBoundPops nodes.  A full stack or the visit limit only drops nodes, which
 // leaves a valid (looser) bound.  +inf when no
 // finite box is met; scaled up by 2^-40 for the rounding of the fp64 values.
+//
+// Sixteen lanes take a query: they test a node's children (the tree's fanout)
+// in one step and measure an item together, and the four queries of a wave
+// wait for the slowest of four instead of 64.  With a lane to a query the
+// launch ran on with 1.6 waves a SIMD behind the queries of the longest walks
+// and widest rows (392,000 points, 100,000 polygons: 1490 us, now 1000).
+constexpr int kBoundLanes = 16;
 constexpr int kBoundStack = 256;
 constexpr int kBoundPops = 4096;  // visit limit per query (bounds the time of a pathological query)
 constexpr int kBoundExact = 2;    // exact item distances per query
-constexpr int kBoundWide = 16;    // up to this many lanes' wide rows are measured by the whole wave, one by one
 
 __device__ __forceinline__ double box_gap2(const double4 q, const double4 b) {
     const double gx = fmax(0.0, fmax(b.x - q.z, q.x - b.z));
@@ -461,100 +472,160 @@ __device__ __forceinline__ double box_gap2(const double4 q, const double4 b) {
     return gx * gx + gy * gy;
 }
 
-//
-// The wave's lanes walk until each holds an item to measure (or is done), and
-// measure together: one by one they would each hold up the other 63 for a
-// whole polygon.  Rows of more than kWaveRowCoords coordinates are measured by
-// the whole wave, one after the other.
-__device__ double nearest_upper_bound(const double4 q, const NearestTree& T, bool live, int lane) {
-    int64_t stack[kBoundStack];
-    int sp = 0;
+// The least of the 16 lanes' values: rotations within a row of 16 lanes (all
+// active), without the LDS crossbar.
+template <int n>
+__device__ __forceinline__ int row_rotate(int v) {
+    return __builtin_amdgcn_update_dpp(v, v, 0x120 + n, 0xf, 0xf, false);
+}
+
+template <int n>
+__device__ __forceinline__ uint32_t rotated(uint32_t v) {
+    return (uint32_t)row_rotate<n>((int)v);
+}
+
+template <int n>
+__device__ __forceinline__ double rotated(double v) {
+    return __hiloint2double(row_rotate<n>(__double2hiint(v)), row_rotate<n>(__double2loint(v)));
+}
+
+__device__ __forceinline__ uint32_t least(uint32_t a, uint32_t b) { return min(a, b); }
+__device__ __forceinline__ double least(double a, double b) { return fmin(a, b); }
+
+template <class V>
+__device__ __forceinline__ V lanes16_min(V v) {
+    v = least(v, rotated<8>(v));
+    v = least(v, rotated<4>(v));
+    v = least(v, rotated<2>(v));
+    return least(v, rotated<1>(v));
+}
+
+// A query's open nodes: the index in the level, the level, and box_gap2
+// rounded down to fp32 (a node is never dropped for a gap it does not have).
+struct BoundStack {
+    uint32_t node[kBoundStack];
+    float gap[kBoundStack];
+    uint8_t level[kBoundStack];
+};
+
+// The tree's levels, indexed by lanes: kept in LDS, a kernel argument so
+// indexed goes to scratch memory.
+struct BoundLevels {
+    int64_t start[VS_MAX_LEVELS];
+    int64_t count[VS_MAX_LEVELS];
+};
+
+__device__ double nearest_upper_bound(const double4 q, const NearestTree& T, const BoundLevels& V, BoundStack& S,
+                                      int lane) {
+    const int sub = lane & (kBoundLanes - 1);
+    const int first = lane - sub;  // of the query's lanes
+    const uint64_t below = (1ull << lane) - 1, mine = 0xffffull << first;
     const int last = T.n_levels - 1;
-    for (int64_t c = 0; live && c < T.level_count[0] && sp < kBoundStack; ++c) stack[sp++] = c;  // level 0
     double ub2 = INFINITY;
     int exact = (T.polys && q.x == q.z && q.y == q.w) ? kBoundExact : 0;
-    int pops = 0;
-    for (;;) {
-        int32_t item = -1;  // row to measure
-        for (; sp > 0 && pops < kBoundPops && item < 0; ++pops) {
-            const int64_t e = stack[--sp];
-            const int l = (int)(e >> 48);
-            const int64_t c = e & ((1ll << 48) - 1);
-            const double4 b = T.box[T.level_start[l] + c];
-            if (!(b.x == b.x) || box_gap2(q, b) > ub2) continue;
+    int sp = 0;
+    int l = 0;  // the children [lo, hi) of level l
+    int64_t lo = 0, hi = V.count[0];
+    // every value that steers the walk is the same on the query's 16 lanes
+    for (int pops = 0;; ++pops) {
+        for (int64_t k0 = lo; k0 < hi; k0 += kBoundLanes) {
+            const int64_t k = k0 + sub;
+            const bool have = k < hi;
+            const double4 b = T.box[V.start[l] + (have ? k : hi - 1)];
+            double gap = INFINITY;
+            if (have && b.x == b.x) gap = box_gap2(q, b);
             if (l == last) {
-                // farthest point of the query box from the item box, and from a
-                // point of the item itself (never farther, often much nearer)
-                const double dx = fmax(q.z - b.x, b.z - q.x), dy = fmax(q.w - b.y, b.w - q.y);
-                ub2 = fmin(ub2, dx * dx + dy * dy);
-                const double2 p = T.rep[c];
-                if (p.x == p.x) {
-                    const double ex = fmax(fabs(p.x - q.x), fabs(p.x - q.z)), ey = fmax(fabs(p.y - q.y), fabs(p.y - q.w));
-                    ub2 = fmin(ub2, ex * ex + ey * ey);
+                double near2 = INFINITY;
+                if (gap <= ub2 && have && b.x == b.x) {
+                    // farthest point of the query box from the item box, and from a
+                    // point of the item itself (never farther, often much nearer)
+                    const double dx = fmax(q.z - b.x, b.z - q.x), dy = fmax(q.w - b.y, b.w - q.y);
+                    near2 = dx * dx + dy * dy;
+                    const double2 p = T.rep[k];
+                    if (p.x == p.x) {
+                        const double ex = fmax(fabs(p.x - q.x), fabs(p.x - q.z)),
+                                     ey = fmax(fabs(p.y - q.y), fabs(p.y - q.w));
+                        near2 = fmin(near2, ex * ex + ey * ey);
+                    }
                 }
-                if (exact > 0) {
+                ub2 = fmin(ub2, lanes16_min(near2));
+                while (exact > 0) {
+                    const double g = lanes16_min(gap);
+                    if (!(g <= ub2) || !(g < INFINITY)) break;
+                    const int j = __ffsll((unsigned long long)(__ballot(gap == g) & mine)) - 1;  // the nearest box
                     --exact;
-                    item = T.item_ids[c];
+                    // at most the box bound just taken up to rounding; +inf
+                    // (rounding, empty row) leaves the bound as it is
+                    const double d = lanes_point_polygon_dist_f64<kBoundLanes>(
+                        q.x, q.y, T.P, T.item_ids[k0 + (j - first)], false, sqrt(ub2), lane);
+                    if (d < INFINITY) ub2 = fmin(ub2, d * d);
+                    if (lane == j) gap = INFINITY;
                 }
                 continue;
             }
-            const int64_t lo = c * T.fanout;
-            const int64_t hi = lo + T.fanout < T.level_count[l + 1] ? lo + T.fanout : T.level_count[l + 1];
             // push the children within the bound, the nearest one last (popped first)
-            int64_t best = -1;
-            double bestd = INFINITY;
-            for (int64_t k0 = lo; k0 < hi; k0 += 4) {
-                double4 cb[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) cb[u] = T.box[T.level_start[l + 1] + (k0 + u < hi ? k0 + u : hi - 1)];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const int64_t k = k0 + u;
-                    if (k >= hi || !(cb[u].x == cb[u].x)) continue;
-                    const double g = box_gap2(q, cb[u]);
-                    if (g > ub2) continue;
-                    if (g < bestd) {
-                        if (best >= 0 && sp < kBoundStack) stack[sp++] = ((int64_t)(l + 1) << 48) | best;
-                        best = k;
-                        bestd = g;
-                    } else if (sp < kBoundStack) {
-                        stack[sp++] = ((int64_t)(l + 1) << 48) | k;
-                    }
-                }
+            const float g32 = __double2float_rd(gap);
+            const uint32_t key = (__float_as_uint(g32) & ~15u) | (uint32_t)sub;  // gaps are not negative
+            const bool open = gap <= ub2 && gap < INFINITY;
+            const uint64_t m = __ballot(open) & mine;
+            const uint32_t nearest = lanes16_min(open ? key : ~0u);
+            if (m == 0) continue;
+            const int n = __popcll(m), at_last = first + (int)(nearest & 15u);
+            int slot = sp + __popcll(m & below) - (lane > at_last ? 1 : 0);
+            if (lane == at_last) slot = min(sp + n, kBoundStack) - 1;
+            const bool fits = lane == at_last || slot < min(sp + n, kBoundStack) - 1;
+            if (open && fits) {
+                S.node[slot] = (uint32_t)k;
+                S.gap[slot] = g32;
+                S.level[slot] = (uint8_t)l;
             }
-            if (best >= 0 && sp < kBoundStack) stack[sp++] = ((int64_t)(l + 1) << 48) | best;
+            sp = min(sp + n, kBoundStack);
         }
-        if (__ballot(item >= 0) == 0) break;
-        // a distance is at most the box bound just taken up to rounding; +inf
-        // (rounding, empty row) leaves the bound as it is
-        bool wide = item >= 0 && row_coords(T.P, item) > kWaveRowCoords;
-        if (__popcll(__ballot(wide)) > kBoundWide) wide = false;
-        double d = INFINITY;
-        if (item >= 0 && !wide) d = point_polygon_dist_f64(q.x, q.y, T.P, item, false, sqrt(ub2));
-        for (uint64_t m = __ballot(wide); m; m &= m - 1) {
-            const int j = __ffsll((unsigned long long)m) - 1;
-            const double dj = wave_point_polygon_dist_f64(__shfl(q.x, j), __shfl(q.y, j), T.P, __shfl(item, j), false,
-                                                          sqrt(__shfl(ub2, j)), lane);
-            if (lane == j) d = dj;
+        if (pops >= kBoundPops) break;
+        wave_lds_order();
+        bool found = false;
+        uint32_t c = 0;
+        while (sp > 0 && !found) {
+            --sp;
+            found = (double)S.gap[sp] <= ub2;
+            if (found) {
+                c = S.node[sp];
+                l = S.level[sp];
+            }
         }
-        if (d < INFINITY) ub2 = fmin(ub2, d * d);
+        wave_lds_order();
+        if (!found) break;
+        lo = (int64_t)c * T.fanout;
+        ++l;
+        hi = lo + T.fanout < V.count[l] ? lo + T.fanout : V.count[l];
     }
     return sqrt(ub2) * (1.0 + 0x1p-40);
 }
 
 // radius[q] = min(bound, cap) for each listed query row q (search follows);
 // a query without a finite bound keeps its radius.
-// Threads take the rows in the Hilbert order of their boxes (perm), so the
+// Queries are taken in the Hilbert order of their boxes (perm), so the
 // lanes of a wave walk nearby parts of the tree.
 __global__ __launch_bounds__(256) void nearest_bound_kernel(const double4* __restrict__ qboxes,
                                                            const int64_t* __restrict__ rows,
                                                            const int32_t* __restrict__ perm, int64_t m,
                                                            NearestTree T, double cap, double* __restrict__ radius,
                                                            double* __restrict__ search) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int64_t q = rows[perm[i < m ? i : m - 1]];
-    const double ub = nearest_upper_bound(qboxes[q], T, i < m, threadIdx.x & 63);  // whole waves
-    if (i < m && ub < INFINITY) {
+    __shared__ BoundStack stacks[256 / kBoundLanes];
+    __shared__ BoundLevels levels;
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int l = 0; l < VS_MAX_LEVELS; ++l) {
+            levels.start[l] = T.level_start[l];
+            levels.count[l] = T.level_count[l];
+        }
+    }
+    __syncthreads();
+    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) / kBoundLanes;
+    if (i >= m) return;
+    const int64_t q = rows[perm[i]];
+    const double ub = nearest_upper_bound(qboxes[q], T, levels, stacks[threadIdx.x / kBoundLanes], threadIdx.x & 63);
+    if (ub < INFINITY && threadIdx.x % kBoundLanes == 0) {
         const double r = fmin(ub, cap);
         radius[q] = r;
         search[q] = r * kSearchSlack;
@@ -802,7 +873,8 @@ int vs_nearest_bound(const double* query_boxes, const int64_t* rows, int64_t n_r
         T.level_start[l] = layout->level_start[l];
         T.level_count[l] = layout->level_count[l];
     }
-    hipLaunchKernelGGL(vs::nearest_bound_kernel, dim3((unsigned)vs::ceil_div(n_rows, 256)), dim3(256), 0, s,
+    hipLaunchKernelGGL(vs::nearest_bound_kernel, dim3((unsigned)vs::ceil_div(n_rows, 256 / vs::kBoundLanes)),
+                       dim3(256), 0, s,
                        reinterpret_cast<const double4*>(query_boxes), rows, perm, n_rows, T, cap, radius, search);
     VS_LAUNCH_CHECK();
     return VS_OK;

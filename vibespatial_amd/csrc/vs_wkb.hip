@@ -11,19 +11,20 @@
 // records with bytes after their geometry.  A zero-length record or a cleared
 // validity byte is a null row.
 //
-// Rows are processed in tiles of kWkbTile = 4096 records (256 threads x 16
-// rows, row = tile * 4096 + j * 256 + thread, so the loads of offsets and
-// record heads are coalesced).  No per-row arrays are kept: the rows pass
+// Rows are processed in tiles of kWkbTile = 1024 records (4 waves x 4 x 64
+// rows, row = tile * 1024 + wave * 256 + j * 64 + lane, so the loads of offsets
+// and record heads are coalesced and a wave's rows are consecutive).  No per-row arrays are kept: the rows pass
 // re-derives each row's counts from its record head, which costs about what
 // reading a stored count would.
 //   count  per row: kind and the part / ring / coordinate counts (record head
 //          and ring headers only, bounds-checked against the record's
-//          bytes); per tile: the five column sums.  The first bad record and
+//          bytes); per tile: the five column sums, and their prefixes at each
+//          of its waves.  The first bad record and
 //          its error go to the status word (atomic min of row << 8 | code).
 //   tiles  one block: exclusive prefixes of the tile sums, the column totals
 //          and the result words.
-//   rows   per tile: counts again, block prefix over the tile + tile prefix
-//          = each row's point index / polygon index / part / ring /
+//   rows   per wave: counts again, prefix over the wave's rows + wave and tile
+//          prefix = each row's point index / polygon index / part / ring /
 //          coordinate base; point rows write x, y and their record number,
 //          polygonal rows their record number, geometry offset and first part
 //          and ring offsets.
@@ -38,8 +39,13 @@ enum { kWkbOk = 0, kWkbTruncated = 1, kWkbType = 2, kWkbByteOrder = 3, kWkbMembe
 enum { kKindNull = 0, kKindPoint = 1, kKindPoly = 2 };
 
 constexpr int kWkbThreads = 256;
-constexpr int kWkbRowsPerThread = 16;
+// Few rows a thread: records of polygons are walked header by header, and a
+// column that ends in 100,000 of them kept a handful of blocks busy alone (10M
+// points first; rows a thread 16 / 8 / 4: count 156 / 120 / 102 us, rows 210 /
+// 164 / 126, the prefix over the tiles 14 / 23 / 44).
+constexpr int kWkbRowsPerThread = 4;
 constexpr int kWkbTile = kWkbThreads * kWkbRowsPerThread;
+constexpr int kWkbWaves = kWkbThreads / 64;
 constexpr int kWkbCols = 5;  // point rows, polygonal rows, parts, rings, coordinates
 constexpr int kWkbPolyThreads = 256;
 constexpr int64_t kWkbPolyWaves = 32768;  // grid of the polys pass (grid-stride)
@@ -107,6 +113,46 @@ __device__ int64_t skip_polygon_body(WkbCursor& c, int64_t& coords) {
     }
     coords += nc;
     return nr;
+}
+
+// Records of 21 bytes that hold a point, kWkbAhead rows (64 apart) at a time:
+// their heads are read side by side, where the general walk of one record
+// after the other waits for offset, head and coordinates in turn.
+constexpr int kWkbAhead = 4;
+
+struct WkbPoints {
+    int64_t b0[kWkbAhead];
+    bool point[kWkbAhead], le[kWkbAhead];
+};
+
+__device__ __forceinline__ WkbPoints point_records(const uint8_t* __restrict__ data, int64_t data_bytes,
+                                                   const int64_t* __restrict__ off,
+                                                   const uint8_t* __restrict__ valid, int64_t row0, int64_t n) {
+    WkbPoints H;
+    uint8_t order[kWkbAhead];
+    uint32_t type[kWkbAhead];
+#pragma unroll
+    for (int u = 0; u < kWkbAhead; ++u) {
+        const int64_t row = row0 + 64 * u < n ? row0 + 64 * u : n - 1;
+        const int64_t b1 = off[row + 1];
+        H.b0[u] = off[row];
+        H.point[u] = row0 + 64 * u < n && b1 >= 21 && b1 <= data_bytes && H.b0[u] == b1 - 21 && (!valid || valid[row]);
+    }
+#pragma unroll
+    for (int u = 0; u < kWkbAhead; ++u) {
+        order[u] = 2;
+        type[u] = 0;
+        if (H.point[u]) {
+            order[u] = data[H.b0[u]];
+            __builtin_memcpy(&type[u], data + H.b0[u] + 1, 4);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < kWkbAhead; ++u) {
+        H.le[u] = order[u] == 1;
+        H.point[u] = (order[u] == 1 && type[u] == 1u) || (order[u] == 0 && type[u] == 0x01000000u);
+    }
+    return H;
 }
 
 struct WkbRow {
@@ -228,6 +274,7 @@ __device__ __forceinline__ bool totals_overflow(const long long* totals) {
 
 struct WkbWs {
     long long* tile;    // [kWkbCols][n_tiles]: column sums per tile, then their exclusive prefixes
+    long long* wave;    // [kWkbCols][n_tiles][waves]: exclusive prefixes in the tile at each wave
     long long* totals;  // [0] point rows [1] polygonal rows [2] parts [3] rings [4] coordinates
     unsigned long long* status;
     int64_t n_tiles;
@@ -237,6 +284,7 @@ static WkbWs carve_wkb(Carver& c, int64_t n) {
     WkbWs W;
     W.n_tiles = ceil_div(n, kWkbTile);
     W.tile = c.take<long long>(kWkbCols * W.n_tiles);
+    W.wave = c.take<long long>(kWkbCols * W.n_tiles * kWkbWaves);
     W.totals = c.take<long long>(8);
     W.status = c.take<unsigned long long>(1);
     return W;
@@ -253,22 +301,36 @@ __global__ __launch_bounds__(kWkbThreads) void wkb_count_kernel(const uint8_t* _
                                                                const uint8_t* __restrict__ valid, int64_t n,
                                                                WkbWs W) {
     __shared__ long long red[kWkbCols * (kWkbThreads / 64)];
-    const int64_t base = (int64_t)blockIdx.x * kWkbTile + threadIdx.x;
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int64_t base = (int64_t)blockIdx.x * kWkbTile + w * (kWkbTile / kWkbWaves) + lane;
     long long sum[kWkbCols] = {0, 0, 0, 0, 0};
     int64_t bad = -1;
     int bad_code = 0;
-    for (int j = 0; j < kWkbRowsPerThread; ++j) {
-        const int64_t row = base + (int64_t)j * kWkbThreads;
-        if (row >= n) break;
-        const WkbRow R = wkb_row(data, data_bytes, off, valid, row);
-        if (R.err != kWkbOk && bad < 0) {
-            bad = row;
-            bad_code = R.err;
-        }
-        long long v[kWkbCols];
-        row_columns(R, v);
+    for (int j0 = 0; j0 < kWkbRowsPerThread; j0 += kWkbAhead) {
+        const int64_t row0 = base + (int64_t)j0 * 64;
+        if (row0 >= n) break;
+        const WkbPoints H = point_records(data, data_bytes, off, valid, row0, n);
+#pragma unroll 1
+        for (int u = 0; u < kWkbAhead; ++u) {
+            const int64_t row = row0 + 64 * u;
+            bool point = false;
 #pragma unroll
-        for (int k = 0; k < kWkbCols; ++k) sum[k] += v[k];
+            for (int q = 0; q < kWkbAhead; ++q) point = q == u ? H.point[q] : point;
+            if (point) {
+                ++sum[0];
+                continue;
+            }
+            if (row >= n) break;
+            const WkbRow R = wkb_row(data, data_bytes, off, valid, row);
+            if (R.err != kWkbOk && bad < 0) {
+                bad = row;
+                bad_code = R.err;
+            }
+            long long v[kWkbCols];
+            row_columns(R, v);
+#pragma unroll
+            for (int k = 0; k < kWkbCols; ++k) sum[k] += v[k];
+        }
     }
     if (bad >= 0) report(W.status, bad, bad_code);
     long long tot[kWkbCols];
@@ -276,6 +338,10 @@ __global__ __launch_bounds__(kWkbThreads) void wkb_count_kernel(const uint8_t* _
     if (threadIdx.x == 0) {
 #pragma unroll
         for (int k = 0; k < kWkbCols; ++k) W.tile[k * W.n_tiles + blockIdx.x] = tot[k];
+    }
+    if (lane == 0) {
+#pragma unroll
+        for (int k = 0; k < kWkbCols; ++k) W.wave[(k * W.n_tiles + blockIdx.x) * kWkbWaves + w] = sum[k];
     }
 }
 
@@ -328,42 +394,75 @@ __global__ __launch_bounds__(1024) void wkb_tiles_kernel(WkbWs W, int64_t* __res
     }
 }
 
+// A wave finds its rows' places with ballots; only a wave that holds a polygonal
+// row scans the part, ring and coordinate columns.  (Block scans of five 64-bit
+// columns for every 256 rows, one record's loads after the other: 10M points
+// and 100,000 polygons, 281 us, now 126; the count pass 149 us, now 102.)
 __global__ __launch_bounds__(kWkbThreads) void wkb_fill_rows_kernel(
-    const uint8_t* __restrict__ data, int64_t data_bytes, const int64_t* __restrict__ off, const uint8_t* __restrict__ valid, int64_t n,
-    WkbWs W, double* __restrict__ px, double* __restrict__ py, int64_t* __restrict__ point_rows,
-    int32_t* __restrict__ geom_offsets, int32_t* __restrict__ part_offsets, int32_t* __restrict__ ring_offsets,
-    int64_t* __restrict__ polygon_rows) {
-    __shared__ long long lds[kWkbCols * (kWkbThreads / 64)];
+    const uint8_t* __restrict__ data, int64_t data_bytes, const int64_t* __restrict__ off,
+    const uint8_t* __restrict__ valid, int64_t n, WkbWs W, double* __restrict__ px, double* __restrict__ py,
+    int64_t* __restrict__ point_rows, int32_t* __restrict__ geom_offsets, int32_t* __restrict__ part_offsets,
+    int32_t* __restrict__ ring_offsets, int64_t* __restrict__ polygon_rows) {
     if (totals_overflow(W.totals)) return;  // the same in every block
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const uint64_t below = (1ull << lane) - 1;
     long long run[kWkbCols];
 #pragma unroll
-    for (int k = 0; k < kWkbCols; ++k) run[k] = W.tile[k * W.n_tiles + blockIdx.x];
-    const int64_t tile0 = (int64_t)blockIdx.x * kWkbTile;
-    for (int j = 0; j < kWkbRowsPerThread; ++j) {
-        if (tile0 + (int64_t)j * kWkbThreads >= n) break;  // the same in every thread of the block
-        const int64_t row = tile0 + (int64_t)j * kWkbThreads + threadIdx.x;
-        WkbRow R = {kKindNull, kWkbOk, 0, 0, 0, 0, true};
-        if (row < n) R = wkb_row(data, data_bytes, off, valid, row);
-        long long v[kWkbCols], tot[kWkbCols];
-        row_columns(R, v);
-        block_scan_cols(v, lds, tot);
-        if (R.kind == kKindPoint) {
-            const long long i = run[0] + v[0];
-            double x, y;
-            read_xy(data, R.xy_pos, R.le, x, y);
-            px[i] = x;
-            py[i] = y;
-            point_rows[i] = row;
-        } else if (R.kind == kKindPoly) {
-            const long long g = run[1] + v[1];
-            const long long part = run[2] + v[2], ring = run[3] + v[3], coord = run[4] + v[4];
-            polygon_rows[g] = row;
-            geom_offsets[g] = (int32_t)part;
-            if (R.parts > 0) part_offsets[part] = (int32_t)ring;
-            if (R.rings > 0) ring_offsets[ring] = (int32_t)coord;
-        }
+    for (int k = 0; k < kWkbCols; ++k)
+        run[k] = W.tile[k * W.n_tiles + blockIdx.x] + W.wave[(k * W.n_tiles + blockIdx.x) * kWkbWaves + w];
+    const int64_t wave0 = (int64_t)blockIdx.x * kWkbTile + w * (kWkbTile / kWkbWaves);
+    for (int j0 = 0; j0 < kWkbRowsPerThread; j0 += kWkbAhead) {
+        if (wave0 + (int64_t)j0 * 64 >= n) break;  // the same in every lane
+        const int64_t row0 = wave0 + (int64_t)j0 * 64 + lane;
+        const WkbPoints H = point_records(data, data_bytes, off, valid, row0, n);
+        double hx[kWkbAhead], hy[kWkbAhead];
 #pragma unroll
-        for (int k = 0; k < kWkbCols; ++k) run[k] += tot[k];
+        for (int u = 0; u < kWkbAhead; ++u) {
+            hx[u] = hy[u] = 0.0;
+            if (H.point[u]) read_xy(data, H.b0[u] + 5, H.le[u], hx[u], hy[u]);
+        }
+#pragma unroll 1
+        for (int u = 0; u < kWkbAhead; ++u) {
+            const int64_t row = row0 + 64 * u;
+            WkbRow R = {kKindNull, kWkbOk, 0, 0, 0, 0, true};
+            double x = 0.0, y = 0.0;
+            bool point = false;
+#pragma unroll
+            for (int q = 0; q < kWkbAhead; ++q) {
+                point = q == u ? H.point[q] : point;
+                x = q == u ? hx[q] : x;
+                y = q == u ? hy[q] : y;
+            }
+            if (point) {
+                R.kind = kKindPoint;
+            } else if (row < n) {
+                R = wkb_row(data, data_bytes, off, valid, row);
+                if (R.kind == kKindPoint) read_xy(data, R.xy_pos, R.le, x, y);
+            }
+            const uint64_t points = __ballot(R.kind == kKindPoint), polys = __ballot(R.kind == kKindPoly);
+            if (R.kind == kKindPoint) {
+                const long long i = run[0] + __popcll(points & below);
+                px[i] = x;
+                py[i] = y;
+                point_rows[i] = row;
+            }
+            run[0] += __popcll(points);
+            if (polys == 0) continue;
+            const long long part_end = wave_inclusive_scan_i64(R.parts), ring_end = wave_inclusive_scan_i64(R.rings),
+                            coord_end = wave_inclusive_scan_i64(R.coords);
+            if (R.kind == kKindPoly) {
+                const long long g = run[1] + __popcll(polys & below);
+                const long long part = run[2] + part_end - R.parts, ring = run[3] + ring_end - R.rings;
+                polygon_rows[g] = row;
+                geom_offsets[g] = (int32_t)part;
+                if (R.parts > 0) part_offsets[part] = (int32_t)ring;
+                if (R.rings > 0) ring_offsets[ring] = (int32_t)(run[4] + coord_end - R.coords);
+            }
+            run[1] += __popcll(polys);
+            run[2] += __shfl(part_end, 63);
+            run[3] += __shfl(ring_end, 63);
+            run[4] += __shfl(coord_end, 63);
+        }
     }
 }
 

@@ -633,6 +633,13 @@ int vs_host_point_point_within(double px, double py, double qx, double qy, doubl
  * NaN / infinity rules.  The device decision for a point and one edge. */
 int vs_host_point_segment_within(double px, double py, double ax, double ay, double bx, double by, double d);
 
+/* Relation of row a of A and row b of B (polygonal rows, host pointers), as
+ * bits: 1 the interiors meet, 2 a lies in b, 4 b lies in a, 8 the boundaries
+ * meet.  The device's full relation (vs_refine_pairs mode 1). */
+int vs_host_polygon_relation(const double* ax, const double* ay, const int32_t* a_geom, const int32_t* a_part,
+                             const int32_t* a_ring, int64_t a, const double* bx, const double* by,
+                             const int32_t* b_geom, const int32_t* b_part, const int32_t* b_ring, int64_t b);
+
 /* 64-bit Hilbert index of 32-bit grid coordinates. */
 uint64_t vs_host_hilbert64(uint32_t x, uint32_t y);
 

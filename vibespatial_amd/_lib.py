@@ -157,6 +157,7 @@ SIGNATURES = {
     "vs_host_segments_touch": (ctypes.c_int, [_d] * 8),
     "vs_host_point_point_within": (ctypes.c_int, [_d] * 5),
     "vs_host_point_segment_within": (ctypes.c_int, [_d] * 7),
+    "vs_host_polygon_relation": (ctypes.c_int, [_p, _p, _p, _p, _p, _i64, _p, _p, _p, _p, _p, _i64]),
     "vs_host_hilbert64": (_u64, [_u32, _u32]),
     "vs_host_cover_ranges": (ctypes.c_int, [_d, _d, _d, _d, _p, _i32, _p]),
     "vs_host_cell_grid": (ctypes.c_int, [_p, _p, _i64, _p, _p, _p]),

@@ -473,4 +473,12 @@ int vs_lexsort_pairs(int64_t* left, int64_t* right, int64_t n_pairs, void* works
     return VS_OK;
 }
 
+int vs_host_polygon_relation(const double* ax, const double* ay, const int32_t* a_geom, const int32_t* a_part,
+                             const int32_t* a_ring, int64_t a, const double* bx, const double* by,
+                             const int32_t* b_geom, const int32_t* b_part, const int32_t* b_ring, int64_t b) {
+    const vs::Polys A = {ax, ay, a_geom, a_part, a_ring}, B = {bx, by, b_geom, b_part, b_ring};
+    const vs::Relation R = vs::relate_polygons(A, a, B, b);
+    return (R.interiors_meet ? 1 : 0) | (R.a_in_b ? 2 : 0) | (R.b_in_a ? 4 : 0) | (R.touch ? 8 : 0);
+}
+
 }  // extern "C"

@@ -145,12 +145,14 @@ struct RelSide {
     bool all_in;    // every part of X shows a piece inside Y or a same-side shared piece
 };
 
-// The next vertex of Y strictly between cur and b on edge (a, b) (nearest to
-// cur), or b.  `ax_major`: compare along x (else y).
-VS_HD void next_cut(double ax, double ay, double bx, double by, double cx, double cy, const Polys& Y, int64_t ry,
+// (nx, ny) = the next vertex of Y strictly between cur and b on edge (a, b)
+// (nearest to cur; returns true), or b (returns false).  `ax_major`: compare
+// along x (else y).
+VS_HD bool next_cut(double ax, double ay, double bx, double by, double cx, double cy, const Polys& Y, int64_t ry,
                     bool ax_major, double& nx, double& ny) {
     nx = bx;
     ny = by;
+    bool cut = false;
     const bool inc = ax_major ? bx > ax : by > ay;
     const int32_t v0 = Y.ring[Y.part[Y.geom[ry]]], v1 = Y.ring[Y.part[Y.geom[ry + 1]]];
     for (int32_t v = v0; v < v1; ++v) {
@@ -162,7 +164,9 @@ VS_HD void next_cut(double ax, double ay, double bx, double by, double cx, doubl
         if (orient2d(ax, ay, bx, by, x, y) != 0) continue;
         nx = x;
         ny = y;
+        cut = true;
     }
+    return cut;
 }
 
 // One boundary edge c of X (ring interior on the left when left_x) against
@@ -184,12 +188,13 @@ VS_HD void relate_edge(const Polys& X, int32_t c, bool left_x, const Polys& Y, i
             const int o3 = orient2d(cx, cy, dx, dy, ax, ay), o4 = orient2d(cx, cy, dx, dy, bx, by);
             if (o3 * o4 < 0) S.cross = true;
         }
-    // pieces between consecutive cut points
+    // pieces between consecutive cut points; the last one ends where no cut is
+    // left, which also ends the walk along an edge to a NaN (equal to nothing)
     const bool ax_major = ax != bx;
     double px = ax, py = ay;
-    for (;;) {
+    for (bool more = true; more;) {
         double qx, qy;
-        next_cut(ax, ay, bx, by, px, py, Y, ry, ax_major, qx, qy);
+        more = next_cut(ax, ay, bx, by, px, py, Y, ry, ax_major, qx, qy);
         const int loc = mid_location(px, py, qx, qy, Y, ry);
         if (loc == 2) {
             S.in_int = true;
@@ -227,7 +232,6 @@ VS_HD void relate_edge(const Polys& X, int32_t c, bool left_x, const Polys& Y, i
                     break;
                 }
         }
-        if (qx == bx && qy == by) break;
         px = qx;
         py = qy;
     }
@@ -335,13 +339,6 @@ VS_HD int polygon_predicate_fast(int pred, const Polys& A, int64_t ra, const Pol
     if (!polygons_intersect_auto(A, ra, B, rb)) return 0;
     if (any_proper_crossing(A, ra, B, rb)) return pred == VS_PRED_OVERLAPS ? 1 : 0;
     return -1;
-}
-
-// predicate(A row, B row), one thread.
-VS_HD bool polygon_predicate(int pred, const Polys& A, int64_t ra, const Polys& B, int64_t rb) {
-    const int f = polygon_predicate_fast(pred, A, ra, B, rb);
-    if (f >= 0) return f != 0;
-    return relation_decides(pred, relate_polygons(A, ra, B, rb));
 }
 
 // ---------------------------------------------------------------------------

@@ -803,7 +803,8 @@ __device__ inline bool ring_intersects_listed(const RingRef& A, int32_t na, cons
     const double fx = A.X(0), fy = A.Y(0);
     int cnt = 0, parity = 0;
     auto touches = [&]() -> bool {  // segment tests over the listed edges; empties the list
-        int32_t e = c0b + (cnt > 0 ? (int32_t)near[0] : 1);
+        if (cnt == 0) return false;  // a ring of one coordinate has no edge to load
+        int32_t e = c0b + (int32_t)near[0];
         double px = bx[e - 1], py = by[e - 1], ex = bx[e], ey = by[e];
         for (int t = 0; t < cnt; ++t) {
             const double sx = px, sy = py, tx = ex, ty = ey;

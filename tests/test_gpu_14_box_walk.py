@@ -1,5 +1,6 @@
 """Box queries of few hits per box: units of 64 and of 16 boxes, unions split
-down to 4 boxes, every fanout's groups per step, the smallest trees."""
+down to 4 boxes, every fanout's groups per step, the smallest trees, and its
+stack at the fullest."""
 
 from __future__ import annotations
 
@@ -7,6 +8,7 @@ import numpy as np
 import pytest
 import torch
 
+from vibespatial_amd import _lib
 from vibespatial_amd import join as J
 
 pytestmark = pytest.mark.gpu
@@ -47,3 +49,48 @@ def test_sparse_and_dense_queries_match_bruteforce(n_q, n_t, fanout):
     for cap in (31 * n_q, max(4, len(el) // 2)):  # below the one-box shape; and a retry
         l, r, st = J.query_boxes(q, tree, capacity=cap)
         assert np.array_equal(l.cpu().numpy(), el[o]) and np.array_equal(r.cpu().numpy(), er[o])
+
+
+@pytest.mark.parametrize("n_t,fanout", [(32_768, 2), (177_147, 3), (262_144, 4), (100_000, 16), (300_000, 64)])
+def test_boxes_over_whole_deep_trees(n_t, fanout):
+    """Boxes that cover every item open every node: the walk's stack at its fullest."""
+    print(f"box walk over {n_t} items, fanout {fanout}", flush=True)
+    rng = np.random.default_rng(fanout)
+    tb = _boxes(rng, n_t, 1000.0, 1.0)
+    qb = np.tile([-1e4, -1e4, 1e4, 1e4], (18, 1))  # one unit of 16 boxes and one of 2
+    qb[3], qb[11] = [500.0, 500.0, 520.0, 520.0], np.nan
+    tree = J.build_tree(torch.from_numpy(tb).cuda(), fanout=fanout)
+    hit = (qb[:, None, 0] <= tb[:, 2]) & (qb[:, None, 2] >= tb[:, 0]) & (qb[:, None, 1] <= tb[:, 3]) & \
+        (qb[:, None, 3] >= tb[:, 1])
+    el, er = np.nonzero(hit)
+    # the walk counts every pair into too few slots, then the other shape writes them
+    l, r, st = J.query_boxes(torch.from_numpy(qb).cuda(), tree, capacity=31 * 18)
+    assert st.retries == 1 and st.staged == len(el)
+    assert np.array_equal(l.cpu().numpy(), el) and np.array_equal(r.cpu().numpy(), er)
+
+
+def test_layout_too_deep_for_the_walk_takes_the_other_shape():
+    """16 levels of fanout 32, 619 nodes staged: more entries than the walk's
+    stack is sized for; the pairs are those of a plain search."""
+    print("box walk, layout too deep", flush=True)
+    rng = np.random.default_rng(5)
+    counts = [1, 20, 619] + [700] * 13
+    tb = _boxes(rng, 700, 1000.0, 30.0)
+    qb = _boxes(rng, 90, 1000.0, 60.0)
+    layout = _lib.TreeLayout(fanout=32, n_levels=16, n_items=700, n_nodes=sum(counts))
+    boxes = []
+    for k, c in enumerate(counts):
+        layout.level_start[k] = sum(counts[:k])
+        layout.level_count[k] = c
+        b = np.full((c, 4), np.nan)
+        below = counts[k + 1] if k < 15 else 0
+        b[: -(-below // 32)] = [-100.0, -100.0, 1100.0, 1100.0]  # the nodes that have children
+        boxes.append(tb if k == 15 else b)
+    dev = torch.device("cuda")
+    tree = J.DeviceTree(layout, torch.from_numpy(np.concatenate(boxes)).to(dev),
+                        torch.arange(700, dtype=torch.int32, device=dev), None, None)
+    hit = (qb[:, None, 0] <= tb[:, 2]) & (qb[:, None, 2] >= tb[:, 0]) & (qb[:, None, 1] <= tb[:, 3]) & \
+        (qb[:, None, 3] >= tb[:, 1])
+    el, er = np.nonzero(hit)
+    l, r, _ = J.query_boxes(torch.from_numpy(qb).to(dev), tree, capacity=31 * 90)
+    assert np.array_equal(l.cpu().numpy(), el) and np.array_equal(r.cpu().numpy(), er) and len(el) < 31 * 90

@@ -363,7 +363,7 @@ __global__ __launch_bounds__(kJoinThreads) void traverse_kernel(
 // 250 with the larger buffer.  72k scattered boxes of a nearest search: 1,410 ->
 // 144 us; 100k x 100k polygon boxes: 231 -> 58 us.
 // ---------------------------------------------------------------------------
-constexpr int kWalkStack = 1152;  // 640 staged nodes + at most 60 more entries per level below + one step's 64
+constexpr int kWalkStack = 1152;  // see walk_fits
 constexpr int kWalkSplit = 1024;
 constexpr int kWalkBlocks = 2;   // blocks per compute unit (LDS)
 
@@ -723,6 +723,22 @@ int launch_traverse(int pred, const double* qx, const double* qy, const double4*
     return VS_OK;
 }
 
+// The walk's stack cannot overflow.  Entries left by one step are followed on
+// the stack only by descendants of that step's entries, so the steps whose
+// entries are on it at one time have different least levels: at most one per
+// level below the staged one, and each kept what it pushed (groups x fanout at
+// most) less the `groups` the next step took.  Every layout of vs_tree_plan
+// fits (925 entries at the worst found); others take the one-box shape.
+bool walk_fits(const TreeView& T) {
+    const int64_t groups = 64 / T.fanout;
+    int staged = -1;
+    for (int l = 0; l + 1 < T.n_levels; ++l)
+        if (T.level_start[l] + T.level_count[l] <= T.n_top) staged = l;
+    const int64_t base = staged >= 0 ? T.level_count[staged] : 1;
+    const int64_t below = std::max(T.n_levels - 2 - staged, 0);
+    return base + below * groups * (T.fanout - 1) + groups <= kWalkStack;
+}
+
 int launch_box_walk(const double4* qbox, const int32_t* perm, int64_t n, const TreeView& T, const JoinWs& J,
                     int64_t capacity, hipStream_t s) {
     // units of 64 boxes once every wave of a full grid gets several of them
@@ -927,7 +943,7 @@ int vs_query_boxes(const double* query_boxes, int64_t n_queries, const vs_tree_l
         VS_TRY(vs::box_order(qb, n_queries, J.perm, J.order_ws, s));  // waves of nearby boxes
         // the traversal's shape follows the hits the caller expects per box
         // (capacity / n_queries); both shapes give the same pairs
-        if (capacity >= (int64_t)vs::kOneBoxHits * n_queries)
+        if (capacity >= (int64_t)vs::kOneBoxHits * n_queries || !vs::walk_fits(T))
             VS_TRY(vs::launch_traverse<vs::kModeBox>(VS_PRED_INTERSECTS, nullptr, nullptr, qb, J.perm, n_queries, T, P,
                                                      J, capacity, s));
         else

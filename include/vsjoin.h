@@ -352,20 +352,38 @@ int vs_learned_query_polygons(const void* index, int64_t n_points, int32_t key_b
                               int64_t* out_left, int64_t* out_right, int64_t* d_result, void* workspace,
                               int64_t workspace_bytes, void* stream);
 
-/* The two queries above in two steps, for callers that do not know how many
- * pairs to expect.  vs_learned_query_plan finds the rank ranges of every query
+/* The two queries above in steps, for callers that do not know how many pairs
+ * to expect.  vs_learned_query_plan finds the rank ranges of every query
  * (boxes n_queries x 4; for polygon queries also their offsets, else null) into
  * `plan` and writes d_positions[0] (device): the index positions the scan will
- * visit, an upper bound of the pairs.  vs_learned_query_run scans the planned
- * ranges with a capacity chosen from it: offsets null: a box query (x, y null,
- * n_parts / n_rings / n_coords 0), else polygon queries with `predicate` as for
- * vs_learned_query_polygons.  A plan holds for the same index, queries and
- * offsets and may be run again (with a larger capacity). */
+ * visit, an upper bound of the pairs.  vs_learned_query_scan scans the planned
+ * ranges into the stage (8 bytes a slot) of its workspace: offsets null: a box
+ * query (x, y null, n_parts / n_rings / n_coords 0), else polygon queries with
+ * `predicate` as for vs_learned_query_polygons; d_result int64[16] as for the
+ * learned join, d_result[1] above `capacity`: pairs were left out, scan again.
+ * vs_learned_query_finish turns the stage of scan_capacity slots into output of
+ * `capacity` slots, which need be no more than the pairs that were staged
+ * (more than `capacity`: nothing is written and the stage stays as it is);
+ * one finish that writes per scan.  vs_learned_query_run is a scan and a finish
+ * at one capacity.  A plan holds for the same index, queries and offsets and
+ * may be scanned again (with a larger capacity). */
 int64_t vs_learned_plan_bytes(int64_t n_queries);
 int vs_learned_query_plan(const void* index, int64_t n_points, int32_t key_bytes, int32_t n_leaves,
                           const double* boxes, const int32_t* geom_offsets, const int32_t* part_offsets,
                           const int32_t* ring_offsets, int64_t n_queries, int32_t lookup_mode, int64_t* d_positions,
                           void* plan, int64_t plan_bytes, void* stream);
+int64_t vs_learned_scan_workspace_bytes(int64_t n_coords, int64_t capacity);
+int vs_learned_query_scan(const void* index, int64_t n_points, int32_t key_bytes, int32_t n_leaves,
+                          const double* boxes, const double* x, const double* y, const int32_t* geom_offsets,
+                          const int32_t* part_offsets, const int32_t* ring_offsets, int64_t n_queries,
+                          int64_t n_parts, int64_t n_rings, int64_t n_coords, int32_t predicate, int64_t capacity,
+                          int64_t* d_result, void* plan, int64_t plan_bytes, void* workspace,
+                          int64_t workspace_bytes, void* stream);
+int64_t vs_learned_finish_workspace_bytes(int64_t capacity);
+int vs_learned_query_finish(int64_t n_points, int64_t n_queries, int64_t scan_capacity, int64_t capacity,
+                            int32_t sort, int64_t* out_left, int64_t* out_right, void* plan, int64_t plan_bytes,
+                            void* scan_workspace, int64_t scan_workspace_bytes, void* workspace,
+                            int64_t workspace_bytes, void* stream);
 int64_t vs_learned_run_workspace_bytes(int64_t n_coords, int64_t capacity);
 int vs_learned_query_run(const void* index, int64_t n_points, int32_t key_bytes, int32_t n_leaves,
                          const double* boxes, const double* x, const double* y, const int32_t* geom_offsets,

@@ -1,5 +1,6 @@
 """Index queries sized by their plan: one scan where the bound is allocated,
-two where it is not, and the empty query."""
+two where it is not, the empty query, output that is sized by the pairs and not
+by the scan, and the C entry that scans and finishes at one capacity."""
 
 from __future__ import annotations
 
@@ -8,9 +9,11 @@ import pytest
 import torch
 
 import oracle
+from vibespatial_amd import _lib
 from vibespatial_amd import join as J
 from vibespatial_amd import synthetic as S
-from vibespatial_amd.device import DevicePoints, DevicePolygons
+from vibespatial_amd.device import DevicePoints, DevicePolygons, ptr, stream
+from vibespatial_amd.geometry import Polygon, PolygonArray
 
 pytestmark = pytest.mark.gpu
 
@@ -39,3 +42,56 @@ def test_planned_queries_match_oracle(monkeypatch, limit, key_bytes):
     assert np.array_equal(l.cpu().numpy(), el[el != 5]) and np.array_equal(r.cpu().numpy(), er[el != 5])
     l, r, _ = idx.query_boxes(b[:0])
     assert l.numel() == 0 and r.numel() == 0
+
+
+def test_few_hits_of_a_long_scan_leave_little_allocated():
+    """Slivers across the map: their boxes hold most points, they hold few."""
+    rng = np.random.default_rng(4)
+    n, k = 400_000, 40
+    x, y = rng.uniform(0, 100, n), rng.uniform(0, 100, n)
+    a = rng.uniform(0, 20, (k, 2))
+    P = PolygonArray.from_geometries([Polygon([tuple(v), (v[0] + 80.0, v[1] + 80.0), (v[0] + 80.1, v[1] + 80.0)])
+                                      for v in a])
+    idx = J.LearnedPointIndex(DevicePoints(torch.from_numpy(x).cuda(), torch.from_numpy(y).cuda()))
+    D = DevicePolygons.from_host(P)
+    b = J.polygon_bounds(D)
+    el, er = oracle.sjoin_points_polygons(x, y, P, "within")
+    o = np.lexsort((el, er))
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    l, r, st = idx.query_polygons(D, b, "contains")
+    peak = torch.cuda.max_memory_allocated() - before
+    assert np.array_equal(l.cpu().numpy(), er[o]) and np.array_equal(r.cpu().numpy(), el[o])
+    assert st.retries == 0 and st.scanned > 100 * st.pairs > 0
+    assert l.untyped_storage().nbytes() == r.untyped_storage().nbytes() == 8 * len(el)
+    assert peak < 10 * st.scanned  # the stage's 8 bytes a position, plan and output beside it
+    l, r, st = idx.query_polygons(D, b, "touches")
+    assert l.numel() == 0 and r.numel() == 0 and st.pairs == 0
+
+
+@pytest.mark.parametrize("slots", [0, 1])
+def test_scan_and_finish_at_one_capacity(slots):
+    """vs_learned_query_run with room for the pairs, and with a slot too few."""
+    w = S.c1(n_points=20_000, n_polys=90)
+    idx = J.LearnedPointIndex(DevicePoints.from_host(w.points))
+    b = J.polygon_bounds(DevicePolygons.from_host(w.polygons))
+    el, er = oracle.box_query_points(w.points.x, w.points.y, b.cpu().numpy())
+    cap = len(el) - slots
+    L = _lib.lib()
+    nq = int(b.shape[0])
+    plan = torch.empty(L.vs_learned_plan_bytes(nq), dtype=torch.uint8, device="cuda")
+    ws = torch.empty(L.vs_learned_run_workspace_bytes(0, cap), dtype=torch.uint8, device="cuda")
+    pos, res = torch.zeros(1, dtype=torch.int64, device="cuda"), torch.zeros(16, dtype=torch.int64, device="cuda")
+    l, r = (torch.full((cap,), -1, dtype=torch.int64, device="cuda") for _ in range(2))
+    index = [ptr(idx.buf), idx.n, idx.key_bytes, idx.n_leaves, ptr(b)]
+    _lib.check(L.vs_learned_query_plan(*index, None, None, None, nq, 0, ptr(pos), ptr(plan), plan.numel(), stream()),
+               "plan")
+    _lib.check(L.vs_learned_query_run(*index, None, None, None, None, None, nq, 0, 0, 0, _lib.PRED["intersects"], cap, 1,
+                                      ptr(l), ptr(r), ptr(res), ptr(plan), plan.numel(), ptr(ws), ws.numel(),
+                                      stream()), "run")
+    assert int(res[1]) == len(el) <= int(pos)
+    if slots == 0:
+        assert np.array_equal(l.cpu().numpy(), el) and np.array_equal(r.cpu().numpy(), er)
+    else:
+        assert bool((l == -1).all()) and bool((r == -1).all())

@@ -111,6 +111,14 @@ SIGNATURES = {
     "vs_learned_plan_bytes": (_i64, [_i64]),
     "vs_learned_query_plan": (ctypes.c_int,
                               [_p, _i64, _i32, _i32, _p, _p, _p, _p, _i64, _i32, _p, _p, _i64, _p]),
+    "vs_learned_scan_workspace_bytes": (_i64, [_i64, _i64]),
+    "vs_learned_query_scan": (
+        ctypes.c_int,
+        [_p, _i64, _i32, _i32, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i32, _i64, _p, _p, _i64, _p, _i64, _p],
+    ),
+    "vs_learned_finish_workspace_bytes": (_i64, [_i64]),
+    "vs_learned_query_finish": (ctypes.c_int,
+                                [_i64, _i64, _i64, _i64, _i32, _p, _p, _p, _i64, _p, _i64, _p, _i64, _p]),
     "vs_learned_run_workspace_bytes": (_i64, [_i64, _i64]),
     "vs_learned_query_run": (
         ctypes.c_int,

@@ -40,32 +40,42 @@ constexpr int kRunTile = 4096;  // int32 elements sorted in LDS by one block (16
 constexpr int kRunThreads = 256;
 
 struct FinishBufs {
-    uint32_t* stage_l;
-    int32_t* stage_r;
     void* sort_ws;
     int32_t* long_runs;
 };
 
 static FinishBufs carve_finish(Carver& c, int64_t capacity) {
     FinishBufs F;
-    F.stage_l = c.take<uint32_t>(capacity);
-    F.stage_r = c.take<int32_t>(capacity);
     F.sort_ws = c.take<char>(sort_workspace_bytes_u32(capacity));
     F.long_runs = c.take<int32_t>(capacity / (kShortRun + 1) + 1);
     return F;
 }
 
-int64_t finish_workspace_bytes(int64_t capacity) {
+int64_t finish_staged_workspace_bytes(int64_t capacity) {
     Carver c(nullptr);
     carve_finish(c, capacity);
     return c.bytes;
 }
 
+PairStage carve_stage(Carver& c, int64_t capacity) {
+    PairStage S;
+    S.l = c.take<uint32_t>(capacity);
+    S.r = c.take<int32_t>(capacity);
+    return S;
+}
+
+int64_t finish_workspace_bytes(int64_t capacity) {
+    Carver c(nullptr);
+    carve_stage(c, capacity);
+    c.take<char>(finish_staged_workspace_bytes(capacity));
+    return c.bytes;
+}
+
 void finish_stage(void* fin_ws, int64_t capacity, uint32_t** stage_l, int32_t** stage_r) {
     Carver c(fin_ws);
-    const FinishBufs F = carve_finish(c, capacity);
-    *stage_l = F.stage_l;
-    *stage_r = F.stage_r;
+    const PairStage S = carve_stage(c, capacity);
+    *stage_l = S.l;
+    *stage_r = S.r;
 }
 
 __global__ __launch_bounds__(256) void emit_pairs_kernel(const uint32_t* __restrict__ keys,
@@ -356,33 +366,31 @@ static int bits_for(int64_t n) {
 }
 
 // Slots per left row from which the pairs are sorted by both ids instead of by
-// left id and then run by run: there most runs pass kShortRun and would go
-// through the block sorts of long runs (2.3e9 ids/s), where a further radix pass
-// over the right ids takes its 20 B per pair at 4 TB/s.  51M pairs in 50k runs:
-// 22 ms of long runs against 0.8 ms of passes (index build + box query 25.2 ->
-// 6.7 ms); 5M pairs in 20k runs, contains query 4.7 -> 2.1 ms.  Below it the
-// short runs, sorted in registers in one pass, are cheaper than three passes.
-constexpr int64_t kLexSlots = 32;
+// left id and then run by run.  The slots are the pairs themselves in a planned
+// query, else the caller's bound on them.  Runs longer than kShortRun go through
+// the block sorts of long runs (2.3e9 ids/s), where a further radix pass over
+// the right ids takes its 20 B per pair at 4 TB/s.  Box query of 100k rows over
+// 4M points, sorted by both ids / by runs, us: 8 hits a row 509 / 470, 16
+// 525 / 510, 20 538 / 525, 24 563 / 599, 32 595 / 1401, 64 748 / 2814; of 2k
+// rows: 16 hits 230 / 215, 32 223 / 226, 64 234 / 242.  The line lies below the
+// crossing of these even rows because uneven ones pass kShortRun sooner.
+constexpr int64_t kLexSlots = 16;
 
-int finish_pairs(void* fin_ws, JoinCtl* ctl, int64_t n_left, int64_t n_right, int64_t capacity, bool sort_right,
-                 int64_t* out_l, int64_t* out_r, int64_t* d_result, hipStream_t s) {
+int finish_staged_pairs(const PairStage& S, void* ws, JoinCtl* ctl, int64_t n_left, int64_t n_right,
+                        int64_t capacity, bool sort_right, int64_t* out_l, int64_t* out_r, hipStream_t s) {
     VS_REQUIRE(capacity >= 0 && capacity < (int64_t)INT32_MAX, "join capacity %lld out of range [0, 2^31-1)",
                (long long)capacity);
     VS_REQUIRE(n_left >= 0 && n_left < (int64_t)UINT32_MAX, "left row count %lld out of range [0, 2^32-1)",
                (long long)n_left);
-    Carver c(fin_ws);
+    Carver c(ws);
     const FinishBufs F = carve_finish(c, capacity);
     const int nbits = bits_for(n_left);
     SortResult<uint32_t> r;
-    if (sort_right && nbits > 0 && n_right > 1 && n_right <= (int64_t)INT32_MAX && capacity / kLexSlots >= n_left) {
-        VS_TRY(sort_lex_wide_u32(F.stage_l, F.stage_r, capacity, &ctl->staged, nbits, bits_for(n_right), F.sort_ws,
-                                 sort_workspace_bytes_u32(capacity), s, out_l, out_r));
-        hipLaunchKernelGGL(publish_result_kernel, dim3(1), dim3(64), 0, s, ctl, d_result);
-        VS_LAUNCH_CHECK();
-        return VS_OK;
-    }
+    if (sort_right && nbits > 0 && n_right > 1 && n_right <= (int64_t)INT32_MAX && capacity / kLexSlots >= n_left)
+        return sort_lex_wide_u32(S.l, S.r, capacity, &ctl->staged, nbits, bits_for(n_right), F.sort_ws,
+                                 sort_workspace_bytes_u32(capacity), s, out_l, out_r);
     if (capacity > 1 && nbits > 0) {  // the sort's last pass writes the output pairs
-        VS_TRY(sort_pairs_u32_dev_wide(F.stage_l, F.stage_r, capacity, &ctl->staged, 0, nbits, F.sort_ws,
+        VS_TRY(sort_pairs_u32_dev_wide(S.l, S.r, capacity, &ctl->staged, 0, nbits, F.sort_ws,
                                        sort_workspace_bytes_u32(capacity), s, out_l, out_r, &r));
         if (sort_right) {
             const unsigned grid =
@@ -394,11 +402,9 @@ int finish_pairs(void* fin_ws, JoinCtl* ctl, int64_t n_left, int64_t n_right, in
                                r.alt_vals, ctl, capacity, F.long_runs, &ctl->n_long, out_r);
             VS_LAUNCH_CHECK();
         }
-        hipLaunchKernelGGL(publish_result_kernel, dim3(1), dim3(64), 0, s, ctl, d_result);
-        VS_LAUNCH_CHECK();
         return VS_OK;
     }
-    VS_TRY(sort_pairs_u32_dev(F.stage_l, F.stage_r, capacity, &ctl->staged, 0, nbits, F.sort_ws,
+    VS_TRY(sort_pairs_u32_dev(S.l, S.r, capacity, &ctl->staged, 0, nbits, F.sort_ws,
                               sort_workspace_bytes_u32(capacity), s, &r));
     if (capacity > 0) {
         const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(ceil_div(capacity, 256), 65536));
@@ -411,6 +417,15 @@ int finish_pairs(void* fin_ws, JoinCtl* ctl, int64_t n_left, int64_t n_right, in
             VS_LAUNCH_CHECK();
         }
     }
+    return VS_OK;
+}
+
+int finish_pairs(void* fin_ws, JoinCtl* ctl, int64_t n_left, int64_t n_right, int64_t capacity, bool sort_right,
+                 int64_t* out_l, int64_t* out_r, int64_t* d_result, hipStream_t s) {
+    Carver c(fin_ws);
+    const PairStage S = carve_stage(c, capacity);
+    void* ws = c.take<char>(finish_staged_workspace_bytes(capacity));
+    VS_TRY(finish_staged_pairs(S, ws, ctl, n_left, n_right, capacity, sort_right, out_l, out_r, s));
     hipLaunchKernelGGL(publish_result_kernel, dim3(1), dim3(64), 0, s, ctl, d_result);
     VS_LAUNCH_CHECK();
     return VS_OK;

@@ -23,12 +23,25 @@ struct JoinCtl {
 void ctl_reset(JoinCtl* ctl, hipStream_t s, unsigned long long* extra = nullptr, int n_extra = 0);
 void fill_i32(int32_t* p, int64_t n, int32_t v, hipStream_t s);
 
-// Finish (vs_finish.hip).  A join appends pairs to the two stage arrays that
-// finish_stage carves from the finish workspace (left ids as u32, right ids as
-// i32, `capacity` slots, ctl->staged the count); finish_pairs turns them into
-// int64 output sorted by left id (and by right id within a left id when
-// sort_right) and publishes d_result[0..3].  n_right: right ids are below it
-// (0: not known); it lets a join of many hits per left row sort by both ids.
+// Finish (vs_finish.hip).  A join appends pairs to two stage arrays (left ids
+// as u32, right ids as i32, ctl->staged the count); finish_staged_pairs turns
+// them into int64 output sorted by left id (and by right id within a left id
+// when sort_right).  capacity: slots of the output, at most those of the stage;
+// a count above it leaves the output unwritten and the stage as it is.  n_right:
+// right ids are below it (0: not known); it lets a join of many hits per left
+// row sort by both ids.  A finish reorders the stage, so it runs once.
+struct PairStage {
+    uint32_t* l;
+    int32_t* r;
+};
+
+PairStage carve_stage(Carver& c, int64_t capacity);
+int64_t finish_staged_workspace_bytes(int64_t capacity);
+int finish_staged_pairs(const PairStage& S, void* ws, JoinCtl* ctl, int64_t n_left, int64_t n_right,
+                        int64_t capacity, bool sort_right, int64_t* out_l, int64_t* out_r, hipStream_t s);
+
+// The same with the stage in one workspace, from which finish_stage carves it;
+// finish_pairs also publishes d_result[0..3].
 int64_t finish_workspace_bytes(int64_t capacity);
 void finish_stage(void* fin_ws, int64_t capacity, uint32_t** stage_l, int32_t** stage_r);
 int finish_pairs(void* fin_ws, JoinCtl* ctl, int64_t n_left, int64_t n_right, int64_t capacity, bool sort_right,

@@ -1898,6 +1898,10 @@ __global__ __launch_bounds__(256) void item_map_kernel(const int32_t* __restrict
 __global__ void publish_learned_kernel(const JoinCtl* __restrict__ ctl, const unsigned long long* __restrict__ cst,
                                        const int32_t* __restrict__ meta, int64_t* __restrict__ result) {
     if (threadIdx.x == 0) {
+        result[0] = (int64_t)ctl->staged;
+        result[1] = (int64_t)ctl->staged;
+        result[2] = (int64_t)ctl->stat[0];
+        result[3] = (int64_t)ctl->stat[1];
         result[4] = (int64_t)ctl->stat[2];
         result[5] = (int64_t)ctl->stat[3];
         result[6] = (int64_t)ctl->escalated_pairs;
@@ -2129,9 +2133,15 @@ QueryBufs carve_plan(Carver& c, int64_t nq, int64_t n_left) {
     return Q;
 }
 
+void carve_query_stage(Carver& c, int64_t capacity, QueryBufs* Q) {
+    const PairStage S = carve_stage(c, capacity);
+    Q->stage_l = S.l;
+    Q->stage_r = S.r;
+}
+
 void carve_finish_ws(Carver& c, int64_t capacity, QueryBufs* Q) {
-    Q->fin_ws = c.take<char>(finish_workspace_bytes(capacity));
-    if (c.base) finish_stage(Q->fin_ws, capacity, &Q->stage_l, &Q->stage_r);
+    carve_query_stage(c, capacity, Q);
+    Q->fin_ws = c.take<char>(finish_staged_workspace_bytes(capacity));
 }
 
 QueryBufs carve_query(Carver& c, int64_t nq, int64_t n_left, int64_t capacity) {
@@ -2184,12 +2194,11 @@ int learned_plan_t(int mode, const double4* qbox, int64_t nq, const LearnedView<
     return VS_OK;
 }
 
-// Second half: the scan and refine of the planned items (Q.ctl cleared by the
-// caller or by learned_plan_t), then the finish pass.
+// Second half: the scan and refine of the planned items into Q's stage (Q.ctl
+// cleared by the caller or by learned_plan_t), and the result words.
 template <class K>
-int learned_run_t(int mode, int pred, const double4* qbox, int64_t nq, int64_t n_points, const IndexBufs<K>& B,
-                  const RefineView& R, int64_t n_left, int64_t capacity, bool sort, const QueryBufs& Q,
-                  int64_t* out_l, int64_t* out_r, int64_t* d_result, hipStream_t s) {
+int learned_scan_t(int mode, int pred, const double4* qbox, int64_t nq, const IndexBufs<K>& B, const RefineView& R,
+                   int64_t capacity, const QueryBufs& Q, int64_t* d_result, hipStream_t s) {
     if (nq > 0) {
         int dev = 0, cus = 256;
         if (hipGetDevice(&dev) == hipSuccess) {
@@ -2216,11 +2225,19 @@ int learned_run_t(int mode, int pred, const double4* qbox, int64_t nq, int64_t n
         VS_LAUNCH_CHECK();
         VS_TRY(timing_end_public(s));
     }
-    VS_TRY(finish_pairs(Q.fin_ws, Q.ctl, n_left, mode == kLModePip ? nq : n_points, capacity, sort, out_l, out_r,
-                        d_result, s));
     hipLaunchKernelGGL(publish_learned_kernel, dim3(1), dim3(64), 0, s, Q.ctl, Q.cstat, B.meta, d_result);
     VS_LAUNCH_CHECK();
     return VS_OK;
+}
+
+// Scan and finish at one capacity.
+template <class K>
+int learned_run_t(int mode, int pred, const double4* qbox, int64_t nq, int64_t n_points, const IndexBufs<K>& B,
+                  const RefineView& R, int64_t n_left, int64_t capacity, bool sort, const QueryBufs& Q,
+                  int64_t* out_l, int64_t* out_r, int64_t* d_result, hipStream_t s) {
+    VS_TRY(learned_scan_t<K>(mode, pred, qbox, nq, B, R, capacity, Q, d_result, s));
+    return finish_staged_pairs({Q.stage_l, Q.stage_r}, Q.fin_ws, Q.ctl, n_left, mode == kLModePip ? nq : n_points,
+                               capacity, sort, out_l, out_r, s);
 }
 
 template <class K>
@@ -2486,12 +2503,83 @@ int vs_learned_query_plan(const void* index, int64_t n_points, int32_t key_bytes
     return VS_OK;
 }
 
-int64_t vs_learned_run_workspace_bytes(int64_t n_coords, int64_t capacity) {
+int64_t vs_learned_scan_workspace_bytes(int64_t n_coords, int64_t capacity) {
     vs::Carver c(nullptr);
     vs::QueryBufs Q = {};
+    vs::carve_query_stage(c, capacity, &Q);
     c.take<uint8_t>(n_coords);
-    vs::carve_finish_ws(c, capacity, &Q);
     return c.bytes;
+}
+
+int vs_learned_query_scan(const void* index, int64_t n_points, int32_t key_bytes, int32_t n_leaves,
+                          const double* boxes, const double* x, const double* y, const int32_t* geom_offsets,
+                          const int32_t* part_offsets, const int32_t* ring_offsets, int64_t n_queries,
+                          int64_t n_parts, int64_t n_rings, int64_t n_coords, int32_t predicate, int64_t capacity,
+                          int64_t* d_result, void* plan, int64_t plan_bytes, void* workspace,
+                          int64_t workspace_bytes, void* stream) {
+    vs::clear_error();
+    VS_REQUIRE(key_bytes == 4 || key_bytes == 8, "vs_learned_query_scan: key_bytes must be 4 or 8");
+    VS_REQUIRE(n_queries >= 0 && n_queries < (int64_t)INT32_MAX, "vs_learned_query_scan: n_queries out of range");
+    VS_REQUIRE(n_coords >= 0 && n_coords < (int64_t)INT32_MAX, "vs_learned_query_scan: n_coords out of range");
+    VS_REQUIRE(capacity >= 0 && capacity < (int64_t)INT32_MAX, "vs_learned_query_scan: capacity out of range");
+    VS_REQUIRE((geom_offsets != nullptr) == (part_offsets != nullptr) &&
+                   (geom_offsets != nullptr) == (ring_offsets != nullptr),
+               "vs_learned_query_scan: all polygon offsets or none");
+    VS_REQUIRE(!geom_offsets || predicate == VS_PRED_CONTAINS || predicate == VS_PRED_CONTAINS_PROPERLY ||
+                   predicate == VS_PRED_COVERS || predicate == VS_PRED_INTERSECTS || predicate == VS_PRED_TOUCHES,
+               "vs_learned_query_scan: unsupported predicate %d", predicate);
+    VS_REQUIRE(d_result != nullptr, "vs_learned_query_scan: null result");
+    VS_REQUIRE(plan_bytes >= vs_learned_plan_bytes(n_queries), "vs_learned_query_scan: plan too small");
+    VS_REQUIRE(workspace_bytes >= vs_learned_scan_workspace_bytes(n_coords, capacity),
+               "vs_learned_query_scan: workspace too small");
+    vs::Carver ci(const_cast<void*>(index));
+    vs::Carver cp(plan);
+    vs::Carver cw(workspace);
+    vs::QueryBufs Q = vs::carve_plan(cp, n_queries, n_queries);
+    vs::carve_query_stage(cw, capacity, &Q);
+    uint8_t* flags = cw.take<uint8_t>(n_coords);
+    hipStream_t s = vs::stream_of(stream);
+    const int mode = geom_offsets ? vs::kLModePipQ : vs::kLModeBox;
+    if (geom_offsets) VS_TRY(vs::build_refine_flags(part_offsets, ring_offsets, n_parts, n_rings, n_coords, flags, s));
+    const vs::RefineView R = {x, y, geom_offsets, part_offsets, ring_offsets, flags};
+    const double4* qb = reinterpret_cast<const double4*>(boxes);
+    vs::ctl_reset(Q.ctl, s);  // a plan may be scanned more than once
+    VS_LAUNCH_CHECK();
+    if (key_bytes == 4)
+        return vs::learned_scan_t<uint32_t>(mode, predicate, qb, n_queries,
+                                            vs::carve_index<uint32_t>(ci, n_points, n_leaves), R, capacity, Q,
+                                            d_result, s);
+    return vs::learned_scan_t<uint64_t>(mode, predicate, qb, n_queries,
+                                        vs::carve_index<uint64_t>(ci, n_points, n_leaves), R, capacity, Q, d_result,
+                                        s);
+}
+
+int64_t vs_learned_finish_workspace_bytes(int64_t capacity) { return vs::finish_staged_workspace_bytes(capacity); }
+
+int vs_learned_query_finish(int64_t n_points, int64_t n_queries, int64_t scan_capacity, int64_t capacity,
+                            int32_t sort, int64_t* out_left, int64_t* out_right, void* plan, int64_t plan_bytes,
+                            void* scan_workspace, int64_t scan_workspace_bytes, void* workspace,
+                            int64_t workspace_bytes, void* stream) {
+    vs::clear_error();
+    VS_REQUIRE(n_queries >= 0 && n_queries < (int64_t)INT32_MAX, "vs_learned_query_finish: n_queries out of range");
+    VS_REQUIRE(capacity >= 0 && capacity <= scan_capacity && scan_capacity < (int64_t)INT32_MAX,
+               "vs_learned_query_finish: capacity out of range");
+    VS_REQUIRE(plan_bytes >= vs_learned_plan_bytes(n_queries), "vs_learned_query_finish: plan too small");
+    VS_REQUIRE(scan_workspace_bytes >= vs_learned_scan_workspace_bytes(0, scan_capacity),
+               "vs_learned_query_finish: scan workspace too small");
+    VS_REQUIRE(workspace_bytes >= vs_learned_finish_workspace_bytes(capacity),
+               "vs_learned_query_finish: workspace too small");
+    vs::Carver cp(plan);
+    vs::Carver cs(scan_workspace);
+    const vs::QueryBufs Q = vs::carve_plan(cp, n_queries, n_queries);
+    const vs::PairStage S = vs::carve_stage(cs, scan_capacity);
+    return vs::finish_staged_pairs(S, workspace, Q.ctl, n_queries, n_points, capacity, sort != 0, out_left, out_right,
+                                   vs::stream_of(stream));
+}
+
+int64_t vs_learned_run_workspace_bytes(int64_t n_coords, int64_t capacity) {
+    return ((vs_learned_scan_workspace_bytes(n_coords, capacity) + 255) & ~int64_t(255)) +
+           vs_learned_finish_workspace_bytes(capacity);
 }
 
 int vs_learned_query_run(const void* index, int64_t n_points, int32_t key_bytes, int32_t n_leaves,
@@ -2500,42 +2588,16 @@ int vs_learned_query_run(const void* index, int64_t n_points, int32_t key_bytes,
                          int64_t n_rings, int64_t n_coords, int32_t predicate, int64_t capacity, int32_t sort,
                          int64_t* out_left, int64_t* out_right, int64_t* d_result, void* plan, int64_t plan_bytes,
                          void* workspace, int64_t workspace_bytes, void* stream) {
-    vs::clear_error();
-    VS_REQUIRE(key_bytes == 4 || key_bytes == 8, "vs_learned_query_run: key_bytes must be 4 or 8");
-    VS_REQUIRE(n_queries >= 0 && n_queries < (int64_t)INT32_MAX, "vs_learned_query_run: n_queries out of range");
-    VS_REQUIRE(n_coords >= 0 && n_coords < (int64_t)INT32_MAX, "vs_learned_query_run: n_coords out of range");
-    VS_REQUIRE(capacity >= 0 && capacity < (int64_t)INT32_MAX, "vs_learned_query_run: capacity out of range");
-    VS_REQUIRE((geom_offsets != nullptr) == (part_offsets != nullptr) &&
-                   (geom_offsets != nullptr) == (ring_offsets != nullptr),
-               "vs_learned_query_run: all polygon offsets or none");
-    VS_REQUIRE(!geom_offsets || predicate == VS_PRED_CONTAINS || predicate == VS_PRED_CONTAINS_PROPERLY ||
-                   predicate == VS_PRED_COVERS || predicate == VS_PRED_INTERSECTS || predicate == VS_PRED_TOUCHES,
-               "vs_learned_query_run: unsupported predicate %d", predicate);
-    VS_REQUIRE(d_result != nullptr, "vs_learned_query_run: null result");
-    VS_REQUIRE(plan_bytes >= vs_learned_plan_bytes(n_queries), "vs_learned_query_run: plan too small");
+    const int64_t scan_bytes = vs_learned_scan_workspace_bytes(n_coords, capacity);
+    const int64_t finish_bytes = vs_learned_finish_workspace_bytes(capacity);
     VS_REQUIRE(workspace_bytes >= vs_learned_run_workspace_bytes(n_coords, capacity),
                "vs_learned_query_run: workspace too small");
-    vs::Carver ci(const_cast<void*>(index));
-    vs::Carver cp(plan);
-    vs::Carver cw(workspace);
-    vs::QueryBufs Q = vs::carve_plan(cp, n_queries, n_queries);
-    uint8_t* flags = cw.take<uint8_t>(n_coords);
-    vs::carve_finish_ws(cw, capacity, &Q);
-    hipStream_t s = vs::stream_of(stream);
-    const int mode = geom_offsets ? vs::kLModePipQ : vs::kLModeBox;
-    if (geom_offsets) VS_TRY(vs::build_refine_flags(part_offsets, ring_offsets, n_parts, n_rings, n_coords, flags, s));
-    const vs::RefineView R = {x, y, geom_offsets, part_offsets, ring_offsets, flags};
-    const double4* qb = reinterpret_cast<const double4*>(boxes);
-    vs::ctl_reset(Q.ctl, s);  // a plan may be run more than once
-    VS_LAUNCH_CHECK();
-    if (key_bytes == 4) {
-        const auto B = vs::carve_index<uint32_t>(ci, n_points, n_leaves);
-        return vs::learned_run_t<uint32_t>(mode, predicate, qb, n_queries, n_points, B, R, n_queries, capacity,
-                                           sort != 0, Q, out_left, out_right, d_result, s);
-    }
-    const auto B = vs::carve_index<uint64_t>(ci, n_points, n_leaves);
-    return vs::learned_run_t<uint64_t>(mode, predicate, qb, n_queries, n_points, B, R, n_queries, capacity, sort != 0,
-                                       Q, out_left, out_right, d_result, s);
+    VS_TRY(vs_learned_query_scan(index, n_points, key_bytes, n_leaves, boxes, x, y, geom_offsets, part_offsets,
+                                 ring_offsets, n_queries, n_parts, n_rings, n_coords, predicate, capacity, d_result,
+                                 plan, plan_bytes, workspace, scan_bytes, stream));
+    void* finish_ws = static_cast<char*>(workspace) + ((scan_bytes + 255) & ~int64_t(255));
+    return vs_learned_query_finish(n_points, n_queries, capacity, capacity, sort, out_left, out_right, plan,
+                                   plan_bytes, workspace, scan_bytes, finish_ws, finish_bytes, stream);
 }
 
 int64_t vs_sjoin_points_polygons_learned_workspace_bytes(int64_t n_points, int64_t n_polys, int64_t n_coords,

@@ -479,8 +479,8 @@ def _learned_stats(h, cap, retries) -> LearnedStats:
 
 LOOKUP_MODES = {"learned": 0, "leaves": 1, "binary": 2}
 
-# Largest output a planned query allocates from its scan length (24 B per slot
-# with the staged pairs, 16 B for the sort's alternates): 2^28 slots, 11 GB.
+# Largest stage a planned query sizes from its scan length: 2^28 slots of 8
+# bytes, given back when the call ends.
 POSITION_LIMIT = 2**28
 
 
@@ -583,9 +583,10 @@ class LearnedPointIndex:
 
     def _planned_query(self, boxes: torch.Tensor, P: DevicePolygons | None, predicate, lookup: str, sort: bool):
         """query_boxes (P None) / query_polygons without a caller capacity: the
-        plan's scan length, an upper bound of the pairs, sizes the output, so
-        the scan runs once.  A bound over POSITION_LIMIT is not allocated: the
-        planned scan then runs twice, the first time to count."""
+        plan's scan length, an upper bound of the pairs, sizes the stage, so the
+        scan runs once; the pairs it staged size the output and the finish.  A
+        bound over POSITION_LIMIT is not allocated: the planned scan then runs
+        twice, the first time to count."""
         dev = require_gpu()
         L = lib()
         nq = int(boxes.shape[0])
@@ -601,22 +602,28 @@ class LearnedPointIndex:
         cap = max(1024, bound if bound <= POSITION_LIMIT else min(4 * nq, PAIR_LIMIT))
         retries = 0
         while True:
-            ws = _ws(L.vs_learned_run_workspace_bytes(sizes[2], cap), dev)
-            out_l = torch.empty(cap, dtype=torch.int64, device=dev)
-            out_r = torch.empty(cap, dtype=torch.int64, device=dev)
-            res = torch.zeros(16, dtype=torch.int64, device=dev)
-            check(L.vs_learned_query_run(*index, *(ptr(t) for t in xy + offsets), nq, *sizes,
-                                         PRED["intersects" if P is None else predicate], cap, int(bool(sort)),
-                                         ptr(out_l), ptr(out_r), ptr(res), ptr(plan), plan.numel(), ptr(ws),
-                                         ws.numel(), stream()), "vs_learned_query_run")
+            stage = _ws(L.vs_learned_scan_workspace_bytes(sizes[2], cap), dev)
+            res = torch.empty(16, dtype=torch.int64, device=dev)
+            check(L.vs_learned_query_scan(*index, *(ptr(t) for t in xy + offsets), nq, *sizes,
+                                          PRED["intersects" if P is None else predicate], cap, ptr(res), ptr(plan),
+                                          plan.numel(), ptr(stage), stage.numel(), stream()), "vs_learned_query_scan")
             h = res.cpu().tolist()
-            if h[1] <= cap:
-                return out_l[: h[0]], out_r[: h[0]], _learned_stats(h, cap, retries)
-            if h[1] > PAIR_LIMIT:
-                raise _PairLimit(h[1])
-            del ws, out_l, out_r
-            cap = int(h[1])
+            n = int(h[1])
+            if n <= cap:
+                break
+            if n > PAIR_LIMIT:
+                raise _PairLimit(n)
+            del stage
+            cap = n
             retries += 1
+        out_l = torch.empty(n, dtype=torch.int64, device=dev)
+        out_r = torch.empty(n, dtype=torch.int64, device=dev)
+        if n:
+            ws = _ws(L.vs_learned_finish_workspace_bytes(n), dev)
+            check(L.vs_learned_query_finish(self.n, nq, cap, n, int(bool(sort)), ptr(out_l), ptr(out_r), ptr(plan),
+                                            plan.numel(), ptr(stage), stage.numel(), ptr(ws), ws.numel(), stream()),
+                  "vs_learned_query_finish")
+        return out_l, out_r, _learned_stats(h, cap, retries)
 
     def query_boxes(self, boxes: torch.Tensor, lookup: str = "learned", capacity: int | None = None,
                     sort: bool = True):

@@ -1,5 +1,5 @@
 """Index queries sized by their plan: one scan where the bound is allocated,
-two where it is not, the empty query, output that is sized by the pairs and not
+two where it is not or where there is no memory for it, the empty query, output that is sized by the pairs and not
 by the scan, and the C entry that scans and finishes at one capacity."""
 
 from __future__ import annotations
@@ -68,6 +68,31 @@ def test_few_hits_of_a_long_scan_leave_little_allocated():
     assert peak < 10 * st.scanned  # the stage's 8 bytes a position, plan and output beside it
     l, r, st = idx.query_polygons(D, b, "touches")
     assert l.numel() == 0 and r.numel() == 0 and st.pairs == 0
+
+
+def test_no_memory_for_the_bound_counts_first(monkeypatch):
+    w = S.c1(n_points=300_000, n_polys=120)
+    idx = J.LearnedPointIndex(DevicePoints.from_host(w.points))
+    D = DevicePolygons.from_host(w.polygons)
+    b = J.polygon_bounds(D)
+    want = idx.query_polygons(D, b, "contains")
+
+    def refuse_from(slots):  # no memory for a stage of that many slots
+        limit = _lib.lib().vs_learned_scan_workspace_bytes(D.n_coords, slots)
+
+        def ws(nbytes, dev):
+            if nbytes >= limit:
+                raise torch.OutOfMemoryError("no room")
+            return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=dev)
+
+        monkeypatch.setattr(J, "_ws", ws)
+
+    refuse_from(want[2].scanned)
+    l, r, st = idx.query_polygons(D, b, "contains")
+    assert st.retries == 1 and torch.equal(l, want[0]) and torch.equal(r, want[1])
+    refuse_from(want[2].pairs)
+    with pytest.raises(torch.OutOfMemoryError):
+        idx.query_polygons(D, b, "contains")
 
 
 @pytest.mark.parametrize("slots", [0, 1])

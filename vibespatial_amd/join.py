@@ -585,8 +585,8 @@ class LearnedPointIndex:
         """query_boxes (P None) / query_polygons without a caller capacity: the
         plan's scan length, an upper bound of the pairs, sizes the stage, so the
         scan runs once; the pairs it staged size the output and the finish.  A
-        bound over POSITION_LIMIT is not allocated: the planned scan then runs
-        twice, the first time to count."""
+        bound over POSITION_LIMIT, or one there is no memory for, is not
+        allocated: the planned scan then runs twice, the first time to count."""
         dev = require_gpu()
         L = lib()
         nq = int(boxes.shape[0])
@@ -599,10 +599,17 @@ class LearnedPointIndex:
         check(L.vs_learned_query_plan(*index, *(ptr(t) for t in offsets), nq, LOOKUP_MODES[lookup], ptr(pos),
                                       ptr(plan), plan.numel(), stream()), "vs_learned_query_plan")
         bound = int(pos.item())
-        cap = max(1024, bound if bound <= POSITION_LIMIT else min(4 * nq, PAIR_LIMIT))
+        count_first = max(1024, min(4 * nq, PAIR_LIMIT))
+        cap = max(1024, bound) if bound <= POSITION_LIMIT else count_first
         retries = 0
         while True:
-            stage = _ws(L.vs_learned_scan_workspace_bytes(sizes[2], cap), dev)
+            try:
+                stage = _ws(L.vs_learned_scan_workspace_bytes(sizes[2], cap), dev)
+            except torch.OutOfMemoryError:
+                if retries or cap <= count_first:
+                    raise
+                cap = count_first
+                continue
             res = torch.empty(16, dtype=torch.int64, device=dev)
             check(L.vs_learned_query_scan(*index, *(ptr(t) for t in xy + offsets), nq, *sizes,
                                           PRED["intersects" if P is None else predicate], cap, ptr(res), ptr(plan),

@@ -1,6 +1,7 @@
 """Index queries sized by their plan: one scan where the bound is allocated,
-two where it is not or where there is no memory for it, the empty query, output that is sized by the pairs and not
-by the scan, and the C entry that scans and finishes at one capacity."""
+two where it is not or where there is no memory for it, the empty query, few
+rows, whose plan is not waited for, output that is sized by the pairs and not by
+the scan, and the C entry that scans and finishes at one capacity."""
 
 from __future__ import annotations
 
@@ -93,6 +94,29 @@ def test_no_memory_for_the_bound_counts_first(monkeypatch):
     refuse_from(want[2].pairs)
     with pytest.raises(torch.OutOfMemoryError):
         idx.query_polygons(D, b, "contains")
+
+
+@pytest.mark.parametrize("n_queries", [1, 15, 16, 17])
+@pytest.mark.parametrize("few_slots", [2**20, 1200])
+def test_few_queries(monkeypatch, n_queries, few_slots):
+    """Either side of the rows from which the plan's scan length is read, with
+    room for the pairs and without."""
+    monkeypatch.setattr(J, "FEW_SLOTS", few_slots)
+    w = S.c1(n_points=200_000, n_polys=120)
+    x, y = w.points.x, w.points.y
+    P = w.polygons.take(np.arange(n_queries))
+    idx = J.LearnedPointIndex(DevicePoints.from_host(w.points))
+    D = DevicePolygons.from_host(P)
+    b = J.polygon_bounds(D)
+    el, er = oracle.sjoin_points_polygons(x, y, P, "within")
+    o = np.lexsort((el, er))
+    l, r, st = idx.query_polygons(D, b, "contains")
+    assert np.array_equal(l.cpu().numpy(), er[o]) and np.array_equal(r.cpu().numpy(), el[o])
+    assert st.retries == int(n_queries <= J.FEW_QUERIES and len(el) > few_slots)
+    el, er = oracle.box_query_points(x, y, b.cpu().numpy())
+    l, r, st = idx.query_boxes(b)
+    assert np.array_equal(l.cpu().numpy(), el) and np.array_equal(r.cpu().numpy(), er)
+    assert st.retries == int(n_queries <= J.FEW_QUERIES and len(el) > few_slots)
 
 
 @pytest.mark.parametrize("slots", [0, 1])

@@ -1579,7 +1579,10 @@ __global__ __launch_bounds__(kLJThreads, 4) void learned_join_kernel(
         const bool direct = MODE == kLModeBox || direct_polygon(qinfo);
         const int per = direct ? kItemPos : kChunk;  // item_positions(qinfo)
         const int first = chunk * per;
-        const int last = (first + per < total) ? first + per : total;
+        int last = first + per;
+        if (!direct)  // claimed items of one streamed row run as one: their candidates share the passes over its edges
+            for (; claim_k < n_claim && uniform_i32(s_claim[claim_k].x) == q; ++claim_k) last += kChunk;
+        last = last < total ? last : total;
         int4 info = make_int4(0, 0, 0, 0);
         double cx = 0, cy = 0;
         float E = 0.0f;
@@ -1792,6 +1795,10 @@ __global__ __launch_bounds__(kLJThreads, 4) void learned_join_kernel(
                         Ft[c - b0 + 1] = R.flags[c];
                     }
                     __syncthreads();
+                    bool live = false;  // a wave without an open candidate leaves the issue slots to others
+#pragma unroll
+                    for (int j = 0; j < kCandPerThread; ++j) live |= !done[j];
+                    if (__ballot(live) == 0) continue;
                     for (int32_t c = b0; c < b1; ++c) {
                         const int f = Ft[c - b0 + 1];
                         if (f & 2) {

@@ -58,3 +58,41 @@ def test_close_rows(n):
         assert set(kl.cpu().tolist()) == {2, 6}, hl
         kl, _ = api._refine(1, "contains_properly", r, l, None, B, A, heavy_log2=hl)
         assert set(kl.cpu().tolist()) == {4}, hl
+
+
+@pytest.mark.parametrize("per_side", [1, 2, 5])
+def test_rows_that_share_edges(per_side):
+    """A grid of squares, each side in one edge or several, with itself and with
+    the squares inset by a quarter: contacts without a crossing, equal rows,
+    nested rows, by every route, against the grid positions."""
+    import torch
+
+    from vibespatial_amd import api
+
+    m = 6
+
+    def square(i, j, d):
+        t = [k / per_side for k in range(per_side)]
+        w = 1 - 2 * d
+        x, y = i + d, j + d
+        return Polygon([(x + w * a, y) for a in t] + [(x + w, y + w * a) for a in t]
+                       + [(x + w - w * a, y + w) for a in t] + [(x, y + w - w * a) for a in t])
+
+    cells = [(i, j) for i in range(m) for j in range(m)]
+    A = PolygonArray.from_geometries([square(i, j, 0.0) for i, j in cells])
+    inner = PolygonArray.from_geometries([square(i, j, 0.25) for i, j in cells])
+    pairs = [(a, b) for a in range(m * m) for b in range(m * m)
+             if max(abs(cells[a][0] - cells[b][0]), abs(cells[a][1] - cells[b][1])) <= 1]
+    l = torch.tensor([p[0] for p in pairs], dtype=torch.int64, device="cuda")
+    r = torch.tensor([p[1] for p in pairs], dtype=torch.int64, device="cuda")
+    same, other = {p for p in pairs if p[0] == p[1]}, {p for p in pairs if p[0] != p[1]}
+    with_itself = {"intersects": same | other, "touches": other, "overlaps": set(), "within": same, "covers": same,
+                   "contains_properly": set()}
+    with_inner = {"intersects": same, "touches": set(), "overlaps": set(), "within": set(), "covers": same,
+                  "contains_properly": same}
+    for B, expect in ((A, with_itself), (inner, with_inner)):
+        for pred, want in expect.items():
+            for hl in (0, 1, 63):
+                print(f"shared edges {per_side} {pred} {hl}", flush=True)
+                kl, kr = api._refine(1, pred, l, r, None, A, B, heavy_log2=hl)
+                assert set(zip(kl.tolist(), kr.tolist())) == want, (pred, hl)

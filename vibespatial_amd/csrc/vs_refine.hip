@@ -45,17 +45,33 @@ __device__ __forceinline__ int loc_keep(int pred, int loc) {
 // Pairs are visited in order[t] when given (polygon pairs grouped by right
 // row, so the lanes of a wave mostly share one right polygon).  Polygon pairs
 // whose coordinate counts multiply to more than the heavy-pair threshold, and
-// those the cheap tests leave undecided, go to `heavy` (count in *n_heavy) for
-// refine_heavy_kernel, one wave per pair, which decides all but rows whose
-// boundaries touch without crossing; those go to `undecided` for
-// refine_relate_kernel, so neither of the others carries the full relation's
-// registers.  At 2^8 small pairs (box x box: 25) stay one per lane; one lane
-// walking the edge pairs of two many-vertex polygons leaves the rest of its
+// those the cheap tests leave undecided with one box inside the other, go to
+// `heavy` (count in *n_heavy) for refine_heavy_kernel, one wave per pair; pairs
+// whose boundaries touch without crossing go to `undecided`, from here or from
+// there, for refine_relate_kernel, so neither of the others carries the full
+// relation's registers.  (With every undecided pair through refine_heavy_kernel
+// first, rows that share edges paid for both: touches among 90k unit squares,
+// 716k pairs, 65.0 ms against 54.2.  The lists are appended to with one atomic
+// per wave, written out: two atomics in two branches become one with a pointer
+// per lane, which the compiler no longer joins, 1.7 -> 7.5 ms there.)
+// At 2^8 small pairs (box x box: 25) stay one per lane; one lane walking the edge pairs of two many-vertex polygons leaves the rest of its
 // wave idle, so those go one wave per pair (100k x 100k star polygons,
 // overlaps: 49 ms per step at 2^15, 24 at 2^12, 15.7 at 2^8, flat below).
 // The caller can move the threshold (bits 8-15 of vs_refine_pairs' mode), so
 // tests run the same pairs through both routes.
 constexpr int kHeavyPairLog2 = 8;
+
+// Appends v to list[0, *count) where `add`, for the active lanes of a wave.
+__device__ __forceinline__ void wave_append(bool add, int32_t v, int32_t* __restrict__ list,
+                                            unsigned long long* __restrict__ count) {
+    const uint64_t m = __ballot(add);
+    if (m == 0) return;
+    const int leader = __ffsll((unsigned long long)m) - 1;
+    unsigned long long base = 0;
+    if ((int)(threadIdx.x & 63) == leader) base = atomicAdd(count, (unsigned long long)__popcll(m));
+    base = __shfl(base, leader, 64);
+    if (add) list[base + __popcll(m & lanemask_lt())] = v;
+}
 
 __global__ __launch_bounds__(256) void refine_pairs_kernel(int mode, int pred, const int64_t* __restrict__ left,
                                                           const int64_t* __restrict__ right, int64_t n,
@@ -64,23 +80,29 @@ __global__ __launch_bounds__(256) void refine_pairs_kernel(int mode, int pred, c
                                                           const double* __restrict__ py, Polys A, Polys B,
                                                           int32_t* __restrict__ keep, int32_t* __restrict__ heavy,
                                                           unsigned long long* __restrict__ n_heavy,
+                                                          int32_t* __restrict__ undecided,
+                                                          unsigned long long* __restrict__ n_undecided,
                                                           int64_t heavy_pair) {
     for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < n; t += (int64_t)gridDim.x * 256) {
         const int64_t i = order ? (int64_t)order[t] : t;
         const int64_t l = left[i], r = right[i];
-        int k;
+        int k, f = 0;
+        bool large = false;
         if (mode == 0 || mode == 2) {
             const int64_t pi = mode == 0 ? l : r, gi = mode == 0 ? r : l;
             const double x = px[pi], y = py[pi];
             const int loc = (x == x && y == y) ? point_location_f64(x, y, B.x, B.y, B.geom, B.part, B.ring, gi) : 0;
             k = loc_keep(pred, loc);
         } else if ((int64_t)row_coords(A, l) * row_coords(B, r) > heavy_pair) {
-            heavy[atomicAdd(n_heavy, 1ull)] = (int32_t)i;
+            large = true;
             k = 0;  // decided by refine_heavy_kernel
         } else {
-            const int f = polygon_predicate_fast(pred, A, l, B, r);
-            if (f < 0) heavy[atomicAdd(n_heavy, 1ull)] = (int32_t)i;
+            f = polygon_predicate_fast(pred, A, l, B, r);
             k = f > 0 ? 1 : 0;
+        }
+        if (mode == 1) {  // one atomic per wave and list
+            wave_append(large || f == -2, (int32_t)i, heavy, n_heavy);
+            wave_append(f == -1, (int32_t)i, undecided, n_undecided);
         }
         keep[i] = k;
     }
@@ -343,7 +365,7 @@ int vs_refine_pairs(int32_t mode, int32_t predicate, const int64_t* left, const 
         }
         const int grid = (int)std::min<int64_t>(vs::ceil_div(n_pairs, 256), 16384);
         hipLaunchKernelGGL(vs::refine_pairs_kernel, dim3(grid), dim3(256), 0, s, mode, predicate, left, right,
-                           n_pairs, ord, px, py, A, B, keep, heavy, n_heavy, heavy_pair);
+                           n_pairs, ord, px, py, A, B, keep, heavy, n_heavy, undecided, n_undecided, heavy_pair);
         VS_LAUNCH_CHECK();
         if (mode == 1) {
             const int hgrid = (int)std::min<int64_t>(vs::ceil_div(n_pairs, 4), 2048);

@@ -321,24 +321,32 @@ VS_HD bool relation_decides(int pred, const Relation& R) {
 // Cheap necessary conditions of predicate(A row, B row) for two polygonal
 // rows (codes of vsjoin.h): box containment for the containment predicates;
 // intersects, then a proper crossing -- which settles every relation -- for
-// touches / overlaps.  1 true, 0 false, -1 undecided (the full relation
-// decides, with intersects known to hold for touches).
-VS_HD int polygon_predicate_fast(int pred, const Polys& A, int64_t ra, const Polys& B, int64_t rb) {
+// touches / overlaps.  1 true, 0 false; undecided (intersects is known to hold
+// for touches then): -2 when one row's box lies strictly inside the other's,
+// else -1.  A polygon whose boundary does not meet another's lies strictly
+// inside it, box and all, or outside, so -1 means that the boundaries touch (or
+// that a row has several parts) and only the full relation can decide.
+__device__ inline int polygon_predicate_fast(int pred, const Polys& A, int64_t ra, const Polys& B, int64_t rb) {
     if (pred == VS_PRED_INTERSECTS) return polygons_intersect_auto(A, ra, B, rb) ? 1 : 0;
     if (pred == VS_PRED_CROSSES) return 0;
-    if (pred == VS_PRED_WITHIN || pred == VS_PRED_COVERED_BY || pred == VS_PRED_CONTAINS ||
-        pred == VS_PRED_COVERS || pred == VS_PRED_CONTAINS_PROPERLY) {
-        const bool a_inner = pred == VS_PRED_WITHIN || pred == VS_PRED_COVERED_BY;
-        const double4 in = a_inner ? row_box(A, ra) : row_box(B, rb);
-        const double4 out = a_inner ? row_box(B, rb) : row_box(A, ra);
+    const bool inclusion = pred != VS_PRED_TOUCHES && pred != VS_PRED_OVERLAPS;
+    const bool a_inner = pred == VS_PRED_WITHIN || pred == VS_PRED_COVERED_BY;
+    double4 in, out;
+    if (inclusion) {
+        in = a_inner ? row_box(A, ra) : row_box(B, rb);
+        out = a_inner ? row_box(B, rb) : row_box(A, ra);
         if (!(out.x <= in.x && in.z <= out.z && out.y <= in.y && in.w <= out.w)) return 0;
-        if (any_proper_crossing(A, ra, B, rb)) return 0;
-        return -1;
+    } else if (!polygons_intersect_auto(A, ra, B, rb)) {
+        return 0;
     }
-    // touches, overlaps
-    if (!polygons_intersect_auto(A, ra, B, rb)) return 0;
     if (any_proper_crossing(A, ra, B, rb)) return pred == VS_PRED_OVERLAPS ? 1 : 0;
-    return -1;
+    if (!inclusion) {
+        in = row_box(A, ra);
+        out = row_box(B, rb);
+    }
+    const bool nested = (out.x < in.x && in.z < out.z && out.y < in.y && in.w < out.w) ||
+                        (in.x < out.x && out.z < in.z && in.y < out.y && out.w < in.w);
+    return nested ? -2 : -1;
 }
 
 // ---------------------------------------------------------------------------

@@ -179,7 +179,8 @@ __device__ __forceinline__ double uniform_f64(double v) {
     return u.d;
 }
 
-// Orders one wave's LDS accesses where its lanes exchange data through LDS.
+// Orders one wave's LDS accesses around a point where its lanes exchange data
+// through LDS (a compiler barrier: a wave's LDS instructions run in order).
 __device__ __forceinline__ void wave_lds_order() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();

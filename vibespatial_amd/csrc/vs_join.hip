@@ -390,19 +390,13 @@ struct BoxWalk {
     int64_t staged_first, staged_count, staged_items;
     int nbuf;
 
-    __device__ __forceinline__ void fence() const {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-
     // Appends the wave's buffered pairs to the stage with one atomic.
     __device__ void flush() {
         if (nbuf == 0) return;
         unsigned long long base = 0;
         if (lane == 0) base = atomicAdd(&ctl->staged, (unsigned long long)nbuf);
         base = __shfl(base, 0, 64);
-        fence();
+        wave_lds_order();
         for (int i = lane; i < nbuf; i += 64) {
             const unsigned long long at = base + (unsigned long long)i;
             if (at < (unsigned long long)capacity) {
@@ -411,7 +405,7 @@ struct BoxWalk {
                 stage_r[at] = e.y;
             }
         }
-        fence();
+        wave_lds_order();
         nbuf = 0;
     }
 
@@ -459,14 +453,14 @@ struct BoxWalk {
         }
         const int sub = lane / U;
         while (sp > 0) {
-            fence();
+            wave_lds_order();
             const int np = sp < groups ? sp : groups;
             const bool act = slot < np;
             const int at = act ? sp - 1 - slot : 0;
             const int l = W.level[at];
             const int64_t pos = (int64_t)W.group[at] * T.fanout + child;
             sp -= np;
-            fence();
+            wave_lds_order();
             const bool in = act && pos < level_count[l];
             double4 b = make_double4(NAN, NAN, NAN, NAN);
             if (in) {

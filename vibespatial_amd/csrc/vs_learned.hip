@@ -1111,14 +1111,6 @@ __device__ int stage_all_edges(int32_t lo, int32_t hi, double cx, double cy, con
     return ne;
 }
 
-// Orders one wave's LDS accesses around a point where its lanes exchange data
-// through LDS (a compiler barrier: a wave's LDS instructions run in order).
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // stage_all_edges + build_slabs for a polygon whose edges fit one pass of the
 // block (hi - lo <= kLJThreads): each thread stages its own edge and counts
 // and lists it in its slabs from registers, so the pair takes four barriers
@@ -1473,7 +1465,7 @@ __global__ __launch_bounds__(kLJThreads, 4) void learned_join_kernel(
                         bool listed = false;
                         if (WS.B > 1) {
                             if (lane <= WS.B) wstart[lane] = 0;
-                            wave_lds_sync();
+                            wave_lds_order();
                             int eb0[2], eb1[2];
 #pragma unroll
                             for (int k = 0; k < 2; ++k) {
@@ -1485,7 +1477,7 @@ __global__ __launch_bounds__(kLJThreads, 4) void learned_join_kernel(
                                     for (int b = eb0[k]; b <= eb1[k]; ++b) atomicAdd(&wstart[b + 1], 1);
                                 }
                             }
-                            wave_lds_sync();
+                            wave_lds_order();
                             const int v = lane < WS.B ? wstart[lane + 1] : 0;
                             const int incs = wave_inclusive_scan(v);
                             if (lane < WS.B) {
@@ -1493,7 +1485,7 @@ __global__ __launch_bounds__(kLJThreads, 4) void learned_join_kernel(
                                 wcur[lane] = incs - v;
                             }
                             const int wtot = readlane_i32(incs, 63);
-                            wave_lds_sync();
+                            wave_lds_order();
                             if (wtot <= kBinCap / kClaim) {
 #pragma unroll
                                 for (int k = 0; k < 2; ++k)
@@ -1514,7 +1506,7 @@ __global__ __launch_bounds__(kLJThreads, 4) void learned_join_kernel(
                             for (int k = 0; k < 2; ++k)
                                 if (erel[k]) wlist[eslot[k]] = (uint16_t)eslot[k];
                         }
-                        wave_lds_sync();
+                        wave_lds_order();
                     }
                     unsigned n_orient = 0;
                     unsigned long long n_esc = 0;

@@ -54,9 +54,11 @@ __device__ __forceinline__ int loc_keep(int pred, int loc) {
 // 716k pairs, 65.0 ms against 54.2.  The lists are appended to with one atomic
 // per wave, written out: two atomics in two branches become one with a pointer
 // per lane, which the compiler no longer joins, 1.7 -> 7.5 ms there.)
-// At 2^8 small pairs (box x box: 25) stay one per lane; one lane walking the edge pairs of two many-vertex polygons leaves the rest of its
-// wave idle, so those go one wave per pair (100k x 100k star polygons,
-// overlaps: 49 ms per step at 2^15, 24 at 2^12, 15.7 at 2^8, flat below).
+// At 2^8 small pairs (box x box: 25) stay one per lane; one lane walking the
+// edge pairs of two many-vertex polygons leaves the rest of its wave idle, so
+// those go one wave per pair (100k x 100k star polygons, overlaps, with all
+// edge pairs tested: 49 ms per step at 2^15, 24 at 2^12, 15.7 at 2^8, flat
+// below).
 // The caller can move the threshold (bits 8-15 of vs_refine_pairs' mode), so
 // tests run the same pairs through both routes.
 constexpr int kHeavyPairLog2 = 8;

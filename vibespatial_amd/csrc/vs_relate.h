@@ -361,13 +361,6 @@ struct WaveEdgeLds {
     int32_t qa[kEdgeTile], qb[kEdgeTile];  // edge pairs whose boxes meet
 };
 
-// Orders one wave's LDS accesses where its lanes exchange data through LDS.
-__device__ __forceinline__ void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Boxes in fp32, every bound rounded to nearest.  Rounding is monotone, so
 // boxes that meet in fp64 meet in fp32: the tests on them only drop pairs that
 // cannot touch, and the exact tests see every other pair.
@@ -445,7 +438,7 @@ __device__ inline int wave_edge_pairs(const Polys& A, const RowSpan& sa, const f
     int found = 0, nq = 0;
     // exact tests of the first `n` (at most 64) queued pairs
     auto test_queue = [&](int n) {
-        wave_lds_fence();
+        wave_lds_order();
         int k = 0;
         if (lane < n) {
             const int32_t c = W.qa[lane], d = W.qb[lane];
@@ -465,7 +458,7 @@ __device__ inline int wave_edge_pairs(const Polys& A, const RowSpan& sa, const f
         }
         const bool last = a0 + 64 >= sa.hi;
         while (na >= 64 || (last && na > 0)) {
-            wave_lds_fence();
+            wave_lds_order();
             const int n = na < 64 ? na : 64;
             int width = 1;  // lanes per pass over A's edges; 64 / width share each B tile
             while (width < n) width <<= 1;
@@ -493,7 +486,7 @@ __device__ inline int wave_edge_pairs(const Polys& A, const RowSpan& sa, const f
                 }
                 nb += __popcll(m);
                 if (nb <= 64 && b0 + 64 < sb.hi) continue;  // room for another 64
-                wave_lds_fence();
+                wave_lds_order();
                 for (int k0 = 0; k0 < nb; k0 += subs) {
                     const int k = k0 + sub;
                     const bool hit = has && k < nb && boxes_meet(abox, W.box[k < nb ? k : 0]);
@@ -514,31 +507,30 @@ __device__ inline int wave_edge_pairs(const Polys& A, const RowSpan& sa, const f
                             ma = W.qa[64 + lane];
                             mb = W.qb[64 + lane];
                         }
-                        wave_lds_fence();
+                        wave_lds_order();
                         if (lane < nq) {
                             W.qa[lane] = ma;
                             W.qb[lane] = mb;
                         }
-                        wave_lds_fence();
+                        wave_lds_order();
                     }
                 }
-                wave_lds_fence();
+                wave_lds_order();
                 nb = 0;
             }
             na -= n;
             const int32_t rest = lane < na ? W.a[64 + lane] : 0;
-            wave_lds_fence();
+            wave_lds_order();
             if (lane < na) W.a[lane] = rest;
-            wave_lds_fence();
+            wave_lds_order();
         }
     }
     if (nq > 0) test_queue(nq);
     return found;
 }
 
-// The point lies inside row s of P or on its boundary, by one wave.
-__device__ inline bool wave_not_outside(double px, double py, const Polys& P, int64_t row, const RowSpan& s,
-                                        int lane) {
+// The point lies inside the row of P or on its boundary, by one wave.
+__device__ inline bool wave_not_outside(double px, double py, const Polys& P, int64_t row, int lane) {
     for (int32_t pp = P.geom[row]; pp < P.geom[row + 1]; ++pp) {
         const RowSpan t = {P.ring[P.part[pp]], P.ring[P.part[pp + 1]], P.part[pp], P.part[pp + 1]};
         int parity = 0;
@@ -554,14 +546,14 @@ __device__ inline bool wave_not_outside(double px, double py, const Polys& P, in
 
 // Some ring of row ra of A starts at a point of row rb of B (not outside).
 __device__ inline bool wave_rings_start_in(const Polys& A, const RowSpan& sa, const Polys& B, int64_t rb,
-                                           const RowSpan& sb, const float4& bb, int lane) {
+                                           const float4& bb, int lane) {
     for (int32_t r = sa.r0; r < sa.r1; ++r) {
         const int32_t c = A.ring[r];
         if (A.ring[r + 1] <= c) continue;
         const double x = A.x[c], y = A.y[c];
         const float fx = (float)x, fy = (float)y;
         if (fx < bb.x || fx > bb.z || fy < bb.y || fy > bb.w) continue;  // outside B's box
-        if (wave_not_outside(x, y, B, rb, sb, lane)) return true;
+        if (wave_not_outside(x, y, B, rb, lane)) return true;
     }
     return false;
 }
@@ -655,8 +647,8 @@ __device__ inline Relation wave_relate_polygons(const Polys& A, int64_t ra, cons
 // One side of the relation of two rows whose boundaries do not meet: every
 // ring of A then lies in one piece inside or outside B, where its first vertex
 // does.  A ring without two distinct points has no piece.
-__device__ inline RelSide wave_apart_side(const Polys& A, int64_t ra, const Polys& B, int64_t rb, const RowSpan& sb,
-                                          const float4& bb, int lane) {
+__device__ inline RelSide wave_apart_side(const Polys& A, int64_t ra, const Polys& B, int64_t rb, const float4& bb,
+                                          int lane) {
     RelSide S = {false, false, false, false, false, true};
     for (int32_t pp = A.geom[ra]; pp < A.geom[ra + 1]; ++pp) {
         bool part_in = false;
@@ -669,8 +661,8 @@ __device__ inline RelSide wave_apart_side(const Polys& A, int64_t ra, const Poly
                 piece = __ballot(c + lane < c1 && (A.x[c + lane] != x || A.y[c + lane] != y)) != 0;
             if (!piece) continue;
             const float fx = (float)x, fy = (float)y;
-            const bool in = !(fx < bb.x || fx > bb.z || fy < bb.y || fy > bb.w) &&
-                            wave_not_outside(x, y, B, rb, sb, lane);
+            const bool in =
+                !(fx < bb.x || fx > bb.z || fy < bb.y || fy > bb.w) && wave_not_outside(x, y, B, rb, lane);
             S.in_int |= in;
             S.in_ext |= !in;
             part_in |= in;
@@ -704,12 +696,12 @@ __device__ inline int wave_polygon_predicate_fast(int pred, const Polys& A, int6
     if (contact == 2) return inclusion || pred == VS_PRED_TOUCHES ? 0 : 1;
     if (!inclusion) {
         // without contact the rows meet only if a ring of one starts in the other
-        const bool meet = contact == 1 || wave_rings_start_in(A, sa, B, rb, sb, bb, lane) ||
-                          wave_rings_start_in(B, sb, A, ra, sa, ba, lane);
+        const bool meet = contact == 1 || wave_rings_start_in(A, sa, B, rb, bb, lane) ||
+                          wave_rings_start_in(B, sb, A, ra, ba, lane);
         if (!meet || pred == VS_PRED_INTERSECTS) return meet ? 1 : 0;
     }
     if (contact == 1) return -1;
-    const RelSide ea = wave_apart_side(A, ra, B, rb, sb, bb, lane), eb = wave_apart_side(B, rb, A, ra, sa, ba, lane);
+    const RelSide ea = wave_apart_side(A, ra, B, rb, bb, lane), eb = wave_apart_side(B, rb, A, ra, ba, lane);
     return relation_decides(pred, merge_sides(ea, eb)) ? 1 : 0;
 }
 

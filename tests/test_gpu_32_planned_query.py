@@ -119,6 +119,26 @@ def test_few_queries(monkeypatch, n_queries, few_slots):
     assert st.retries == int(n_queries <= J.FEW_QUERIES and len(el) > few_slots)
 
 
+def test_pairs_are_complete_on_return():
+    """As from every join: another stream may read them without waiting."""
+    from vibespatial_amd import GeoSeries
+
+    w = S.c1(n_points=2_000_000, n_polys=400)
+    D = DevicePolygons.from_host(w.polygons)
+    b = J.polygon_bounds(D)
+    idx = J.LearnedPointIndex(DevicePoints.from_host(w.points))
+    for _ in range(3):
+        idx.query_polygons(D, b, "contains")
+        assert torch.cuda.current_stream().query()
+        idx.query_boxes(b)
+        assert torch.cuda.current_stream().query()
+    tree = GeoSeries(w.points).sindex
+    rows = GeoSeries(w.polygons).values
+    for k in range(3):
+        tree.query(rows[k], predicate="contains", return_device=True)
+        assert torch.cuda.current_stream().query()
+
+
 @pytest.mark.parametrize("slots", [0, 1])
 def test_scan_and_finish_at_one_capacity(slots):
     """vs_learned_query_run with room for the pairs, and with a slot too few."""

@@ -260,11 +260,11 @@ def _pairs_family(q_fam: str, qarr, t_fam: str, tarr, tindex: _FamilyIndex, pred
         return l, r
     if how == "learned_boxes":
         qb = J.point_boxes(device_points(qarr)) if q_fam == "point" else J.polygon_bounds(device_polygons(qarr))
-        l, r, _ = tindex.learned().query_boxes(qb)
+        l, r, _ = tindex.learned().query_boxes(qb, wait=False)
         return l, r
     if how == "learned_polygons":
         P = device_polygons(qarr)
-        l, r, _ = tindex.learned().query_polygons(P, J.polygon_bounds(P), predicate)
+        l, r, _ = tindex.learned().query_polygons(P, J.polygon_bounds(P), predicate, wait=False)
         return l, r
     tree = tindex.tree(t_fam)
     if predicate == "dwithin":
@@ -407,7 +407,10 @@ class SpatialIndex:
             self.last_strategy = []
             l, r = query_pairs(q, self._ga, self._index, predicate, dist, self.last_strategy)
         if return_device:
-            return r if scalar else torch.stack([l, r])
+            if not scalar:
+                return torch.stack([l, r])
+            torch.cuda.current_stream().synchronize()  # of pairs that were not waited for
+            return r
         if output_format == "indices":  # one copy of the stacked rows
             return r.cpu().numpy() if scalar else torch.stack([l, r]).cpu().numpy()
         lh, rh = l.cpu().numpy(), r.cpu().numpy()

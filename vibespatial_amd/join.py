@@ -588,12 +588,14 @@ class LearnedPointIndex:
         s = st.cpu().tolist()
         return out[:m], {"probes": s[0], "mlp_fallbacks": s[1], "window_fallbacks": s[2]}
 
-    def _planned_query(self, boxes: torch.Tensor, P: DevicePolygons | None, predicate, lookup: str, sort: bool):
+    def _planned_query(self, boxes: torch.Tensor, P: DevicePolygons | None, predicate, lookup: str, sort: bool,
+                       wait: bool):
         """query_boxes (P None) / query_polygons without a caller capacity: the
         plan's scan length, an upper bound of the pairs, sizes the stage, so the
         scan runs once; the pairs it staged size the output and the finish.
-        FEW_QUERIES rows or less are scanned without that wait.  A bound over POSITION_LIMIT, or one there is no memory for, is not
-        allocated: the planned scan then runs twice, the first time to count."""
+        FEW_QUERIES rows or less are scanned without that wait.  A bound over
+        POSITION_LIMIT, or one there is no memory for, is not allocated: the
+        planned scan then runs twice, the first time to count."""
         dev = require_gpu()
         L = lib()
         nq = int(boxes.shape[0])
@@ -637,18 +639,22 @@ class LearnedPointIndex:
             check(L.vs_learned_query_finish(self.n, nq, cap, n, int(bool(sort)), ptr(out_l), ptr(out_r), ptr(plan),
                                             plan.numel(), ptr(stage), stage.numel(), ptr(ws), ws.numel(), stream()),
                   "vs_learned_query_finish")
+            if wait:
+                torch.cuda.current_stream().synchronize()
         return out_l, out_r, _learned_stats(h, cap, retries)
 
     def query_boxes(self, boxes: torch.Tensor, lookup: str = "learned", capacity: int | None = None,
-                    sort: bool = True):
+                    sort: bool = True, wait: bool = True):
         """(box, point) pairs with the point in the box (inclusive); lexsorted
-        when `sort`, else grouped by box with points in unspecified order."""
+        when `sort`, else grouped by box with points in unspecified order.
+        Unless `wait`, the pairs may still be in the making on the current
+        stream."""
         dev = require_gpu()
         L = lib()
 
         def run(bx):
             if capacity is None:
-                return self._planned_query(bx, None, None, lookup, sort)
+                return self._planned_query(bx, None, None, lookup, sort, wait)
             nb = int(bx.shape[0])
             cap = int(capacity)
             cap = min(cap, PAIR_LIMIT)
@@ -673,18 +679,18 @@ class LearnedPointIndex:
         return _split_boxes(run, boxes)
 
     def query_polygons(self, P: DevicePolygons, bounds: torch.Tensor, predicate: str, lookup: str = "learned",
-                       capacity: int | None = None, sort: bool = True):
+                       capacity: int | None = None, sort: bool = True, wait: bool = True):
         """(polygon row, point) pairs with predicate(polygon, point) exact
         (contains / contains_properly: interior, touches: boundary, covers /
         intersects: not outside), through the index and the FP32 refine with
-        exact escalation (vs_learned_query_polygons); lexsorted when `sort`."""
+        exact escalation; lexsorted when `sort`; `wait` as for query_boxes."""
         dev = require_gpu()
         L = lib()
         if predicate not in ("contains", "contains_properly", "covers", "intersects", "touches"):
             raise NotImplementedError(f"polygon x point predicate {predicate!r}")
         if capacity is None:
             try:
-                return self._planned_query(bounds, P, predicate, lookup, sort)
+                return self._planned_query(bounds, P, predicate, lookup, sort, wait)
             except _PairLimit as e:
                 raise OverflowError(f"{e.args[0]} pairs exceed the int32 pair limit of one call") from None
         nq = len(P)

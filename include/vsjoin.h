@@ -362,9 +362,8 @@ int vs_learned_query_polygons(const void* index, int64_t n_points, int32_t key_b
  * `predicate` as for vs_learned_query_polygons; d_result int64[16] as for the
  * learned join, d_result[1] above `capacity`: pairs were left out, scan again.
  * vs_learned_query_finish turns the stage of scan_capacity slots into output of
- * `capacity` slots, which need be no more than the pairs that were staged
- * (more than `capacity`: nothing is written and the stage stays as it is);
- * one finish that writes per scan.  vs_learned_query_run is a scan and a finish
+ * `capacity` slots: the pairs that were staged (with more of them nothing is
+ * written and the stage stays as it is); one finish that writes per scan.  vs_learned_query_run is a scan and a finish
  * at one capacity.  A plan holds for the same index, queries and offsets and
  * may be scanned again (with a larger capacity). */
 int64_t vs_learned_plan_bytes(int64_t n_queries);

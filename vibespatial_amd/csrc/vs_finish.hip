@@ -20,7 +20,7 @@
 //      global memory (merge by co-rank: each element's output slot is its
 //      index in its own half plus its rank in the other half).
 //
-// A stage with room for many pairs per left row (kLexSlots) is sorted by both
+// A stage with many pairs per left row (kLexPairs) is sorted by both
 // ids instead: radix passes over the right ids, then over the left ids.
 //
 // Pairs with the same left id come from one join and have distinct right ids,
@@ -365,19 +365,21 @@ static int bits_for(int64_t n) {
     return b;
 }
 
-// Slots per left row from which the pairs are sorted by both ids instead of by
-// left id and then run by run.  The slots are the pairs themselves in a planned
-// query, else the caller's bound on them.  Runs longer than kShortRun go through
-// the block sorts of long runs (2.3e9 ids/s), where a further radix pass over
-// the right ids takes its 20 B per pair at 4 TB/s.  Box query of 100k rows over
-// 4M points, sorted by both ids / by runs, us: 8 hits a row 509 / 470, 16
-// 525 / 510, 20 538 / 525, 24 563 / 599, 32 595 / 1401, 64 748 / 2814; of 2k
-// rows: 16 hits 230 / 215, 32 223 / 226, 64 234 / 242.  The line lies below the
-// crossing of these even rows because uneven ones pass kShortRun sooner.
-constexpr int64_t kLexSlots = 16;
+// Pairs per left row from which the pairs are sorted by both ids instead of by
+// left id and then run by run.  Runs longer than kShortRun go through the block
+// sorts of long runs (2.3e9 ids/s), where a further radix pass over the right
+// ids takes its 20 B per pair at 4 TB/s.  Box query of 100k rows over 4M points,
+// sorted by both ids / by runs, us: 8 hits a row 509 / 470, 16 525 / 510, 20
+// 538 / 525, 24 563 / 599, 32 595 / 1401, 64 748 / 2814; of 2k rows: 16 hits
+// 230 / 215, 32 223 / 226, 64 234 / 242.  The line lies below the crossing of
+// these even rows because uneven ones pass kShortRun sooner.  A capacity that
+// is a guess (`exact` false) is taken for twice the pairs: the callers' run from
+// 1.25 times what the last query found to 16 slots for a row with one or two.
+constexpr int64_t kLexPairs = 16;
 
 int finish_staged_pairs(const PairStage& S, void* ws, JoinCtl* ctl, int64_t n_left, int64_t n_right,
-                        int64_t capacity, bool sort_right, int64_t* out_l, int64_t* out_r, hipStream_t s) {
+                        int64_t capacity, bool exact, bool sort_right, int64_t* out_l, int64_t* out_r,
+                        hipStream_t s) {
     VS_REQUIRE(capacity >= 0 && capacity < (int64_t)INT32_MAX, "join capacity %lld out of range [0, 2^31-1)",
                (long long)capacity);
     VS_REQUIRE(n_left >= 0 && n_left < (int64_t)UINT32_MAX, "left row count %lld out of range [0, 2^32-1)",
@@ -386,7 +388,8 @@ int finish_staged_pairs(const PairStage& S, void* ws, JoinCtl* ctl, int64_t n_le
     const FinishBufs F = carve_finish(c, capacity);
     const int nbits = bits_for(n_left);
     SortResult<uint32_t> r;
-    if (sort_right && nbits > 0 && n_right > 1 && n_right <= (int64_t)INT32_MAX && capacity / kLexSlots >= n_left)
+    const int64_t pairs = exact ? capacity : capacity / 2;
+    if (sort_right && nbits > 0 && n_right > 1 && n_right <= (int64_t)INT32_MAX && pairs / kLexPairs >= n_left)
         return sort_lex_wide_u32(S.l, S.r, capacity, &ctl->staged, nbits, bits_for(n_right), F.sort_ws,
                                  sort_workspace_bytes_u32(capacity), s, out_l, out_r);
     if (capacity > 1 && nbits > 0) {  // the sort's last pass writes the output pairs
@@ -425,7 +428,7 @@ int finish_pairs(void* fin_ws, JoinCtl* ctl, int64_t n_left, int64_t n_right, in
     Carver c(fin_ws);
     const PairStage S = carve_stage(c, capacity);
     void* ws = c.take<char>(finish_staged_workspace_bytes(capacity));
-    VS_TRY(finish_staged_pairs(S, ws, ctl, n_left, n_right, capacity, sort_right, out_l, out_r, s));
+    VS_TRY(finish_staged_pairs(S, ws, ctl, n_left, n_right, capacity, false, sort_right, out_l, out_r, s));
     hipLaunchKernelGGL(publish_result_kernel, dim3(1), dim3(64), 0, s, ctl, d_result);
     VS_LAUNCH_CHECK();
     return VS_OK;

@@ -27,7 +27,8 @@ void fill_i32(int32_t* p, int64_t n, int32_t v, hipStream_t s);
 // as u32, right ids as i32, ctl->staged the count); finish_staged_pairs turns
 // them into int64 output sorted by left id (and by right id within a left id
 // when sort_right).  capacity: slots of the output, at most those of the stage;
-// a count above it leaves the output unwritten and the stage as it is.  n_right:
+// a count above it leaves the output unwritten and the stage as it is.  exact:
+// the capacity is the count itself, not a guess above it.  n_right:
 // right ids are below it (0: not known); it lets a join of many hits per left
 // row sort by both ids.  A finish reorders the stage, so it runs once.
 struct PairStage {
@@ -38,7 +39,8 @@ struct PairStage {
 PairStage carve_stage(Carver& c, int64_t capacity);
 int64_t finish_staged_workspace_bytes(int64_t capacity);
 int finish_staged_pairs(const PairStage& S, void* ws, JoinCtl* ctl, int64_t n_left, int64_t n_right,
-                        int64_t capacity, bool sort_right, int64_t* out_l, int64_t* out_r, hipStream_t s);
+                        int64_t capacity, bool exact, bool sort_right, int64_t* out_l, int64_t* out_r,
+                        hipStream_t s);
 
 // The same with the stage in one workspace, from which finish_stage carves it;
 // finish_pairs also publishes d_result[0..3].

@@ -2236,7 +2236,7 @@ int learned_run_t(int mode, int pred, const double4* qbox, int64_t nq, int64_t n
                   int64_t* out_l, int64_t* out_r, int64_t* d_result, hipStream_t s) {
     VS_TRY(learned_scan_t<K>(mode, pred, qbox, nq, B, R, capacity, Q, d_result, s));
     return finish_staged_pairs({Q.stage_l, Q.stage_r}, Q.fin_ws, Q.ctl, n_left, mode == kLModePip ? nq : n_points,
-                               capacity, sort, out_l, out_r, s);
+                               capacity, false, sort, out_l, out_r, s);
 }
 
 template <class K>
@@ -2572,8 +2572,8 @@ int vs_learned_query_finish(int64_t n_points, int64_t n_queries, int64_t scan_ca
     vs::Carver cs(scan_workspace);
     const vs::QueryBufs Q = vs::carve_plan(cp, n_queries, n_queries);
     const vs::PairStage S = vs::carve_stage(cs, scan_capacity);
-    return vs::finish_staged_pairs(S, workspace, Q.ctl, n_queries, n_points, capacity, sort != 0, out_left, out_right,
-                                   vs::stream_of(stream));
+    return vs::finish_staged_pairs(S, workspace, Q.ctl, n_queries, n_points, capacity, true,
+                                   sort != 0, out_left, out_right, vs::stream_of(stream));
 }
 
 int64_t vs_learned_run_workspace_bytes(int64_t n_coords, int64_t capacity) {
@@ -2588,15 +2588,17 @@ int vs_learned_query_run(const void* index, int64_t n_points, int32_t key_bytes,
                          int64_t* out_left, int64_t* out_right, int64_t* d_result, void* plan, int64_t plan_bytes,
                          void* workspace, int64_t workspace_bytes, void* stream) {
     const int64_t scan_bytes = vs_learned_scan_workspace_bytes(n_coords, capacity);
-    const int64_t finish_bytes = vs_learned_finish_workspace_bytes(capacity);
     VS_REQUIRE(workspace_bytes >= vs_learned_run_workspace_bytes(n_coords, capacity),
                "vs_learned_query_run: workspace too small");
     VS_TRY(vs_learned_query_scan(index, n_points, key_bytes, n_leaves, boxes, x, y, geom_offsets, part_offsets,
                                  ring_offsets, n_queries, n_parts, n_rings, n_coords, predicate, capacity, d_result,
                                  plan, plan_bytes, workspace, scan_bytes, stream));
     void* finish_ws = static_cast<char*>(workspace) + ((scan_bytes + 255) & ~int64_t(255));
-    return vs_learned_query_finish(n_points, n_queries, capacity, capacity, sort, out_left, out_right, plan,
-                                   plan_bytes, workspace, scan_bytes, finish_ws, finish_bytes, stream);
+    vs::Carver cp(plan);
+    vs::Carver cs(workspace);
+    const vs::QueryBufs Q = vs::carve_plan(cp, n_queries, n_queries);
+    return vs::finish_staged_pairs(vs::carve_stage(cs, capacity), finish_ws, Q.ctl, n_queries, n_points, capacity,
+                                   false, sort != 0, out_left, out_right, vs::stream_of(stream));
 }
 
 int64_t vs_sjoin_points_polygons_learned_workspace_bytes(int64_t n_points, int64_t n_polys, int64_t n_coords,

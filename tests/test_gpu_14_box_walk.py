@@ -22,7 +22,8 @@ def _boxes(rng, n, extent, side):
 
 @pytest.mark.parametrize("n_q,n_t,fanout", [(1, 1, 16), (15, 2, 2), (17, 16, 16), (65, 17, 16), (400, 1000, 2),
                                             (400, 1000, 3), (700, 5000, 16), (700, 5000, 64), (3000, 20_000, 16),
-                                            (524_287, 300, 16), (524_290, 300, 16)])
+                                            (262_143, 300, 16), (262_144, 300, 16), (524_287, 300, 16),
+                                            (524_290, 300, 16)])
 def test_sparse_and_dense_queries_match_bruteforce(n_q, n_t, fanout):
     rng = np.random.default_rng(n_q + n_t)
     tb = _boxes(rng, n_t, 1000.0, 20.0)

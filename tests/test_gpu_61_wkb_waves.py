@@ -1,5 +1,5 @@
 """The WKB row passes at the edges of a wave's 64 and 256 rows, of a tile's
-1,024 and of four tiles: points alone, one polygonal row at a wave's first or last place,
+1,024, of four tiles and of the prefix's 4,096 tiles: points alone, one polygonal row at a wave's first or last place,
 a null or a tagged point among plain ones, mixed byte orders, and a record that
 is 21 bytes long and no point, against the oracle."""
 
@@ -43,3 +43,27 @@ def test_waves(n, odd):
         assert np.array_equal(ga.polygon_rows, exp["polygon_rows"])
         for k in ("x", "y", "ring_offsets", "part_offsets", "geom_offsets"):
             assert np.array_equal(getattr(ga.polygons, k), exp[k]), k
+
+
+@pytest.mark.parametrize("extra", [-1, 0, 1, 1500])
+def test_more_tiles_than_one_round_of_the_prefix(extra):
+    """4,096 tiles of points, a square as the last record of each round."""
+    n = 4096 * 1024 + extra
+    print(f"wkb tiles n {n}", flush=True)
+    rng = np.random.default_rng(extra + 1)
+    rec = np.zeros(n, dtype=np.dtype([("order", "u1"), ("type", "<u4"), ("x", "<f8"), ("y", "<f8")]))
+    rec["order"], rec["type"] = 1, 1
+    rec["x"], rec["y"] = rng.uniform(-1e3, 1e3, (2, n))
+    at = sorted({4096 * 1024 - 1, n - 1} & set(range(n)))
+    cuts = [0, *(k * 21 for k in at), n * 21]
+    raw = rec.tobytes()
+    payload = b"".join(raw[a + 21 * (i > 0) : b] + (SQUARE if i < len(at) else b"")
+                       for i, (a, b) in enumerate(zip(cuts, cuts[1:])))
+    size = np.full(n, 21, dtype=np.int64)
+    size[at] = len(SQUARE)
+    ga = decode_wkb(np.frombuffer(payload, np.uint8), np.concatenate([[0], np.cumsum(size)]), None)
+    keep = np.ones(n, dtype=bool)
+    keep[at] = False
+    assert np.array_equal(ga.point_rows, np.flatnonzero(keep)) and np.array_equal(ga.polygon_rows, at)
+    assert np.array_equal(ga.points.x, rec["x"][keep]) and np.array_equal(ga.points.y, rec["y"][keep])
+    assert np.array_equal(ga.polygons.ring_offsets, 4 * np.arange(len(at) + 1))

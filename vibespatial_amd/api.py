@@ -17,9 +17,10 @@ mixed point/polygon columns and assembles frames), chosen per family pair by
                     refine with exact escalation (vs_sjoin_points_polygons_learned)
   polygon x point   (point tree) contains / contains_properly / covers /
                     intersects / touches -> the tree's learned index and the
-                    same FP32 refine (vs_learned_query_polygons); axis-aligned
-                    rectangles with intersects / covers, and predicate None,
-                    -> the learned box query alone (vs_learned_query_boxes)
+                    same FP32 refine (vs_learned_query_plan / _scan /
+                    _finish with polygon offsets); axis-aligned rectangles
+                    with intersects / covers, and predicate None, -> the
+                    learned box query alone (the same without offsets)
   point  x point    intersects / within / contains / covers / covered_by /
                     contains_properly / None -> learned box query (equality)
   polygon x polygon every predicate -> packed-tree bbox query + exact refine
@@ -227,7 +228,7 @@ def _strategy(q_fam: str, t_fam: str, predicate, qarr) -> str:
                        (spatial/query_box.py:760-863: the pure box path);
       learned_polygons other polygon-over-point predicates on point trees:
                        the FP32 point-in-polygon refine over the tree's
-                       learned index (vs_learned_query_polygons);
+                       learned index (vs_learned_query_plan / _scan / _finish);
       tree             polygon trees queried by polygons, bbox-only point
                        queries of polygon trees, and dwithin: packed Hilbert
                        tree + exact refine."""

@@ -354,8 +354,9 @@ __global__ __launch_bounds__(kJoinThreads) void traverse_kernel(
 // those as four of 4; each item is then tested by 16 or 4 lanes, 4 or 16 items
 // at a time.
 //
-// Bound by latency and by the atomics on the stage counter, not by work (3% of
-// the issue slots): each costs about 20 ns in turn, whichever wave sends it.
+// Bound by latency and by the atomics on the stage counter, not by work (the
+// vector units are busy 16% of the time): each atomic costs about 20 ns in turn,
+// whichever wave sends it.
 // So the units are dealt out in turn with no queue, and a wave buffers 1,024
 // pairs.  3M points x 100k boxes (6.4M pairs): 2,180 us with one node group
 // per step, item ids loaded one by one, unions left whole, eight queues and 256

@@ -460,7 +460,9 @@ struct NearestTree {
 // in one step and measure an item together, and the four queries of a wave
 // wait for the slowest of four instead of 64.  With a lane to a query the
 // launch ran on with 1.6 waves a SIMD behind the queries of the longest walks
-// and widest rows (392,000 points, 100,000 polygons: 1490 us, now 1000).
+// and widest rows (392,000 points, 100,000 polygons: 2240 us with each lane
+// measuring its items alone, 1490 with the wave's lanes measuring together, now
+// 1000, the vector units busy 55% of the time).
 constexpr int kBoundLanes = 16;
 constexpr int kBoundStack = 256;
 constexpr int kBoundPops = 4096;  // visit limit per query (bounds the time of a pathological query)

@@ -426,11 +426,13 @@ VS_HD int segment_contact(double ax, double ay, double bx, double by, double cx,
 // other, so: A's edges near B's box are listed and taken 64 at a time, one per
 // lane (fewer: each edge gets several lanes, which share B's edges); B's edges
 // near them are collected in LDS tiles as fp32 boxes; box pairs that meet are
-// queued, and a full queue gets the exact test with all lanes at work.  Bound
-// by instruction issue: testing every edge pair of the rows in fp64, with a
-// wave waiting for any lane's exact test, took 11.1 ms for 600k pairs of
-// 57 x 57 coordinates; this takes 2.0 ms (about 860 vector instructions a pair),
+// queued, and a full queue gets the exact test with all lanes at work.  Testing
+// every edge pair of the rows in fp64, with a wave waiting for any lane's exact
+// test, took 11.1 ms for 600k pairs of 57 x 57 coordinates; this takes 2.0 ms,
 // and rows without contact need no full relation (2.9 ms for the 3% that did).
+// Bound by latency: 412M vector and 409M scalar instructions (some 690 of each a
+// pair) keep the vector units busy a third of the time at 3.2 waves a SIMD; the
+// rest waits for the chain of offset loads and the LDS lists' order points.
 __device__ inline int wave_edge_pairs(const Polys& A, const RowSpan& sa, const float4& ba, const Polys& B,
                                       const RowSpan& sb, const float4& bb, int enough, WaveEdgeLds& W, int lane) {
     const float4 both = box_cut(ba, bb);

@@ -510,7 +510,9 @@ int rs_small(const K* ki, const int32_t* vi, void* ko, void* vo, int64_t n, cons
 
 // Blocks up to which a pass is two launches: each scatter block reads every
 // block's histogram (1 KB each, from L2) instead of waiting for two scan
-// launches of 4-5 us.
+// launches of 4-5 us.  Ten sorts by 32 bits of u32 keys, two launches / four, us:
+// 8 tiles 586 / 848, 64 718 / 975, 128 878 / 1038, 192 985 / 1070, 256 1136 /
+// 1081; of u64 keys: 128 896 / 1072, 192 1060 / 1128, 256 1137 / 1126.
 constexpr int kRsFusedBlocks = 128;
 
 // One radix pass: digit (key >> shift) & dmask, stable.
